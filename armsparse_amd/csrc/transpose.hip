@@ -3,12 +3,10 @@
 // Reference: toCSC's column-major scan (SpMM.cpp:80-95) and scipy's tocsc in
 // the GCN script (gcn_custom.py:48-55) produce, for every column, its entries
 // with ascending rows; csr2cscKernel (gcn/pytorch-custom/spmm_kernel.cu:381-423)
-// would call cuSPARSE for it.  Here: an LSD radix sort of (column, position)
-// pairs, 8 bits per pass.  The input is already in row order, and every pass
-// is stable (per-block digit histograms, a device-wide exclusive scan, and a
-// scatter whose in-block ranks come from wave ballots in item order), so rows
-// stay ascending inside each column.  The last pass gathers row ids and
-// values; colptr is read off the sorted column keys.
+// would call cuSPARSE for it.  Here: a stable LSD radix sort of (column, row,
+// value) records, up to 10 bits per pass (k_radix_scatter).  The input is already
+// in row order and every pass is stable, so rows stay ascending inside each
+// column; colptr is read off the sorted column keys.
 //
 // COO → CSR (the canonical CSR of toCSR, SDMM.cpp:355-370 / SpMM.cpp:64-79,
 // built from unordered triplets on the device): the same stable sort by
@@ -27,93 +25,302 @@
 namespace armsp {
 namespace {
 
-constexpr int TPB = 256, IPT = 16, TILE = TPB * IPT;  // items per block: 4 waves × 16 rounds × 64
-constexpr int NB = 256;                               // 8-bit digits
-constexpr int SCAN_CHUNK = 2048;                       // 256 threads × 8
+constexpr int TPB = 256;
+constexpr int SCAN_CHUNK = 2048;  // 256 threads × 8
 
-__global__ __launch_bounds__(256) void k_expand_rows(int M, const int* __restrict__ rowptr, int* __restrict__ rows) {
-    const int lane = threadIdx.x & 63;
-    const int r = uniform((int)(blockIdx.x * 4u + (threadIdx.x >> 6)));
-    if (r >= M) return;
-    const int b = rowptr[r], e = rowptr[r + 1];
-    for (int p = b + lane; p < e; p += 64) rows[p] = r;
+// ------------------------------------------------------------- radix sort
+// One pass sorts the records by a digit of `db` bits: k_radix_hist counts the
+// digits of every tile, k_radix_scan turns the counts into each tile's first
+// position within its digit (and the digits' totals), k_radix_scatter ranks a
+// tile's records, orders them by digit in LDS and writes every digit's run of
+// the tile as consecutive elements.
+// Bound: a record (key, companion index, value) is read and written once per
+// pass, 24 bytes, plus 4 for the histogram, and ranked with one ballot per digit
+// bit.  Digits are as wide as the LDS ranks allow (10 bits: a million columns
+// take two passes), the value travels with its key, and the row of a CSR entry
+// is formed in the first pass from rowptr.  (Sorting positions in 8-bit digits
+// and gathering rows and values at the end took 1523 us for the 1M R-MAT's 2^24
+// entries; 393 us now: 205 MB read and 213 MB written a pass, by the counters.)
+// Consecutive tiles go to one XCD, so the lines two tiles share are completed in
+// that XCD's L2 (in launch order instead: 480 -> 503 us).
+constexpr int RADIX_MAX_BITS = 10;
+constexpr int RADIX_MIN_BITS = 4;  // k_radix_scan takes 16 digits a workgroup
+
+// Tile of block b: XCD b % 8 walks a contiguous eighth of the tiles (-1: none).
+__device__ __forceinline__ int xcd_tile(int ntiles) {
+    const int per = (ntiles + 7) >> 3, i = (int)(blockIdx.x >> 3);
+    const int t = (int)(blockIdx.x & 7u) * per + i;
+    return t < ntiles ? t : -1;
+}
+inline unsigned xcd_grid(int ntiles) { return (unsigned)((ntiles + 7) / 8) * 8u; }
+
+// hist[tile·bins + d] = records of the tile with digit d.  With `other`, also sets
+// *bad where a key is outside [0, krange) or other[p] outside [0, orange).
+template <int THREADS, int IPT>
+__global__ __launch_bounds__(THREADS) void k_radix_hist(int n, int shift, int db, int ntiles,
+                                                        const int* __restrict__ keys, int* __restrict__ hist,
+                                                        const int* __restrict__ other, int krange, int orange,
+                                                        int* __restrict__ bad) {
+    __shared__ int cnt[1 << RADIX_MAX_BITS];
+    const int bins = 1 << db, tile = xcd_tile(ntiles);
+    if (tile < 0) return;
+    for (int d = threadIdx.x; d < bins; d += THREADS) cnt[d] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)tile * (THREADS * IPT);
+    int key[IPT];
+    bool oob = false;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const int64_t e = base + j * THREADS + threadIdx.x;
+        key[j] = e < n ? keys[e] : 0;
+        if (other && e < n) {
+            const int o = other[e];
+            oob |= key[j] < 0 || key[j] >= krange || o < 0 || o >= orange;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+        if (base + j * THREADS + threadIdx.x < n) atomicAdd(&cnt[(key[j] >> shift) & (bins - 1)], 1);
+    if (oob) atomicOr(bad, 1);
+    __syncthreads();
+    for (int d = threadIdx.x; d < bins; d += THREADS) hist[(int64_t)tile * bins + d] = cnt[d];
 }
 
-__global__ __launch_bounds__(256) void k_radix_hist(int n, int shift, const int* __restrict__ keys,
-                                                    int* __restrict__ hist, int nblocks) {
-    __shared__ int cnt[NB];
-    cnt[threadIdx.x] = 0;
+// Per digit, the exclusive scan of its counts over the tiles, in place, and its
+// total: a workgroup takes 16 digits (64-byte rows of hist), 64 threads a digit,
+// each a run of consecutive tiles.
+__global__ __launch_bounds__(1024) void k_radix_scan(int ntiles, int bins, int* __restrict__ hist,
+                                                     int* __restrict__ totals) {
+    constexpr int KEEP = 32;  // counts a thread holds between the two sweeps
+    __shared__ int part[64][16];
+    const int d = (int)(threadIdx.x & 15u), seg = (int)(threadIdx.x >> 4);
+    int* h = hist + (int)blockIdx.x * 16 + d;
+    const int per = (ntiles + 63) / 64;
+    const int t0 = seg * per, t1 = min(t0 + per, ntiles);
+    int v[KEEP];
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+        v[i] = t0 + i < t1 ? h[(int64_t)(t0 + i) * bins] : 0;
+        s += v[i];
+    }
+    for (int t = t0 + KEEP; t < t1; ++t) s += h[(int64_t)t * bins];
+    part[seg][d] = s;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * TILE;
-    for (int j = 0; j < IPT; ++j) {
-        const int64_t e = base + (int64_t)j * TPB + threadIdx.x;
-        if (e < n) atomicAdd(&cnt[(keys[e] >> shift) & (NB - 1)], 1);
+    if (threadIdx.x < 16) {
+        int run = 0;
+        for (int q = 0; q < 64; ++q) {
+            const int x = part[q][d];
+            part[q][d] = run;
+            run += x;
+        }
+        totals[blockIdx.x * 16 + d] = run;
     }
     __syncthreads();
-    hist[(int64_t)threadIdx.x * nblocks + blockIdx.x] = cnt[threadIdx.x];
+    int run = part[seg][d];
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i)
+        if (t0 + i < t1) {
+            h[(int64_t)(t0 + i) * bins] = run;
+            run += v[i];
+        }
+    for (int t = t0 + KEEP; t < t1; ++t) {
+        const int x = h[(int64_t)t * bins];
+        h[(int64_t)t * bins] = run;
+        run += x;
+    }
 }
 
-// idx_in == nullptr: item e carries its own position.  final_pass: instead of
-// idx_out, write rowind[dst] = rows[idx], valT[dst] = val[idx].
-__global__ __launch_bounds__(256) void k_radix_scatter(int n, int shift, const int* __restrict__ keys_in,
-                                                       const int* __restrict__ idx_in, const int* __restrict__ offs,
-                                                       int nblocks, int* __restrict__ keys_out,
-                                                       int* __restrict__ idx_out, const int* __restrict__ rows,
-                                                       const float* __restrict__ val, int* __restrict__ rowind,
-                                                       float* __restrict__ valT, int final_pass) {
-    __shared__ int wcnt[4][NB];
-    __shared__ int wpre[4][NB];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    for (int i = tid; i < 4 * NB; i += TPB) wcnt[i / NB][i % NB] = 0;
+// Exclusive scan of one value per thread over the workgroup; red: WAVES ints of LDS.
+template <int WAVES>
+__device__ __forceinline__ int block_exclusive(int x, int* red) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int inc = x;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(inc, d);
+        if (lane >= d) inc += o;
+    }
+    if (lane == 63) red[w] = inc;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * TILE + (int64_t)w * (IPT * 64);
-    const uint64_t lt = (1ull << lane) - 1ull;
-    int key[IPT], idx[IPT], dig[IPT], pos[IPT];
+    int before = 0;
+#pragma unroll
+    for (int q = 0; q < WAVES; ++q) before += q < w ? red[q] : 0;
+    __syncthreads();
+    return before + inc - x;
+}
+
+__host__ __device__ constexpr size_t radix_lds(int threads, int ipt, int bins) {
+    return (size_t)threads * ipt * 4 + (size_t)bins * 8 + (size_t)(threads / 64) * bins * 2 + (threads / 64) * 4;
+}
+
+// Records (key, a, v): CSR_ROWS takes a from rowptr (the row of entry p), VAL says
+// whether there is a v.  keys_out, a_out and v_out are written at the same places.
+template <int THREADS, int IPT, bool CSR_ROWS, bool VAL>
+__global__ __launch_bounds__(THREADS) void k_radix_scatter(int n, int shift, int db, int ntiles,
+                                                           const int* __restrict__ keys_in,
+                                                           const int* __restrict__ a_in,
+                                                           const float* __restrict__ v_in, int M,
+                                                           const int* __restrict__ rowptr,
+                                                           const int* __restrict__ offs,
+                                                           const int* __restrict__ totals, int* __restrict__ keys_out,
+                                                           int* __restrict__ a_out, float* __restrict__ v_out) {
+    constexpr int T = THREADS * IPT, WAVES = THREADS / 64, WT = 64 * IPT;
+    constexpr int DPT = (1 << RADIX_MAX_BITS) / THREADS;  // most digits per thread
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int bins = 1 << db, tile = xcd_tile(ntiles);
+    if (tile < 0) return;
+    int* stage = reinterpret_cast<int*>(smem);          // T
+    int* start = stage + T;                             // bins: a digit's first place in the ordered tile
+    int* goff = start + bins;                           // bins: where that place goes in the output, less the place
+    uint16_t* wcnt = reinterpret_cast<uint16_t*>(goff + bins);  // WAVES × bins
+    int* red = reinterpret_cast<int*>(wcnt + WAVES * bins);     // WAVES
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int64_t tbase = (int64_t)tile * T;
+    const int cnt = (int)min((int64_t)T, (int64_t)n - tbase);
+    int key[IPT], a[IPT], pos[IPT];
+    float v[IPT];
+    // item r of a lane: w·WT + r·64 + lane, so a wave's items are consecutive
 #pragma unroll
     for (int r = 0; r < IPT; ++r) {
-        const int64_t e = base + r * 64 + lane;
-        const bool valid = e < n;
-        key[r] = valid ? keys_in[e] : 0;
-        idx[r] = valid ? (idx_in ? idx_in[e] : (int)e) : -1;
-        const int d = (key[r] >> shift) & (NB - 1);
-        dig[r] = d;
-        uint64_t m = __ballot(valid);
-#pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            const bool on = (d >> bit) & 1;
-            const uint64_t bal = __ballot(on);
-            m &= on ? bal : ~bal;
+        const int i = w * WT + r * 64 + lane;
+        key[r] = i < cnt ? keys_in[tbase + i] : 0;
+        if constexpr (!CSR_ROWS) a[r] = i < cnt ? a_in[tbase + i] : 0;
+        if constexpr (VAL) v[r] = i < cnt ? v_in[tbase + i] : 0.0f;
+    }
+    for (int i = tid; i < WAVES * bins / 2; i += THREADS) reinterpret_cast<uint32_t*>(wcnt)[i] = 0u;
+    if constexpr (CSR_ROWS) {
+        // every row that begins inside the tile marks its first entry (the last such
+        // row where empty rows share it); a running maximum over the marks gives rows
+        for (int i = tid; i < T; i += THREADS) stage[i] = 0;
+        const int p0 = (int)tbase, p1 = p0 + cnt;
+        const int r0 = uniform(min(rows_ending_by_wave(p0, rowptr, M), M - 1));
+        __syncthreads();
+        for (int rb = r0 + 1 + w * 64; rb < M; rb += THREADS) {
+            const int r = rb + lane;
+            const int b = r < M ? rowptr[r] : INT_MAX;
+            if (b >= p0 && b < p1) atomicMax(&stage[b - p0], r - r0);
+            if (read_lane(b, 0) >= p1) break;  // later rows begin after the tile
         }
+        __syncthreads();
+        int run = 0;
+#pragma unroll
+        for (int r = 0; r < IPT; ++r) {  // the lane's row: the last mark at or before it
+            const int m = stage[w * WT + r * 64 + lane];
+            const uint64_t marks = __ballot(m != 0) & (~0ull >> (63 - lane));
+            const int from = __shfl(m, marks ? 63 - __builtin_clzll(marks) : 0);
+            a[r] = marks ? from : run;
+            run = read_lane(a[r], 63);
+        }
+        if (lane == 0) red[w] = run;
+        __syncthreads();
         int before = 0;
-        if (valid) before = wcnt[w][d];
+#pragma unroll
+        for (int q = 0; q < WAVES; ++q) before = max(before, q < w ? red[q] : 0);
+#pragma unroll
+        for (int r = 0; r < IPT; ++r) a[r] = r0 + max(a[r], before);
+    }
+    __syncthreads();
+    // rank among the wave's records of the same digit, in order
+    const uint64_t lt = (1ull << lane) - 1ull;
+    uint16_t* wc = wcnt + w * bins;
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const bool valid = w * WT + r * 64 + lane < cnt;
+        const int d = (key[r] >> shift) & (bins - 1);
+        // the wave's records with this digit: bit by bit, the lanes that agree with ours
+        const uint64_t all = __ballot(valid);
+        uint32_t lo = (uint32_t)all, hi = (uint32_t)(all >> 32);
+#pragma unroll
+        for (int bit = 0; bit < RADIX_MAX_BITS; ++bit) {
+            if (bit < db) {
+                const int on = __builtin_amdgcn_sbfe(d, bit, 1);  // 0 or -1
+                const uint64_t bal = __ballot(on != 0);
+                lo &= ~((uint32_t)bal ^ (uint32_t)on);
+                hi &= ~((uint32_t)(bal >> 32) ^ (uint32_t)on);
+            }
+        }
+        const uint64_t m = ((uint64_t)hi << 32) | lo;
+        const int before = valid ? wc[d] : 0;
         pos[r] = before + __popcll(m & lt);
-        __builtin_amdgcn_wave_barrier();
-        if (valid && (m >> lane) == 1ull) wcnt[w][d] = before + __popcll(m);  // highest peer updates
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync_lds();
+        if (valid && (m >> lane) == 1ull) wc[d] = (uint16_t)(before + __popcll(m));  // the digit's last record
+        wave_sync_lds();
     }
     __syncthreads();
     {
-        int run = 0;
+        int c[DPT], g[DPT], cs = 0, gs = 0;
+        const int dpt = (bins + THREADS - 1) / THREADS, d0 = tid * dpt;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            wpre[q][tid] = run;
-            run += wcnt[q][tid];
+        for (int i = 0; i < DPT; ++i) {
+            c[i] = g[i] = 0;
+            const int d = d0 + i;
+            if (i < dpt && d < bins) {
+                int run = 0;
+#pragma unroll
+                for (int q = 0; q < WAVES; ++q) {
+                    const int x = wcnt[q * bins + d];
+                    wcnt[q * bins + d] = (uint16_t)run;
+                    run += x;
+                }
+                c[i] = run;
+                g[i] = totals[d];
+            }
+            cs += c[i];
+            gs += g[i];
+        }
+        int cb = block_exclusive<WAVES>(cs, red);
+        int gb = block_exclusive<WAVES>(gs, red);
+#pragma unroll
+        for (int i = 0; i < DPT; ++i) {
+            const int d = d0 + i;
+            if (i < dpt && d < bins) {
+                start[d] = cb;
+                goff[d] = gb + offs[(int64_t)tile * bins + d] - cb;
+            }
+            cb += c[i];
+            gb += g[i];
         }
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < IPT; ++r) {
-        if (idx[r] < 0) continue;
-        const int d = dig[r];
-        const int dst = offs[(int64_t)d * nblocks + blockIdx.x] + wpre[w][d] + pos[r];
-        keys_out[dst] = key[r];
-        if (final_pass) {
-            rowind[dst] = rows[idx[r]];
-            if (valT) valT[dst] = val[idx[r]];
-        } else {
-            idx_out[dst] = idx[r];
+        const int d = (key[r] >> shift) & (bins - 1);
+        pos[r] += start[d] + wc[d];
+        if (w * WT + r * 64 + lane < cnt) stage[pos[r]] = key[r];
+    }
+    __syncthreads();
+    int dst[IPT];  // of the ordered tile's place tid + r·THREADS
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const int i = tid + r * THREADS;
+        dst[r] = 0;
+        if (i < cnt) {
+            const int k = stage[i];
+            dst[r] = goff[(k >> shift) & (bins - 1)] + i;
+            keys_out[dst[r]] = k;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < IPT; ++r)
+        if (w * WT + r * 64 + lane < cnt) stage[pos[r]] = a[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const int i = tid + r * THREADS;
+        if (i < cnt) a_out[dst[r]] = stage[i];
+    }
+    if constexpr (VAL) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPT; ++r)
+            if (w * WT + r * 64 + lane < cnt) stage[pos[r]] = __float_as_int(v[r]);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPT; ++r) {
+            const int i = tid + r * THREADS;
+            if (i < cnt) v_out[dst[r]] = __int_as_float(stage[i]);
         }
     }
 }
@@ -153,73 +360,175 @@ __global__ void k_scan_add(int64_t n, int* __restrict__ data, const int* __restr
     if (i < n) data[i] += sums[i / SCAN_CHUNK];
 }
 
-// colptr[c] = first sorted position whose column is ≥ c.
-__global__ void k_colptr(int nnz, int K, const int* __restrict__ keys, int* __restrict__ colptr) {
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p > nnz) return;
-    const int k = p < nnz ? keys[p] : K;
-    const int kp = p > 0 ? keys[p - 1] : -1;
-    for (int c = kp + 1; c <= k; ++c) colptr[c] = (int)p;
-}
-
-// rowptr[r] = first position whose row is ≥ r, for the *n_dev sorted rows.
-__global__ void k_rowptr_dev(const int* __restrict__ n_dev, int M, const int* __restrict__ keys,
-                             int* __restrict__ rowptr) {
-    const int n = *n_dev;
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p > n) return;
-    const int k = p < n ? keys[p] : M;
-    const int kp = p > 0 ? keys[p - 1] : -1;
-    for (int c = kp + 1; c <= k; ++c) rowptr[c] = (int)p;
-}
-
-__global__ void k_coo_check(int nnz, int M, int K, const int* __restrict__ rows, const int* __restrict__ cols,
-                            int* __restrict__ bad) {
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p >= nnz) return;
-    const int r = rows[p], c = cols[p];
-    if (r < 0 || r >= M || c < 0 || c >= K) atomicOr(bad, 1);
-}
-
-__global__ void k_gather_keys(int n, const int* __restrict__ idx, const int* __restrict__ src,
-                              int* __restrict__ dst) {
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p < n) dst[p] = src[idx[p]];
-}
-
-// keep[p] = 1 where p heads a run of equal (row, column) and the run is kept;
-// sums[p] = the run's values added in order (runs of duplicates are short).
-__global__ void k_coo_runs(int n, const int* __restrict__ srow, const int* __restrict__ scol,
-                           const float* __restrict__ sval, float* __restrict__ sums, int* __restrict__ keep,
-                           int drop_zeros) {
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const int r = srow[p], c = scol[p];
-    const bool head = p == 0 || srow[p - 1] != r || scol[p - 1] != c;
-    int k = 0;
-    if (head) {
-        float s = sval ? sval[p] : 1.0f;
-        for (int64_t q = p + 1; q < n && srow[q] == r && scol[q] == c; ++q)
-            if (sval) s += sval[q];
-        if (sval) sums[p] = s;
-        k = (!drop_zeros || !sval || s != 0.0f) ? 1 : 0;
+// ptr[c] = v for c in (lo, hi]; the whole wave calls it, and fills long gaps together
+// (the keys of a power-law matrix leave gaps of thousands, and one lane's walk of
+// such a gap outlasts the rest of the kernel).
+__device__ __forceinline__ void fill_gap(int* __restrict__ ptr, int lo, int hi, int v) {
+    const bool wide = hi - lo > 8;
+    if (!wide)
+        for (int c = lo + 1; c <= hi; ++c) ptr[c] = v;
+    for (uint64_t m = __ballot(wide); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const int a = read_lane(lo, l), b = read_lane(hi, l), x = read_lane(v, l);
+        for (int c = a + 1 + (int)__lane_id(); c <= b; c += 64) ptr[c] = x;
     }
-    keep[p] = k;
 }
 
-__global__ void k_coo_compact(int n, const int* __restrict__ srow, const int* __restrict__ scol,
-                              const float* __restrict__ sums, const int* __restrict__ keep,
-                              const int* __restrict__ pos, int* __restrict__ urow, int* __restrict__ colind,
-                              float* __restrict__ val, int* __restrict__ n_out) {
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    if (keep[p]) {
-        const int d = pos[p];
-        urow[d] = srow[p];
-        colind[d] = scol[p];
-        if (val) val[d] = sums[p];
+// ptr[c] = first sorted position whose key is ≥ c, c = 0..K; four keys a thread.
+__global__ __launch_bounds__(256) void k_colptr(int nnz, int K, const int* __restrict__ keys, int* __restrict__ ptr) {
+    const int64_t p0 = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
+    int k[5];  // past the end no key changes, so no gap is filled
+    k[0] = p0 > 0 ? (p0 <= nnz ? keys[p0 - 1] : K) : -1;
+    if (p0 + 4 <= nnz) {  // keys come from the workspace, 256-byte aligned
+        const int4 q = *reinterpret_cast<const int4*>(keys + p0);
+        k[1] = q.x; k[2] = q.y; k[3] = q.z; k[4] = q.w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) k[i + 1] = p0 + i < nnz ? keys[p0 + i] : K;
     }
-    if (p == n - 1) *n_out = pos[p] + keep[p];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fill_gap(ptr, k[i], k[i + 1], (int)(p0 + i));
+}
+
+// ------------------------------------------------ sorted triplets to CSR
+// A run of equal (row, column) is one entry: its head is kept, unless zeros are
+// dropped and the run's sum, in order, is zero.  k_coo_count counts a tile's
+// kept heads; after a scan of the counts k_coo_emit places them and writes
+// rowptr where the row changes.  (Runs of duplicates are short.)
+constexpr int COO_IPT = 16, COO_TILE = TPB * COO_IPT;
+
+// The wave's records base + 64·j + lane, j < COO_IPT: their rows and columns (row M,
+// column -1 past the end), kept[j] = the lanes whose record heads a kept run, sum
+// the runs' sums, and the row before the wave's first record (-1: none).
+__device__ __forceinline__ int coo_runs(int64_t base, int n, int M, const int* __restrict__ srow,
+                                        const int* __restrict__ scol, const float* __restrict__ sval, int drop_zeros,
+                                        int (&row)[COO_IPT], int (&col)[COO_IPT], float (&sum)[COO_IPT],
+                                        uint64_t (&kept)[COO_IPT]) {
+    const int lane = threadIdx.x & 63;
+    float v[COO_IPT];
+#pragma unroll
+    for (int j = 0; j < COO_IPT; ++j) {
+        const int64_t p = base + j * 64 + lane;
+        row[j] = p < n ? srow[p] : M;
+        col[j] = p < n ? scol[p] : -1;
+        v[j] = sval && p < n ? sval[p] : 0.0f;
+    }
+    const int64_t before = base - 1, after = base + 64 * COO_IPT;  // the wave's neighbours
+    const int row_before = before < 0 ? -1 : before < n ? srow[before] : M;
+    int pr = row_before, pc = before >= 0 && before < n ? scol[before] : -1;
+    const int nr = after < n ? srow[after] : M, nc = after < n ? scol[after] : -1;
+    uint64_t head[COO_IPT + 1];
+#pragma unroll
+    for (int j = 0; j < COO_IPT; ++j) {
+        const int ur = __shfl_up(row[j], 1), uc = __shfl_up(col[j], 1);
+        head[j] = __ballot((lane ? ur : pr) != row[j] || (lane ? uc : pc) != col[j]);
+        pr = read_lane(row[j], 63);
+        pc = read_lane(col[j], 63);
+    }
+    head[COO_IPT] = pr != nr || pc != nc ? 1u : 0u;
+#pragma unroll
+    for (int j = 0; j < COO_IPT; ++j) {
+        const int64_t p = base + j * 64 + lane;
+        bool keep = p < n && ((head[j] >> lane) & 1);
+        sum[j] = v[j];
+        if (sval && (~head[j] != 0ull || !(head[j + 1] & 1))) {  // some run has several records (uniform)
+            // lane's run goes on for `len` records here; a run that reaches lane 63 may go on in the next
+            const uint64_t later = lane < 63 ? head[j] >> (lane + 1) : 0ull;
+            const int len = later ? __builtin_ctzll(later) : 63 - lane;
+            for (int k = 1; __ballot(keep && k <= len); ++k) {
+                const float t = __shfl_down(v[j], k);
+                if (k <= len) sum[j] += t;
+            }
+            const bool goes_on = keep && !later && !(head[j + 1] & 1);
+            if (__ballot(goes_on)) {
+                const uint64_t h = j + 1 < COO_IPT ? head[j + 1] : 0ull;
+                if (h) {
+                    for (int k = 0; k < __builtin_ctzll(h); ++k) {
+                        const float t = read_lane(v[j + 1 < COO_IPT ? j + 1 : j], k);
+                        if (goes_on) sum[j] += t;
+                    }
+                } else if (goes_on) {
+                    for (int64_t q = base + (j + 1) * 64; q < n && srow[q] == row[j] && scol[q] == col[j]; ++q)
+                        sum[j] += sval[q];
+                }
+            }
+        }
+        if (drop_zeros && sval) keep = keep && sum[j] != 0.0f;
+        kept[j] = __ballot(keep);
+    }
+    return row_before;
+}
+
+__global__ __launch_bounds__(TPB) void k_coo_count(int n, int M, const int* __restrict__ srow,
+                                                   const int* __restrict__ scol, const float* __restrict__ sval,
+                                                   int drop_zeros, int* __restrict__ cnt) {
+    __shared__ int red[TPB / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int row[COO_IPT], col[COO_IPT];
+    float sum[COO_IPT];
+    uint64_t kept[COO_IPT];
+    coo_runs((int64_t)blockIdx.x * COO_TILE + w * (64 * COO_IPT), n, M, srow, scol, drop_zeros ? sval : nullptr,
+             drop_zeros, row, col, sum, kept);
+    int have = 0;
+#pragma unroll
+    for (int j = 0; j < COO_IPT; ++j) have += __popcll(kept[j]);
+    if (lane == 0) red[w] = have;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int s = 0;
+        for (int q = 0; q < TPB / 64; ++q) s += red[q];
+        cnt[blockIdx.x] = s;
+    }
+}
+
+__global__ void k_coo_empty(int M, int* __restrict__ rowptr, int* __restrict__ n_out) {
+    const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (r <= M) rowptr[r] = 0;
+    if (r == 0) *n_out = 0;
+}
+
+__global__ void k_clear_int(int* p) { *p = 0; }
+
+// first[b]: kept entries before tile b.  Nothing is written when *bad.
+__global__ __launch_bounds__(TPB) void k_coo_emit(int n, int M, const int* __restrict__ srow,
+                                                  const int* __restrict__ scol, const float* __restrict__ sval,
+                                                  int drop_zeros, const int* __restrict__ first,
+                                                  const int* __restrict__ bad, int* __restrict__ rowptr,
+                                                  int* __restrict__ colind, float* __restrict__ val,
+                                                  int* __restrict__ n_out) {
+    __shared__ int red[TPB / 64];
+    if (*bad) return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t lt = (1ull << lane) - 1ull;
+    const int64_t base = (int64_t)blockIdx.x * COO_TILE + w * (64 * COO_IPT);
+    int row[COO_IPT], col[COO_IPT];
+    float sum[COO_IPT];
+    uint64_t kept[COO_IPT];
+    int rbefore = coo_runs(base, n, M, srow, scol, sval, drop_zeros, row, col, sum, kept);
+    int have = 0;
+#pragma unroll
+    for (int j = 0; j < COO_IPT; ++j) have += __popcll(kept[j]);
+    if (lane == 0) red[w] = have;
+    __syncthreads();
+    int at = first[blockIdx.x];
+    for (int q = 0; q < w; ++q) at += red[q];
+#pragma unroll
+    for (int j = 0; j < COO_IPT; ++j) {
+        const int64_t p = base + j * 64 + lane;
+        const int d = at + __popcll(kept[j] & lt);
+        if ((kept[j] >> lane) & 1) {
+            colind[d] = col[j];
+            if (sval) val[d] = sum[j];
+        }
+        // rows up to this record's begin here; past the last record, the rest do
+        const int ur = __shfl_up(row[j], 1);
+        fill_gap(rowptr, lane ? ur : rbefore, row[j], d);
+        rbefore = read_lane(row[j], 63);
+        at += __popcll(kept[j]);
+        if (p == n - 1) *n_out = d + (int)((kept[j] >> lane) & 1);
+    }
+    // the last record ends the last tile's last wave: nothing past it there
+    if (base + 64 * COO_IPT == n) fill_gap(rowptr, lane ? M : rbefore, M, at);
 }
 
 int64_t scan_ws_ints(int64_t n) {
@@ -240,35 +549,83 @@ void exclusive_scan(int64_t n, int* data, int* ws, hipStream_t s) {
     }
 }
 
-// One stable LSD sort of keys (values in [0, range)) carrying positions:
-// idx_in == nullptr sorts positions 0..n-1.  Non-final: sorted keys and
-// positions land in *kout_final / *iout_final (ping-pong buffers A/B).  Final
-// (gather_src != nullptr): the last pass writes gathered[dst] = gather_src[pos]
-// and gvals[dst] = vals[pos] instead of positions.
-void radix_sort(int n, int range, const int* keys_in, const int* idx_in, int* keysA, int* keysB, int* idxA,
-                int* idxB, int* hist, int* scanws, const int* gather_src, const float* vals, int* gathered,
-                float* gvals, const int** kout_final, const int** iout_final, hipStream_t s) {
-    const int nblocks = (int)(((int64_t)n + TILE - 1) / TILE);
-    const int64_t nhist = (int64_t)NB * nblocks;
-    int passes = 1;
-    while (range > 1 && ((range - 1) >> (8 * passes)) > 0) ++passes;
-    const int* kin = keys_in;
-    const int* iin = idx_in;
-    int* kout = keysA;
-    int* iout = idxA;
-    for (int pass = 0; pass < passes; ++pass) {
-        const bool last = gather_src && pass == passes - 1;
-        hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(TPB), 0, s, n, 8 * pass, kin, hist, nblocks);
-        exclusive_scan(nhist, hist, scanws, s);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(TPB), 0, s, n, 8 * pass, kin, iin, hist, nblocks,
-                           kout, iout, gather_src, vals, gathered, gvals, last ? 1 : 0);
-        kin = kout;
-        iin = iout;
-        kout = (kout == keysA) ? keysB : keysA;
-        iout = (iout == idxA) ? idxB : idxA;
+// A sort of n records by keys in [0, range): `passes` passes of `db` bits over
+// tiles of `tile` records.
+struct RadixPlan {
+    int db, passes, tile, ntiles;
+};
+// Tiles of 512 threads × 8 records: longer runs per digit than shorter tiles, yet
+// four workgroups a CU, whose phases overlap (1M R-MAT transpose and 6M triplets to
+// CSR: 2048 records 506 and 401 us, 4096 393 and 373, 8192 430 and 407, 16,384 525
+// and 501; 512 threads against 256 and 1024: 393, 457, 525 us).  With fewer records
+// than RADIX_BIG some CUs would have no such tile, so they are 2,048.
+constexpr int RADIX_BIG = 2 << 20;
+constexpr int RADIX_BIG_TILE = 4096, RADIX_BIG_THREADS = 512;
+
+RadixPlan radix_plan(int n, int range) {
+    int bits = 0;
+    while (bits < 31 && ((int64_t)1 << bits) < range) ++bits;
+    RadixPlan p;
+    p.passes = bits > 0 ? (bits + RADIX_MAX_BITS - 1) / RADIX_MAX_BITS : 1;
+    p.db = (bits + p.passes - 1) / p.passes;
+    if (p.db < RADIX_MIN_BITS) p.db = RADIX_MIN_BITS;
+    p.tile = n >= RADIX_BIG ? RADIX_BIG_TILE : 2048;
+    p.ntiles = (int)(((int64_t)n + p.tile - 1) / p.tile);
+    return p;
+}
+// ints of histogram workspace: the tiles' counts and the digits' totals
+size_t radix_hist_ints(const RadixPlan& p) { return ((size_t)p.ntiles + 1) << p.db; }
+
+struct Records {
+    const int* k;
+    const int* a;
+    const float* v;
+};
+
+template <int THREADS, int IPT>
+void radix_pass(const RadixPlan& p, int pass, int n, const Records& in, bool csr_rows, int M, const int* rowptr,
+                int* hist, int* ko, int* ao, float* vo, const int* other, int krange, int orange, int* bad,
+                hipStream_t s) {
+    const int bins = 1 << p.db, shift = p.db * pass;
+    int* totals = hist + (size_t)p.ntiles * bins;
+    const dim3 grid(xcd_grid(p.ntiles));
+    const size_t lds = radix_lds(THREADS, IPT, bins);
+    hipLaunchKernelGGL((k_radix_hist<THREADS, IPT>), grid, dim3(THREADS), 0, s, n, shift, p.db, p.ntiles, in.k, hist,
+                       other, krange, orange, bad);
+    hipLaunchKernelGGL(k_radix_scan, dim3(bins / 16), dim3(1024), 0, s, p.ntiles, bins, hist, totals);
+#define ARMSP_RADIX(CR, VA)                                                                                        \
+    hipLaunchKernelGGL((k_radix_scatter<THREADS, IPT, CR, VA>), grid, dim3(THREADS), lds, s, n, shift, p.db, p.ntiles, \
+                       in.k, in.a, in.v, M, rowptr, hist, totals, ko, ao, vo)
+    if (csr_rows) {
+        if (in.v) ARMSP_RADIX(true, true); else ARMSP_RADIX(true, false);
+    } else {
+        if (in.v) ARMSP_RADIX(false, true); else ARMSP_RADIX(false, false);
     }
-    *kout_final = kin;
-    *iout_final = iin;
+#undef ARMSP_RADIX
+}
+
+// Stable sort of the records by key.  With rowptr, a is the row of each entry of a
+// CSR matrix.  The passes alternate between buf[0] and buf[1] (k, a, v each; `from`:
+// the one to write first); the last one writes a and v to a_last and v_last when
+// they are given.  Returns the sorted records.  other, krange, orange, bad: the
+// range check of k_radix_hist, done by the first pass.
+Records radix_sort(const RadixPlan& p, int n, Records in, int M, const int* rowptr, int* hist, int* const (*buf)[3],
+                   int from, int* a_last, float* v_last, const int* other, int krange, int orange, int* bad,
+                   hipStream_t s) {
+    for (int pass = 0; pass < p.passes; ++pass) {
+        const bool last = pass == p.passes - 1;
+        int* const* o = buf[(from + pass) & 1];
+        int* ao = last && a_last ? a_last : o[1];
+        float* vo = last && a_last ? v_last : reinterpret_cast<float*>(o[2]);
+        const bool csr = rowptr && pass == 0;
+        const int* chk = pass == 0 ? other : nullptr;
+        if (p.tile == RADIX_BIG_TILE)
+            radix_pass<RADIX_BIG_THREADS, RADIX_BIG_TILE / RADIX_BIG_THREADS>(p, pass, n, in, csr, M, rowptr, hist, o[0], ao, vo, chk, krange, orange, bad, s);
+        else
+            radix_pass<256, 8>(p, pass, n, in, csr, M, rowptr, hist, o[0], ao, vo, chk, krange, orange, bad, s);
+        in = Records{o[0], ao, in.v ? vo : nullptr};
+    }
+    return in;
 }
 
 // ------------------------------------------------ column blocks of a CSR matrix
@@ -461,31 +818,21 @@ extern "C" int armsp_csr_transpose(int M, int K, int nnz, const int* rowptr, con
         t.stop();
         return ARMSP_SUCCESS;
     }
-    const int nblocks = (int)(((int64_t)nnz + TILE - 1) / TILE);
-    const int64_t nhist = (int64_t)NB * nblocks;
-    if (nhist > INT_MAX) return ARMSP_ERROR_NOT_SUPPORTED;
+    const RadixPlan plan = radix_plan(nnz, K);
     const size_t n4 = ((size_t)nnz * 4 + 255) & ~(size_t)255;
-    const size_t h4 = ((size_t)nhist * 4 + 255) & ~(size_t)255;
-    const size_t s4 = ((size_t)scan_ws_ints(nhist) * 4 + 255) & ~(size_t)255;
+    const size_t h4 = (radix_hist_ints(plan) * 4 + 255) & ~(size_t)255;
     void* ws = nullptr;
-    int st = ws_alloc(&ws, 5 * n4 + h4 + s4, s);
+    int st = ws_alloc(&ws, (plan.passes > 2 ? 6 : plan.passes > 1 ? 4 : 1) * n4 + h4, s);
     if (st) return st;
     char* p = static_cast<char*>(ws);
-    int* rows = reinterpret_cast<int*>(p);
-    int* keysA = reinterpret_cast<int*>(p + n4);
-    int* keysB = reinterpret_cast<int*>(p + 2 * n4);
-    int* idxA = reinterpret_cast<int*>(p + 3 * n4);
-    int* idxB = reinterpret_cast<int*>(p + 4 * n4);
-    int* hist = reinterpret_cast<int*>(p + 5 * n4);
-    int* scanws = reinterpret_cast<int*>(p + 5 * n4 + h4);
-
-    hipLaunchKernelGGL(k_expand_rows, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, s, M, rowptr, rows);
-    const int* sorted_keys = nullptr;
-    const int* sorted_idx = nullptr;
-    radix_sort(nnz, K, colind, nullptr, keysA, keysB, idxA, idxB, hist, scanws, rows, val, rowind, valT,
-               &sorted_keys, &sorted_idx, s);
-    hipLaunchKernelGGL(k_colptr, dim3((unsigned)(((int64_t)nnz + 1 + 255) / 256)), dim3(256), 0, s, nnz, K,
-                       sorted_keys, colptr);
+    int* hist = reinterpret_cast<int*>(p);
+    auto arr = [&](int i) { return reinterpret_cast<int*>(p + h4 + i * n4); };
+    // the last pass writes only its keys here; the passes before it, whole records
+    int* const buf[2][3] = {{arr(0), arr(4), arr(5)}, {arr(1), arr(2), arr(3)}};
+    const Records sorted = radix_sort(plan, nnz, Records{colind, nullptr, val}, M, rowptr, hist, buf,
+                                      (plan.passes - 1) & 1, rowind, valT, nullptr, 0, 0, nullptr, s);
+    hipLaunchKernelGGL(k_colptr, dim3((unsigned)(((int64_t)nnz / 4 + 1 + 255) / 256)), dim3(256), 0, s, nnz, K,
+                       sorted.k, colptr);
     hipError_t e = hipGetLastError();
     ws_free(ws, s);
     if (e != hipSuccess) return hip_fail(e);
@@ -502,88 +849,51 @@ extern "C" int armsp_coo_to_csr(int M, int K, int nnz, const int* rows, const in
     if (nnz > 0 && (M == 0 || K == 0)) return ARMSP_ERROR_INVALID_VALUE;
     hipStream_t s = as_stream(stream);
     TimedLaunch t("coo_to_csr", s);
-    const int nblocks = (int)(((int64_t)nnz + TILE - 1) / TILE);
-    const int64_t nhist = (int64_t)NB * (nblocks > 0 ? nblocks : 1);
-    if (nhist > INT_MAX) return ARMSP_ERROR_NOT_SUPPORTED;
-    const int64_t nscan = nhist > nnz ? nhist : (int64_t)nnz;
-    const size_t n4 = ((size_t)(nnz > 0 ? nnz : 1) * 4 + 255) & ~(size_t)255;
-    const size_t h4 = ((size_t)nhist * 4 + 255) & ~(size_t)255;
-    const size_t s4 = ((size_t)scan_ws_ints(nscan) * 4 + 255) & ~(size_t)255;
-    void* ws = nullptr;
-    int st = ws_alloc(&ws, 11 * n4 + h4 + s4 + 256, s);
-    if (st) return st;
-    char* p = static_cast<char*>(ws);
-    int* keysA = reinterpret_cast<int*>(p);
-    int* keysB = reinterpret_cast<int*>(p + n4);
-    int* idxA = reinterpret_cast<int*>(p + 2 * n4);
-    int* idxB = reinterpret_cast<int*>(p + 3 * n4);
-    int* rperm = reinterpret_cast<int*>(p + 4 * n4);
-    int* scol = reinterpret_cast<int*>(p + 5 * n4);
-    float* sval = reinterpret_cast<float*>(p + 6 * n4);
-    float* sums = reinterpret_cast<float*>(p + 7 * n4);
-    int* keep = reinterpret_cast<int*>(p + 8 * n4);
-    int* pos = reinterpret_cast<int*>(p + 9 * n4);
-    int* urow = reinterpret_cast<int*>(p + 10 * n4);
-    int* hist = reinterpret_cast<int*>(p + 11 * n4);
-    int* scanws = reinterpret_cast<int*>(p + 11 * n4 + h4);
-    int* bad = reinterpret_cast<int*>(p + 11 * n4 + h4 + s4);
-    auto fail = [&](int code) {
-        ws_free(ws, s);
-        return code;
-    };
     if (nnz == 0) {
-        hipError_t e = hipMemsetAsync(nnz_out, 0, sizeof(int), s);
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_rowptr_dev, dim3(1), dim3(64), 0, s, (const int*)nnz_out, M, (const int*)nullptr,
-                               rowptr);
-            e = hipGetLastError();
-        }
-        if (e != hipSuccess) return fail(hip_fail(e));
-        ws_free(ws, s);
+        hipLaunchKernelGGL(k_coo_empty, dim3((unsigned)(((int64_t)M + 1 + 255) / 256)), dim3(256), 0, s, M, rowptr,
+                           nnz_out);
+        ARMSP_LAUNCHED();
         t.stop();
         return ARMSP_SUCCESS;
     }
-    // every index in range, or an error before anything is written through one
+    const RadixPlan pc = radix_plan(nnz, K), pr = radix_plan(nnz, M);
+    const size_t hc = radix_hist_ints(pc), hr = radix_hist_ints(pr);
+    const int ctiles = (int)(((int64_t)nnz + COO_TILE - 1) / COO_TILE);
+    const size_t n4 = ((size_t)nnz * 4 + 255) & ~(size_t)255;
+    const size_t h4 = ((hc > hr ? hc : hr) * 4 + 255) & ~(size_t)255;
+    const size_t c4 = ((size_t)ctiles * 4 + 255) & ~(size_t)255;
+    const size_t s4 = ((size_t)scan_ws_ints(ctiles) * 4 + 255) & ~(size_t)255;
+    void* ws = nullptr;
+    int st = ws_alloc(&ws, 6 * n4 + h4 + c4 + s4 + 256, s);
+    if (st) return st;
+    char* p = static_cast<char*>(ws);
+    auto arr = [&](int i) { return reinterpret_cast<int*>(p + i * n4); };
+    int* hist = reinterpret_cast<int*>(p + 6 * n4);
+    int* cnt = reinterpret_cast<int*>(p + 6 * n4 + h4);
+    int* scanws = reinterpret_cast<int*>(p + 6 * n4 + h4 + c4);
+    int* bad = reinterpret_cast<int*>(p + 6 * n4 + h4 + c4 + s4);
+    int* const buf[2][3] = {{arr(0), arr(1), arr(2)}, {arr(3), arr(4), arr(5)}};
+    // by column, then (stably) by row: (row, column) order, duplicates in input order.
+    // The first histogram also checks every index; the sort masks its digits, so it
+    // stays inside its buffers whatever they are, and k_coo_emit writes nothing when
+    // one is out of range: a single wait at the end serves the check.
+    hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, bad);
+    const Records bc = radix_sort(pc, nnz, Records{cols, rows, vals}, 0, nullptr, hist, buf, 0, nullptr, nullptr,
+                                  rows, K, M, bad, s);
+    const Records br = radix_sort(pr, nnz, Records{bc.a, bc.k, bc.v}, 0, nullptr, hist, buf, pc.passes & 1, nullptr,
+                                  nullptr, nullptr, 0, 0, nullptr, s);
+    hipLaunchKernelGGL(k_coo_count, dim3((unsigned)ctiles), dim3(TPB), 0, s, nnz, M, br.k, br.a, br.v,
+                       drop_zeros, cnt);
+    exclusive_scan(ctiles, cnt, scanws, s);
+    hipLaunchKernelGGL(k_coo_emit, dim3((unsigned)ctiles), dim3(TPB), 0, s, nnz, M, br.k, br.a, br.v, drop_zeros,
+                       (const int*)cnt, (const int*)bad, rowptr, colind, val, nnz_out);
     int bad_h = 0;
-    hipError_t e = hipMemsetAsync(bad, 0, sizeof(int), s);
-    const unsigned g1 = (unsigned)(((int64_t)nnz + 255) / 256);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_coo_check, dim3(g1), dim3(256), 0, s, nnz, M, K, rows, cols, bad);
-        e = hipGetLastError();
-    }
+    hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(&bad_h, bad, sizeof(int), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return fail(hip_fail(e));
-    if (bad_h) return fail(ARMSP_ERROR_INVALID_VALUE);
-
-    // by column, then (stably) by row: (row, column) order, duplicates in input order
-    const int* ck = nullptr;
-    const int* ci = nullptr;
-    radix_sort(nnz, K, cols, nullptr, keysA, keysB, idxA, idxB, hist, scanws, nullptr, nullptr, nullptr, nullptr,
-               &ck, &ci, s);
-    hipLaunchKernelGGL(k_gather_keys, dim3(g1), dim3(256), 0, s, nnz, ci, rows, rperm);
-    // the column pass left its positions in idxA or idxB; sort rows into the other pair
-    int* k2a = (ci == idxA) ? keysA : keysB;
-    int* k2b = (ci == idxA) ? keysB : keysA;
-    int* i2a = (ci == idxA) ? idxB : idxA;
-    int* i2b = (ci == idxA) ? idxA : idxB;
-    (void)i2b;
-    const int* srow = nullptr;
-    const int* si = nullptr;
-    radix_sort(nnz, M, rperm, ci, k2a, k2b, i2a, const_cast<int*>(ci), hist, scanws, cols, vals, scol,
-               vals ? sval : nullptr, &srow, &si, s);
-    hipLaunchKernelGGL(k_coo_runs, dim3(g1), dim3(256), 0, s, nnz, srow, scol, vals ? sval : nullptr, sums, keep,
-                       drop_zeros);
-    e = hipMemcpyAsync(pos, keep, (size_t)nnz * sizeof(int), hipMemcpyDeviceToDevice, s);
-    if (e != hipSuccess) return fail(hip_fail(e));
-    exclusive_scan(nnz, pos, scanws, s);
-    hipLaunchKernelGGL(k_coo_compact, dim3(g1), dim3(256), 0, s, nnz, srow, scol, sums, keep, pos, urow, colind,
-                       val, nnz_out);
-    hipLaunchKernelGGL(k_rowptr_dev, dim3((unsigned)(((int64_t)nnz + 1 + 255) / 256)), dim3(256), 0, s,
-                       (const int*)nnz_out, M, urow, rowptr);
-    e = hipGetLastError();
     ws_free(ws, s);
     if (e != hipSuccess) return hip_fail(e);
+    if (bad_h) return ARMSP_ERROR_INVALID_VALUE;
     t.stop();
     return ARMSP_SUCCESS;
 }
