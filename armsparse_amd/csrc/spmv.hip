@@ -10,9 +10,10 @@
 //          between lanes, and a carry per wave is added by a fixup kernel.
 //  VCSR  — the reference's blocked format with its exact summation order:
 //          every row's four partial sums s0..s3 are each added in block order
-//          (by four lanes of a short row, by a wave for a medium row, by a
-//          workgroup for a long one) and the row total is (s0+s2)+(s1+s3), as
+//          (by four lanes of a short row, sixteen of a medium one, a workgroup
+//          for a long one) and the row total is (s0+s2)+(s1+s3), as
 //          vadd/vpadd compute it.
+#include <algorithm>
 #include <climits>
 #include <cstdlib>
 
@@ -281,31 +282,40 @@ __global__ __launch_bounds__(256) void k_spmv_vcsr(int M, const int* __restrict_
 }
 
 // One launch, three walkers: rows of at most VCSR_MED_MIN blocks get four lanes
-// each, rows of up to `long_blocks` blocks a wave each (vcsr_medium_rows), and
+// each, rows of up to `long_blocks` blocks 16 lanes each (vcsr_medium_rows), and
 // longer rows a workgroup each: k_vcsr_find_long lists the medium and the long
-// rows, and workgroups of 256 lanes take listed long rows from a shared counter
-// while the other workgroups of the same launch walk the rest (so the walkers
-// overlap, and the hub rows, listed and started first, are the critical path).  A
-// workgroup walks its row in batches of 256 blocks, one block per lane: each
-// lane keeps the loads of its next D batches in flight (values and x, 16 bytes
-// each; a block's column index one ring further ahead, so no x load waits for
-// its index), stages the block in LDS transposed — one array per position l of
-// the 4-block — and wave 0's lanes 0-3 keep the reference's four partial sums
-// s_l, adding each batch in block order four blocks per LDS read while the
-// next batch is staged into the other LDS buffer.  With the unfused reading
-// the lanes form the rounded products a·b, so lanes 0-3 only add; with the
-// fused one they stage values and x and lanes 0-3 run the fmaf chain.  Either
-// way each s_l sees the reference's sequence of operations: bit-exact.
-constexpr int VCSR_LONG_DEFAULT = 1024;    // 512, 1024, 2048, 4096: 381, 351, 390, 385 us (1M R-MAT)
-constexpr int VCSR_MED_MIN = 16;          // rows of more blocks than this (and at most long_blocks) take a wave each
-constexpr int VCSR_MED_AHEAD = 4;         // steps of 16 blocks in flight per medium-row wave
-constexpr int VCSR_BATCH = 256;           // blocks per batch, one per lane
+// rows, and workgroups take listed long rows from a shared counter while the
+// other workgroups of the same launch walk the rest (so the walkers overlap, and
+// the hub rows, listed first, start first).  A workgroup walks its row in batches of
+// VCSR_BATCH blocks.  Waves 1-3 stage, one block per lane: each lane keeps the
+// loads of its next VCSR_AHEAD batches in flight (values and x, 16 bytes each; a
+// block's column index one ring further ahead, so no x load waits for its index)
+// and puts a block into LDS transposed, one array per position l of the 4-block.
+// Wave 0's lanes 0-3 keep the reference's four partial sums s_l and do nothing but
+// add: a batch in block order, the next VCSR_STEP blocks' terms read from LDS
+// during the adds, while the other waves stage the next batch.  With the unfused
+// reading the staging lanes form the rounded products a·b; with the fused one they
+// stage values and x and lanes 0-3 run the fmaf chain.  Either way each s_l sees the
+// reference's sequence of operations: bit-exact.
+//
+// Bound: the chain of adds of the longest row (27,800 blocks of the 1M R-MAT: 120 us
+// on its own, 10 cycles a block), and for the rest the memory requests in flight,
+// which is why registers count: 62 VGPRs, 8 waves per SIMD, 233 us (222 with the next
+// iteration of a medium row in flight); with 4 batches and 32 blocks ahead 91 VGPRs,
+// 5 waves, 286 us.  (345 us with a wave per medium row
+// and a staging wave that also added.)
+constexpr int VCSR_LONG_DEFAULT = 256;    // calls at 192, 256, 384: 322, 239, 242 us; 2048 rows, 60,000 nonzeros: 24, 25, 29
+constexpr int VCSR_MED_MIN = 16;          // rows of more blocks than this (and at most long_blocks) are medium
+constexpr int VCSR_MED_AHEAD = 4;         // steps of 4 blocks of an iteration of a medium row
+constexpr int VCSR_BATCH = 192;           // blocks per batch, one per lane of the staging waves
+constexpr int VCSR_STEP = 16;             // blocks whose terms the adding wave reads ahead (a batch is 2n steps)
 constexpr int VCSR_PAD = VCSR_BATCH + 4;  // row pitch: lanes 0-3 read from distinct LDS banks
-constexpr int VCSR_AHEAD = 4;             // batches in flight per lane
+constexpr int VCSR_AHEAD = 2;             // batches in flight per lane
 
-// Workgroups of medium-row waves per CU (1M R-MAT, 64.5M padded entries: 1, 2, 4, 8,
-// 16, 32 per CU give 987, 596, 383, 355, 351, 357 us).
+// Workgroups of medium rows per CU (1M R-MAT: 8, 12, 16, 24 per CU give 244, 232, 232,
+// 242 us) and of long rows (1, 2, 3, 4: 310, 233, 234, 244 us).
 constexpr int VCSR_MED_WG_PER_CU = 16;
+constexpr int VCSR_LONG_WG_PER_CU = 2;
 
 // Rows longer than this many blocks take the workgroup-per-row path
 // (ARMSP_VCSR_LONG_BLOCKS overrides it, read once per process).
@@ -318,34 +328,51 @@ int vcsr_long_blocks() {
     return v;
 }
 
-// Lists the long rows (more than long_blocks blocks) in list[0, count[0]) and the
-// medium rows (more than VCSR_MED_MIN blocks, at most long_blocks) in
+// Lists the long rows (more than long_blocks blocks) in list — those over 8 times the
+// limit from the front, count[0] of them, the others from the back, count[3], so that
+// the longest start first (in the order of listing: 255 us, not 231) — and the medium rows (more than VCSR_MED_MIN blocks, at most long_blocks) in
 // list_med[0, count[2]); the order within a list does not matter, each row is
-// summed by one walker.  A workgroup of 1024 rows ranks its listed rows by wave
+// summed by one walker.  A workgroup ranks the listed rows of its 8192 by wave
 // ballots and a scan of the 16 wave counts, and takes its slots with one atomic
-// per list (an atomic per row, or per wave, serialises on the counter: 1.5 ms and
-// 117 us for the 1M R-MAT's 10^5 medium rows).
-constexpr int VCSR_FIND_ROWS = 1024;  // rows per workgroup of k_vcsr_find_long
-
-__global__ __launch_bounds__(VCSR_FIND_ROWS) void k_vcsr_find_long(int M, const int* __restrict__ rowptr,
-                                                                   int long_blocks, int* __restrict__ list,
-                                                                   int* __restrict__ list_med,
-                                                                   int* __restrict__ count) {
-    constexpr int NW = VCSR_FIND_ROWS / 64;
-    __shared__ int s_off[2][NW];  // per wave: its rows' first slot within the workgroup
-    __shared__ int s_base[2];     // the workgroup's first slot in each list
-    const int r = blockIdx.x * VCSR_FIND_ROWS + threadIdx.x;
-    const int n = r < M ? rowptr[r + 1] - rowptr[r] : 0;
-    const bool is_long = r < M && n > 4 * long_blocks;
-    const bool is_med = r < M && !is_long && n > 4 * VCSR_MED_MIN;
-    const uint64_t bl = __ballot(is_long), bm = __ballot(is_med);
+// per list: atomics on one counter follow each other at about 15 ns (one per row
+// 1.5 ms for the 1M R-MAT's 10^5 medium rows, one per wave 117 us, one per 1024
+// rows 13 us, one per 8192 8 us).
+constexpr int VCSR_FIND_THREADS = 1024;
+// Rows per thread: 8, or 1 for matrices of few workgroups.
+template <int R>
+__global__ __launch_bounds__(VCSR_FIND_THREADS) void k_vcsr_find_long(int M, const int* __restrict__ rowptr,
+                                                                      int long_blocks, int* __restrict__ list,
+                                                                      int* __restrict__ list_med,
+                                                                      int* __restrict__ count) {
+    constexpr int NW = VCSR_FIND_THREADS / 64;
+    __shared__ int s_off[3][NW];  // per wave: its rows' first slot within the workgroup
+    __shared__ int s_base[3];     // the workgroup's first slot in each list
     const int lane = (int)__lane_id(), wid = (int)(threadIdx.x >> 6);
+    const int64_t r0 = (int64_t)blockIdx.x * (VCSR_FIND_THREADS * R) + wid * (64 * R) + lane;
+    uint64_t bh[R], bl[R], bm[R];
+    int n[R], nh = 0, nl = 0, nm = 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int64_t r = r0 + 64 * j;
+        n[j] = r < M ? rowptr[r + 1] - rowptr[r] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const bool is_long = n[j] > 4 * long_blocks, is_huge = n[j] / 32 > long_blocks;
+        bh[j] = __ballot(is_huge);
+        bl[j] = __ballot(is_long && !is_huge);
+        bm[j] = __ballot(!is_long && n[j] > 4 * VCSR_MED_MIN);
+        nh += __popcll(bh[j]);
+        nl += __popcll(bl[j]);
+        nm += __popcll(bm[j]);
+    }
     if (lane == 0) {
-        s_off[0][wid] = __popcll(bl);
-        s_off[1][wid] = __popcll(bm);
+        s_off[0][wid] = nh;
+        s_off[1][wid] = nl;
+        s_off[2][wid] = nm;
     }
     __syncthreads();
-    if (threadIdx.x < 2) {
+    if (threadIdx.x < 3) {
         const int t = (int)threadIdx.x;
         int acc = 0;
         for (int w = 0; w < NW; ++w) {
@@ -353,206 +380,287 @@ __global__ __launch_bounds__(VCSR_FIND_ROWS) void k_vcsr_find_long(int M, const 
             s_off[t][w] = acc;
             acc += c;
         }
-        s_base[t] = acc > 0 ? atomicAdd(&count[t == 0 ? 0 : 2], acc) : 0;
+        s_base[t] = acc > 0 ? atomicAdd(&count[t == 0 ? 0 : t == 1 ? 3 : 2], acc) : 0;
     }
     __syncthreads();
-    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    if (is_long) list[s_base[0] + s_off[0][wid] + __popcll(bl & below)] = r;
-    if (is_med) list_med[s_base[1] + s_off[1][wid] + __popcll(bm & below)] = r;
+    const uint64_t below = (1ull << lane) - 1ull;
+    int ah = s_base[0] + s_off[0][wid], al = s_base[1] + s_off[1][wid], am = s_base[2] + s_off[2][wid];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int r = (int)(r0 + 64 * j);
+        if ((bh[j] >> lane) & 1) list[ah + __popcll(bh[j] & below)] = r;
+        if ((bl[j] >> lane) & 1) list[M - 1 - (al + __popcll(bl[j] & below))] = r;
+        if ((bm[j] >> lane) & 1) list_med[am + __popcll(bm[j] & below)] = r;
+        ah += __popcll(bh[j]);
+        al += __popcll(bl[j]);
+        am += __popcll(bm[j]);
+    }
 }
 
-// count[0] = listed long rows, count[1] = the long rows' work counter, count[2] =
-// listed medium rows
+// count[0], count[3] = long rows listed from the front and from the back, count[1] =
+// the long rows' work counter, count[2] = listed medium rows
 __global__ void k_zero_count(int* count) {
     count[0] = 0;
     count[1] = 0;
     count[2] = 0;
+    count[3] = 0;
 }
 
-// Medium rows, one wave each: wave gw of nmw takes list_med[gw], list_med[gw + nmw],
-// ... (a fixed assignment, no shared counter).  A step covers 16 blocks, lane
-// 4q + l holding position l of block q; each lane keeps its next VCSR_MED_AHEAD
-// steps' value and x loads in flight (the column index one ring further ahead).
+// Medium rows, a DPP row of 16 lanes each, four rows a wave: group gg of ngg takes
+// list_med[gg], list_med[gg + ngg], ... (a fixed assignment, no shared counter), each
+// at its own pace.  A step covers 4 blocks, lane 4q + l holding position l of block
+// q, and an iteration VCSR_MED_AHEAD steps.  The next iteration's values and x (of the
+// next row, when this one ends) are in flight during an iteration's adds, and the
+// column indices of the one after it behind them.
 // The lanes form the rounded products (the unfused reading) or keep value and x
-// (fused), and lane l's partial sum s_l takes block 0..15's position-l term by a
-// shuffle from lane 4q + l, in block order: the reference's sequence of
-// operations per s_l, as in the other walkers.
+// (fused); the four partial sums travel round the 16 lanes, four lanes on per block,
+// and add each block's term where they find it: s = rotate(s) + p, one DPP add a
+// block, the reference's sequence of operations per s_l, as in the other walkers.
+// (A wave per row that fetched each block's terms by a shuffle was bound by the LDS
+// crossbar: rows of 17-256 blocks of the 1M R-MAT, 31M padded entries, took 201 us.)
+__device__ __forceinline__ float rotate4(float s) {  // lane i of each 16 gets lane i - 4's
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x124, 0xf, 0xf, false));
+}
+
 template <bool FUSED>
-__device__ void vcsr_medium_rows(int gw, int nmw, const int* __restrict__ list_med, const int* __restrict__ count,
+__device__ void vcsr_medium_rows(int gg, int ngg, const int* __restrict__ list_med, const int* __restrict__ count,
                                  const int* __restrict__ rowptr, const int* __restrict__ colind,
                                  const float* __restrict__ val, const float* __restrict__ x, float* __restrict__ y) {
     constexpr int D = VCSR_MED_AHEAD;
-    const int lane = threadIdx.x & 63;
-    const int q = lane >> 2, l = lane & 3;
+    constexpr int IT = 4 * D;  // blocks of an iteration
+    const int q = (threadIdx.x >> 2) & 3, l = threadIdx.x & 3;
     const int nmed = __builtin_amdgcn_readfirstlane(count[2]);
-    for (int i = gw; i < nmed; i += nmw) {
-        const int r = __builtin_amdgcn_readfirstlane(list_med[i]);
-        const int beg = __builtin_amdgcn_readfirstlane(rowptr[r]);
-        const int nb = (__builtin_amdgcn_readfirstlane(rowptr[r + 1]) - beg) >> 2;
-        const int nsteps = (nb + 15) >> 4;
-        auto col_of = [&](int k) {
-            const int b = k * 16 + q;
-            return b < nb ? colind[beg + 4 * b] : 0;
-        };
-        auto fetch = [&](int k, int c, float& v, float& xv) {
-            const int b = k * 16 + q;
-            v = 0.0f;
-            xv = 0.0f;
-            if (b < nb) {
-                v = val[beg + 4 * b + l];
-                xv = x[c + l];
-            }
-        };
-        int rc[D];
-        float rv[D], rx[D];
-#pragma unroll
-        for (int u = 0; u < D; ++u) rc[u] = col_of(u);
+    // row i of the list; past its end no blocks (row 0's index, so every load stays in bounds)
+    auto row_at = [&](int i) { return i < nmed ? list_med[i] : 0; };
+    auto blocks_of = [&](int i, int r, int b) { return i < nmed ? (rowptr[r + 1] - b) >> 2 : 0; };
+    auto columns = [&](int beg, int nb, int pos, int (&c)[D]) {
 #pragma unroll
         for (int u = 0; u < D; ++u) {
-            fetch(u, rc[u], rv[u], rx[u]);
-            rc[u] = col_of(u + D);
+            const int b = pos + 4 * u + q;
+            c[u] = b < nb ? colind[beg + 4 * b] : 0;
         }
-        float s = 0.0f;
-        for (int k0 = 0; k0 < nsteps; k0 += D) {
+    };
+    auto terms = [&](int beg, int nb, int pos, const int (&c)[D], float (&v)[D], float (&xv)[D]) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+            const int b = pos + 4 * u + q;
+            v[u] = 0.0f;
+            xv[u] = 0.0f;
+            if (b < nb) {
+                v[u] = val[beg + 4 * b + l];
+                xv[u] = x[c[u] + l];
+            }
+        }
+    };
+    // the group's row, the two after it, and the index of the third
+    int i = gg;
+    int r0 = row_at(i), r1 = row_at(i + ngg), r2 = row_at(i + 2 * ngg), r3 = row_at(i + 3 * ngg);
+    int b0 = rowptr[r0], b1 = rowptr[r1], b2 = rowptr[r2];
+    int n0 = blocks_of(i, r0, b0), n1 = blocks_of(i + ngg, r1, b1), n2 = blocks_of(i + 2 * ngg, r2, b2);
+    float y0 = y[r0], y1 = y[r1];
+    int pos = 0, c[D];
+    float v[D], xv[D];
+    columns(b0, n0, 0, c);
+    terms(b0, n0, 0, c, v, xv);
+    // the next iteration: of this row, or the first of the next
+    bool last = IT >= n0;
+    columns(last ? b1 : b0, last ? n1 : n0, last ? 0 : IT, c);
+    float s = 0.0f;
+    while (__ballot(i < nmed) != 0ull) {
+        const int bn = last ? b1 : b0, nn = last ? n1 : n0, pn = last ? 0 : pos + IT;
+        float vn[D], xn[D];
+        terms(bn, nn, pn, c, vn, xn);  // the next iteration's terms, and behind them the
+        const bool lastn = pn + IT >= nn;  // column indices of the one after it
+        columns(!lastn ? bn : last ? b2 : b1, !lastn ? nn : last ? n2 : n1, lastn ? 0 : pn + IT, c);
+        if (__ballot(pos + IT > n0) == 0ull) {
 #pragma unroll
             for (int u = 0; u < D; ++u) {
-                const int k = k0 + u;
-                if (k >= nsteps) break;  // uniform: nsteps is the wave's
-                const int cnt = min(16, nb - k * 16);
-                const float pv = rv[u], px = rx[u];
-                float p = 0.0f;
-                if constexpr (!FUSED) p = unfused_product(pv, px);  // vmlaq_f32 rounds the product on its own
-                fetch(k + D, rc[u], rv[u], rx[u]);  // in flight for D steps
-                rc[u] = col_of(k + 2 * D);
+                const float p = FUSED ? 0.0f : unfused_product(v[u], xv[u]);
 #pragma unroll
-                for (int b = 0; b < 16; ++b) {
-                    if (b < cnt) {  // uniform
-                        if constexpr (FUSED) {
-                            const float a = __shfl(pv, 4 * b + l);
-                            const float c = __shfl(px, 4 * b + l);
-                            s = fmaf(a, c, s);
-                        } else {
-                            s = __fadd_rn(s, __shfl(p, 4 * b + l));
-                        }
-                    }
+                for (int j = 0; j < 4; ++j) {
+                    const float t = rotate4(s);
+                    s = FUSED ? fmaf(v[u], xv[u], t) : __fadd_rn(t, p);
+                }
+            }
+        } else {  // a row ends among these blocks: past it the sums only move on
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                const float p = FUSED ? 0.0f : unfused_product(v[u], xv[u]);
+                const bool in = pos + 4 * u + q < n0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float t = rotate4(s);
+                    s = !in ? t : FUSED ? fmaf(v[u], xv[u], t) : __fadd_rn(t, p);
                 }
             }
         }
-        // every lane group now holds s0..s3 of the row
-        const float t = __fadd_rn(s, __shfl_xor(s, 2, 4));   // lanes 0/2: s0+s2, lanes 1/3: s1+s3
+        // whole steps: the sums are in lanes 12-15 of the group
+        const float t = __fadd_rn(s, __shfl_xor(s, 2, 4));    // lanes 0/2: s0+s2, lanes 1/3: s1+s3
         const float tot = __fadd_rn(t, __shfl_xor(t, 1, 4));  // (s0+s2)+(s1+s3)
-        if (lane == 0) y[r] = __fadd_rn(y[r], tot);
+        if (last) {
+            if (i < nmed && q == 3 && l == 0) y[r0] = __fadd_rn(y0, tot);
+            i += ngg;
+            s = 0.0f;
+            r0 = r1;
+            b0 = b1;
+            n0 = n1;
+            y0 = y1;
+            r1 = r2;
+            b1 = b2;
+            n1 = n2;
+            y1 = y[r1];
+            r2 = r3;
+            b2 = rowptr[r2];
+            n2 = blocks_of(i + 2 * ngg, r2, b2);
+            r3 = row_at(i + 3 * ngg);
+        }
+        pos = pn;
+        last = lastn;
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+            v[u] = vn[u];
+            xv[u] = xn[u];
+        }
     }
 }
 
 template <bool FUSED>
-__device__ void vcsr_long_rows(const int* __restrict__ list, int* __restrict__ count,
+__device__ void vcsr_long_rows(int M, const int* __restrict__ list, int* __restrict__ count,
                                const int* __restrict__ rowptr, const int* __restrict__ colind,
                                const float* __restrict__ val, const float* __restrict__ x, float* __restrict__ y,
                                float (*s_a)[4][VCSR_PAD], float (*s_b)[4][VCSR_PAD], int* s_row) {
     constexpr int D = VCSR_AHEAD;
-    const int t = threadIdx.x;
-    const int nlong = count[0];
+    const int t = (int)threadIdx.x - 64;  // staging lane of waves 1-3; wave 0 adds
+    const int l = (int)threadIdx.x & 3;
+    const int nfront = count[0], nlong = nfront + count[3];
     while (true) {
-        if (t == 0) *s_row = atomicAdd(&count[1], 1);
+        if (threadIdx.x == 0) *s_row = atomicAdd(&count[1], 1);
         __syncthreads();
         const int i = *s_row;
         __syncthreads();  // every lane has read the row before lane 0 takes the next
         if (i >= nlong) break;  // the same for the whole workgroup once the list is drained
-        const int r = list[i];
+        const int r = list[i < nfront ? i : M - 1 - (i - nfront)];
         const int beg = rowptr[r];
         const int nb = (rowptr[r + 1] - beg) >> 2;
         const int nbat = (nb + VCSR_BATCH - 1) / VCSR_BATCH;
-        // lane t owns block k·256 + t of batch k
-        auto col_of = [&](int k) {
-            const int b = k * VCSR_BATCH + t;
-            return b < nb ? colind[beg + 4 * b] : -1;
-        };
-        float4 rv[D], rx[D];
-        int rc[D];
-        auto fetch = [&](int k, int c, float4& v, float4& xv) {
-            const int b = k * VCSR_BATCH + t;
-            v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            xv = v;
-            if (b < nb) {
-                v = *reinterpret_cast<const float4*>(val + beg + 4 * b);
-                xv = *reinterpret_cast<const float4*>(x + c);
-            }
-        };
+        if (t >= 0) {
+            // lane t owns block k·VCSR_BATCH + t of batch k
+            auto col_of = [&](int k) {
+                const int b = k * VCSR_BATCH + t;
+                return b < nb ? colind[beg + 4 * b] : -1;
+            };
+            float4 rv[D], rx[D];
+            int rc[D];
+            auto fetch = [&](int k, int c, float4& v, float4& xv) {
+                const int b = k * VCSR_BATCH + t;
+                v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                xv = v;
+                if (b < nb) {
+                    v = *reinterpret_cast<const float4*>(val + beg + 4 * b);
+                    xv = *reinterpret_cast<const float4*>(x + c);
+                }
+            };
 #pragma unroll
-        for (int u = 0; u < D; ++u) rc[u] = col_of(u);
-#pragma unroll
-        for (int u = 0; u < D; ++u) {
-            fetch(u, rc[u], rv[u], rx[u]);
-            rc[u] = col_of(u + D);
-        }
-        float s = 0.0f;
-        for (int k0 = 0; k0 < nbat; k0 += D) {
+            for (int u = 0; u < D; ++u) rc[u] = col_of(u);
 #pragma unroll
             for (int u = 0; u < D; ++u) {
-                const int k = k0 + u;
-                if (k >= nbat) break;  // uniform: nbat is the workgroup's
-                const int buf = k & 1;
-                if constexpr (FUSED) {
-                    s_a[buf][0][t] = rv[u].x;
-                    s_a[buf][1][t] = rv[u].y;
-                    s_a[buf][2][t] = rv[u].z;
-                    s_a[buf][3][t] = rv[u].w;
-                    s_b[buf][0][t] = rx[u].x;
-                    s_b[buf][1][t] = rx[u].y;
-                    s_b[buf][2][t] = rx[u].z;
-                    s_b[buf][3][t] = rx[u].w;
-                } else {  // vmlaq_f32 rounds the product on its own
-                    s_a[buf][0][t] = unfused_product(rv[u].x, rx[u].x);
-                    s_a[buf][1][t] = unfused_product(rv[u].y, rx[u].y);
-                    s_a[buf][2][t] = unfused_product(rv[u].z, rx[u].z);
-                    s_a[buf][3][t] = unfused_product(rv[u].w, rx[u].w);
-                }
-                fetch(k + D, rc[u], rv[u], rx[u]);  // in flight for D batches
-                rc[u] = col_of(k + 2 * D);
-                // batch k staged; wave 0 has also finished adding batch k-1, whose
-                // buffer batch k+1 is about to overwrite
-                __syncthreads();
-                if (t < 4) {
-                    const int cnt = min(VCSR_BATCH, nb - k * VCSR_BATCH);
-                    const float* pa = &s_a[buf][t][0];
-                    const float* pb = &s_b[buf][FUSED ? t : 0][0];
-                    int b = 0;
-                    for (; b + 4 <= cnt; b += 4) {
-                        const float4 a4 = *reinterpret_cast<const float4*>(pa + b);
-                        if constexpr (FUSED) {
-                            const float4 x4 = *reinterpret_cast<const float4*>(pb + b);
-                            s = fmaf(a4.x, x4.x, s);
-                            s = fmaf(a4.y, x4.y, s);
-                            s = fmaf(a4.z, x4.z, s);
-                            s = fmaf(a4.w, x4.w, s);
-                        } else {
-                            s = __fadd_rn(s, a4.x);
-                            s = __fadd_rn(s, a4.y);
-                            s = __fadd_rn(s, a4.z);
-                            s = __fadd_rn(s, a4.w);
-                        }
+                fetch(u, rc[u], rv[u], rx[u]);
+                rc[u] = col_of(u + D);
+            }
+            for (int k0 = 0; k0 < nbat; k0 += D) {
+#pragma unroll
+                for (int u = 0; u < D; ++u) {
+                    const int k = k0 + u;
+                    if (k >= nbat) break;  // uniform: nbat is the workgroup's
+                    const int buf = k & 1;
+                    if constexpr (FUSED) {
+                        s_a[buf][0][t] = rv[u].x;
+                        s_a[buf][1][t] = rv[u].y;
+                        s_a[buf][2][t] = rv[u].z;
+                        s_a[buf][3][t] = rv[u].w;
+                        s_b[buf][0][t] = rx[u].x;
+                        s_b[buf][1][t] = rx[u].y;
+                        s_b[buf][2][t] = rx[u].z;
+                        s_b[buf][3][t] = rx[u].w;
+                    } else {  // vmlaq_f32 rounds the product on its own
+                        s_a[buf][0][t] = unfused_product(rv[u].x, rx[u].x);
+                        s_a[buf][1][t] = unfused_product(rv[u].y, rx[u].y);
+                        s_a[buf][2][t] = unfused_product(rv[u].z, rx[u].z);
+                        s_a[buf][3][t] = unfused_product(rv[u].w, rx[u].w);
                     }
-                    for (; b < cnt; ++b) {
-                        if constexpr (FUSED)
-                            s = fmaf(pa[b], pb[b], s);
-                        else
-                            s = __fadd_rn(s, pa[b]);
-                    }
+                    fetch(k + D, rc[u], rv[u], rx[u]);  // in flight for D batches
+                    rc[u] = col_of(k + 2 * D);
+                    // batch k staged; wave 0 has also finished adding batch k-1, whose
+                    // buffer batch k+1 is about to overwrite
+                    __syncthreads();
                 }
             }
-        }
-        if (t < 64) {  // wave 0: lanes 0-3 hold s0..s3
+        } else {
+            // 32 blocks a step, the next step's LDS reads in flight during the adds (a batch
+            // holds whole steps, so a read past the row's end stays inside the batch)
+            __builtin_amdgcn_s_setprio(3);  // the chain of adds is the row's time: first in the SIMD's queue
+            float s = 0.0f;
+            for (int k = 0; k < nbat; ++k) {
+                __syncthreads();
+                const int cnt = min(VCSR_BATCH, nb - k * VCSR_BATCH);
+                const float4* pa = reinterpret_cast<const float4*>(&s_a[k & 1][l][0]);
+                const float4* pb = reinterpret_cast<const float4*>(&s_b[FUSED ? (k & 1) : 0][FUSED ? l : 0][0]);
+                constexpr int Q = VCSR_STEP / 4;
+                float4 a0[Q], a1[Q], b0[FUSED ? Q : 1], b1[FUSED ? Q : 1];
+                auto read = [&](int at, float4 (&a)[Q], float4 (&b)[FUSED ? Q : 1]) {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        a[q] = pa[at + q];
+                        if constexpr (FUSED) b[q] = pb[at + q];
+                    }
+                };
+                auto one = [&](float a, float b) {
+                    if constexpr (FUSED)
+                        s = fmaf(a, b, s);
+                    else
+                        s = __fadd_rn(s, a);
+                };
+                auto add = [&](int at, const float4 (&a)[Q], const float4 (&b)[FUSED ? Q : 1]) {
+                    if (4 * at + VCSR_STEP <= cnt) {
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) {
+                            const float4 w = b[FUSED ? q : 0];
+                            one(a[q].x, w.x);
+                            one(a[q].y, w.y);
+                            one(a[q].z, w.z);
+                            one(a[q].w, w.w);
+                        }
+                    } else {  // the row's last blocks (uniform tests)
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) {
+                            const float4 w = b[FUSED ? q : 0];
+                            if (4 * (at + q) + 0 < cnt) one(a[q].x, w.x);
+                            if (4 * (at + q) + 1 < cnt) one(a[q].y, w.y);
+                            if (4 * (at + q) + 2 < cnt) one(a[q].z, w.z);
+                            if (4 * (at + q) + 3 < cnt) one(a[q].w, w.w);
+                        }
+                    }
+                };
+                read(0, a0, b0);
+                for (int at = 0; 4 * at < cnt; at += 2 * Q) {
+                    read(at + Q, a1, b1);
+                    add(at, a0, b0);
+                    if (at + 2 * Q < VCSR_BATCH / 4) read(at + 2 * Q, a0, b0);
+                    add(at + Q, a1, b1);
+                }
+            }
+            // lanes 0-3 hold s0..s3
             const float tt = __fadd_rn(s, __shfl_xor(s, 2, 4));  // lanes 0/2: s0+s2, lanes 1/3: s1+s3
             const float tot = __fadd_rn(tt, __shfl_xor(tt, 1, 4));  // (s0+s2)+(s1+s3)
-            if (t == 0) y[r] = __fadd_rn(y[r], tot);
+            if (threadIdx.x == 0) y[r] = __fadd_rn(y[r], tot);
+            __builtin_amdgcn_s_setprio(0);
         }
         __syncthreads();  // the LDS buffers are free for the next row
     }
 }
 
 // One launch: workgroups [0, n_long_wg) walk the listed long rows, the next
-// n_med_wg the listed medium rows (a wave each), the rest the short rows (64 per
+// n_med_wg the listed medium rows (16 lanes each), the rest the short rows (64 per
 // workgroup).
 template <bool FUSED>
 __global__ __launch_bounds__(256) void k_spmv_vcsr_split(int M, const int* __restrict__ rowptr,
@@ -566,13 +674,13 @@ __global__ __launch_bounds__(256) void k_spmv_vcsr_split(int M, const int* __res
     __shared__ int s_row;
     const int b = (int)blockIdx.x;
     if (b < n_long_wg) {
-        vcsr_long_rows<FUSED>(list, count, rowptr, colind, val, x, y, s_a,
+        vcsr_long_rows<FUSED>(M, list, count, rowptr, colind, val, x, y, s_a,
                               reinterpret_cast<float (*)[4][VCSR_PAD]>(&s_b[0][0][0]), &s_row);
         return;
     }
     if (b < n_long_wg + n_med_wg) {
-        const int gw = (b - n_long_wg) * 4 + (int)(threadIdx.x >> 6);
-        vcsr_medium_rows<FUSED>(gw, n_med_wg * 4, list_med, count, rowptr, colind, val, x, y);
+        const int gg = (b - n_long_wg) * 16 + (int)(threadIdx.x >> 4);
+        vcsr_medium_rows<FUSED>(gg, n_med_wg * 16, list_med, count, rowptr, colind, val, x, y);
         return;
     }
     // the short walker takes what neither list holds: rows of at most VCSR_MED_MIN
@@ -700,11 +808,11 @@ int armsp_spmv_vcsr_f32(int M, int nnz_padded, const int* rowptr, const int* col
         return launch_merge<8>(M, nnz_padded, rowptr, colind, val, x, y, ARMSP_ACCUMULATE, s);
     }
     const int fused = (flags & ARMSP_FUSED_MLA) ? 1 : 0;
-    // Rows of more than VCSR_MED_MIN blocks take a wave each, rows of more than
+    // Rows of more than VCSR_MED_MIN blocks take 16 lanes each, rows of more than
     // long_blocks a workgroup each; the workgroup walker's 16-byte loads need
     // 16-byte-aligned values and x (VCSR rows hold whole 4-blocks and block columns
     // are multiples of 4, so rowptr entries and the gathered x offsets are multiples
-    // of 4 as well), so with unaligned operands every long row goes to the waves.
+    // of 4 as well), so with unaligned operands every long row is a medium one.
     const bool aligned = ((uintptr_t)val % 16) == 0 && ((uintptr_t)x % 16) == 0;
     // (a long-row limit below VCSR_MED_MIN acts as VCSR_MED_MIN: rows up to it are the short walker's)
     const int lb = vcsr_long_blocks();
@@ -721,15 +829,20 @@ int armsp_spmv_vcsr_f32(int M, int nnz_padded, const int* rowptr, const int* col
         list = count + 64;
         list_med = list + M;
         hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, s, count);
-        hipLaunchKernelGGL(k_vcsr_find_long, dim3((unsigned)((M + VCSR_FIND_ROWS - 1) / VCSR_FIND_ROWS)),
-                           dim3(VCSR_FIND_ROWS), 0, s, M, rowptr,
-                           long_blocks, list, list_med, count);
+        if (M <= 128 * VCSR_FIND_THREADS)
+            hipLaunchKernelGGL((k_vcsr_find_long<1>), dim3((unsigned)((M + VCSR_FIND_THREADS - 1) / VCSR_FIND_THREADS)),
+                               dim3(VCSR_FIND_THREADS), 0, s, M, rowptr, long_blocks, list, list_med, count);
+        else
+            hipLaunchKernelGGL((k_vcsr_find_long<8>),
+                               dim3((unsigned)(((int64_t)M + 8 * VCSR_FIND_THREADS - 1) / (8 * VCSR_FIND_THREADS))),
+                               dim3(VCSR_FIND_THREADS), 0, s, M, rowptr, long_blocks, list, list_med, count);
     }
     TimedLaunch t("spmv_vcsr", s);
     const unsigned short_wg = (unsigned)(((int64_t)M * 4 + 255) / 256);
     if (split_long) {  // long-row workgroups first (the hub rows are the critical path), then medium-row waves
-        const int n_long_wg = 2 * device_cus();
-        const int n_med_wg = VCSR_MED_WG_PER_CU * device_cus();
+        // (no more workgroups than rows: a small matrix would wait for idle ones)
+        const int n_long_wg = std::min(VCSR_LONG_WG_PER_CU * device_cus(), M);
+        const int n_med_wg = std::min(VCSR_MED_WG_PER_CU * device_cus(), (M + 15) / 16);
         const dim3 grid((unsigned)(n_long_wg + n_med_wg) + short_wg);
         if (fused)
             hipLaunchKernelGGL(k_spmv_vcsr_split<true>, grid, dim3(256), 0, s, M, rowptr, colind, val, x, y, list,
