@@ -104,6 +104,7 @@ _SIGS = {
     "armsp_spmm_fp8": (c_int, [_I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _CFG, _P]),
     "armsp_spmm_ex": (c_int, [_I, _I, _I, _I, _P, _P, _P, _I, _P, _P, _I, _P, _I, _I, POINTER(Epilogue), _CFG,
                               _P]),
+    "armsp_spmm_bf16_out": (c_int, [_I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _I, POINTER(Epilogue), _P]),
     "armsp_spmv_f32": (c_int, [_I, _I, _I, _P, _P, _P, _P, _P, _I, _CFG, _P]),
     "armsp_spmv_vcsr_f32": (c_int, [_I, _I, _P, _P, _P, _P, _P, _I, _P]),
     "armsp_sddmm_csr_f32": (c_int, [_I, _I, _I, _I, _P, _P, _P, _P, _I, _P, _I, _P, _CFG, _P]),
@@ -121,6 +122,7 @@ _SIGS = {
     "armsp_gemm_bf16_ex": (c_int, [_I, _I, _I, _P, c_int64, c_int64, _P, c_int64, c_int64, _P, _I, c_int64, _I, _P]),
     "armsp_convert_f32_to_bf16": (c_int, [c_int64, _P, _P, _P]),
     "armsp_convert_rows_f32_to_bf16": (c_int, [_I, _I, _P, c_int64, _P, c_int64, _P]),
+    "armsp_convert_rows_colsum_bf16": (c_int, [_I, _I, _P, c_int64, _P, c_int64, _P, _P]),
     "armsp_quantize_fp8_rows": (c_int, [_I, _I, _P, _I, _P, _P, _P]),
     "armsp_dequantize_fp8_rows": (c_int, [_I, _I, _P, _I, _P, _P, _I, _P]),
     "armsp_fill_uniform_f32": (c_int, [c_int64, c_uint64, c_uint64, c_float, c_float, _P, _P]),

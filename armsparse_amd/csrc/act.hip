@@ -127,6 +127,57 @@ __global__ __launch_bounds__(256) void k_act_backward(int M, int N, int R, const
     }
 }
 
+// Rows [b·R, (b+1)·R) of x to bf16, 8 columns per thread, with the block's fp32 column
+// sums in part[b][·]: k_act_backward's layout without the mask.  HBM-bound: it reads 4
+// and writes 2 bytes a value, where a conversion and a separate column sum read x
+// twice (170,000 x 256: 145 us for the two, 47 + 10 for this).
+__global__ __launch_bounds__(256) void k_rows_colsum(int M, int N, int R, const float* __restrict__ X, int64_t ldx,
+                                                     uint16_t* __restrict__ Y, int64_t ldy,
+                                                     float* __restrict__ part) {
+    extern __shared__ float s_acc[];  // [P][N]
+    constexpr int U = 4;
+    const int ipr = N >> 3;
+    const int P = 256 / ipr;
+    const int t = threadIdx.x;
+    const int cg = t % ipr, ph = t / ipr;
+    const int64_t r0 = (int64_t)blockIdx.x * R;
+    const int64_t r1 = r0 + R < M ? r0 + R : M;
+    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (ph < P) {
+        for (int64_t m0 = r0 + ph; m0 < r1; m0 += U * P) {
+            float4 a[U], b[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t m = m0 + u * P < r1 ? m0 + u * P : m0;
+                const float4* src = reinterpret_cast<const float4*>(X + m * ldx + cg * 8);
+                a[u] = src[0];
+                b[u] = src[1];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (m0 + u * P >= r1) break;
+                const float v[8] = {a[u].x, a[u].y, a[u].z, a[u].w, b[u].x, b[u].y, b[u].z, b[u].w};
+                uint32_t o[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    acc[2 * j] += v[2 * j];
+                    acc[2 * j + 1] += v[2 * j + 1];
+                    o[j] = (uint32_t)f32_to_bf16_rne(v[2 * j]) | (uint32_t)f32_to_bf16_rne(v[2 * j + 1]) << 16;
+                }
+                *reinterpret_cast<uint4*>(Y + (m0 + u * P) * ldy + cg * 8) = make_uint4(o[0], o[1], o[2], o[3]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s_acc[ph * N + cg * 8 + j] = acc[j];
+    }
+    __syncthreads();
+    for (int n = t; n < N; n += 256) {
+        float sum = 0.0f;
+        for (int q = 0; q < P; ++q) sum += s_acc[q * N + n];
+        part[(int64_t)blockIdx.x * N + n] = sum;
+    }
+}
+
 // out[n] = Σ_b part[b][n]: 16 columns × 16 phases per block, phases joined in
 // order; 8 loads in flight ahead of each thread's in-order adds.
 __global__ __launch_bounds__(256) void k_parts_sum(int nb, int N, const float* __restrict__ part,
@@ -222,6 +273,34 @@ int armsp_bias_relu_dropout_backward_bf16(int M, int N, const uint16_t* G, const
         e = hipGetLastError();
     }
     if (ws) ws_free(ws, s);
+    return e == hipSuccess ? ARMSP_SUCCESS : hip_fail(e);
+}
+
+int armsp_convert_rows_colsum_bf16(int M, int N, const float* x, int64_t ldx, uint16_t* y, int64_t ldy,
+                                   float* colsum, void* stream) {
+    using namespace armsp;
+    if (M < 0 || N < 0 || N % 8 || N > 2048 || ldx < N || ldx % 4 || ldy < N || ldy % 8) return ARMSP_ERROR_INVALID_VALUE;
+    if (N == 0) return ARMSP_SUCCESS;
+    if (!colsum || (M > 0 && (!x || !y || !aligned16(x) || !aligned16(y)))) return ARMSP_ERROR_INVALID_VALUE;
+    hipStream_t s = as_stream(stream);
+    if (M == 0) {
+        hipLaunchKernelGGL(k_zero, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, N, colsum);
+        ARMSP_LAUNCHED();
+        return ARMSP_SUCCESS;
+    }
+    int R = (int)(((int64_t)M + 2047) / 2048);
+    if (R < 32) R = 32;
+    const int nb = (int)(((int64_t)M + R - 1) / R);
+    const int P = 256 / (N / 8);
+    void* ws = nullptr;
+    const int st = ws_alloc(&ws, (size_t)nb * N * sizeof(float), s);
+    if (st) return st;
+    float* part = static_cast<float*>(ws);
+    hipLaunchKernelGGL(k_rows_colsum, dim3((unsigned)nb), dim3(256), (size_t)P * N * sizeof(float), s, M, N, R, x, ldx, y,
+                       ldy, part);
+    hipLaunchKernelGGL(k_parts_sum, dim3((unsigned)((N + 15) / 16)), dim3(256), 0, s, nb, N, part, colsum);
+    const hipError_t e = hipGetLastError();
+    ws_free(ws, s);
     return e == hipSuccess ? ARMSP_SUCCESS : hip_fail(e);
 }
 

@@ -89,6 +89,21 @@ __device__ __forceinline__ void store_c(float* __restrict__ p, const float (&o)[
     }
 }
 
+// bf16 rows of C: each value rounded to nearest even
+template <int V>
+__device__ __forceinline__ void store_c(uint16_t* __restrict__ p, const float (&o)[V]) {
+    if constexpr (V == 1) {
+        p[0] = f32_to_bf16_rne(o[0]);
+    } else {
+        uint32_t w[V / 2];
+#pragma unroll
+        for (int i = 0; i < V / 2; ++i)
+            w[i] = (uint32_t)f32_to_bf16_rne(o[2 * i]) | (uint32_t)f32_to_bf16_rne(o[2 * i + 1]) << 16;
+#pragma unroll
+        for (int i = 0; i < V / 2; ++i) __builtin_nontemporal_store(w[i], reinterpret_cast<uint32_t*>(p) + i);
+    }
+}
+
 // Optional operand scales and output epilogue (armsp_epilogue + the fp8
 // per-row scale of B).  coefficient of nonzero (r, c): val · bscale[c] ·
 // cscale[c]; output row r: rscale[r] · (A·B)[r] + bias, then ReLU.
@@ -144,8 +159,8 @@ __host__ __device__ inline size_t merge_wave_lds(int chunk, bool row_scales) {
 // were the loaded value merged with a default after the branch, the wait for
 // it would run on every row and, the memory counter being in order, drain the
 // B gathers already in flight for the next rows.
-template <int V>
-__device__ __forceinline__ void write_row(float* cp, const float (&acc)[V], const Epi& ep, float rs,
+template <int V, typename TC>
+__device__ __forceinline__ void write_row(TC* cp, const float (&acc)[V], const Epi& ep, float rs,
                                           const float (&bc)[V], bool acc_mode, bool final) {
     float o[V];
 #pragma unroll
@@ -159,7 +174,13 @@ __device__ __forceinline__ void write_row(float* cp, const float (&acc)[V], cons
         for (int v = 0; v < V; ++v) o[v] += bc[v];
     }
     const bool relu = final && ep.relu;
-    if (acc_mode) {
+    if constexpr (sizeof(TC) == 2) {  // never accumulates
+        if (relu) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) o[v] = fmaxf(o[v], 0.0f);
+        }
+        store_c<V>(cp, o);
+    } else if (acc_mode) {
         float cold[V];
         load_c<V>(cp, cold);
 #pragma unroll
@@ -435,13 +456,13 @@ __device__ __forceinline__ void gather_b(__amdgpu_buffer_rsrc_t rs, uint32_t vof
     }
 }
 
-template <typename TB, int V, int U>
+template <typename TB, typename TC, int V, int U>
 __global__ __launch_bounds__(256) void k_spmm_stream(int M, int N, int nnz, int chunk,
                                                      const int* __restrict__ rowptr, const int* __restrict__ colind,
                                                      const float* __restrict__ val, const TB* __restrict__ B,
-                                                     int ldb, Epi ep, float* __restrict__ C, int ldc, int flags,
+                                                     int ldb, Epi ep, TC* __restrict__ C, int ldc, int flags,
                                                      const int* __restrict__ part, int* __restrict__ carry_row,
-                                                     float* __restrict__ carry_val) {
+                                                     float* __restrict__ carry_val, float* __restrict__ head_val) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
@@ -496,9 +517,14 @@ __global__ __launch_bounds__(256) void k_spmm_stream(int M, int N, int nnz, int 
     load_bias<V>(bc, ep, col, active);
     auto emit = [&]() {
         const int r = i0 + rr;
-        if (active)
-            write_row<V>(C + (size_t)r * ldc + col, acc, ep, has_rs ? s_rs[rr] : 1.0f, bc, acc_mode,
-                         r != carry_in_row);
+        if (active) {
+            const float rs1 = has_rs ? s_rs[rr] : 1.0f;
+            // (bf16 rows: the part of a row begun in an earlier wave stays fp32 until its carries join it)
+            if (sizeof(TC) == 2 && r == carry_in_row)
+                write_row<V>(head_val + (size_t)wave * N + col, acc, ep, rs1, bc, false, false);
+            else
+                write_row<V>(C + (size_t)r * ldc + col, acc, ep, rs1, bc, acc_mode, r != carry_in_row);
+        }
 #pragma unroll
         for (int v = 0; v < V; ++v) acc[v] = 0.0f;
         ++rr;
@@ -579,13 +605,13 @@ __global__ __launch_bounds__(256) void k_spmm_stream(int M, int N, int nnz, int 
 // slice (when the slice count divides 8): each XCD's L2 then holds one line
 // per B row instead of all of them, i.e. several times more distinct rows of
 // the hot set.  The numbering only affects speed, never results.
-template <typename TB, int V, int U>
+template <typename TB, typename TC, int V, int U>
 __global__ __launch_bounds__(256) void k_spmm_slice(int M, int N, int nnz, int chunk, int S, int G,
                                                     const int* __restrict__ rowptr, const int* __restrict__ colind,
                                                     const float* __restrict__ val, const TB* __restrict__ B, int ldb,
-                                                    Epi ep, float* __restrict__ C, int ldc, int flags,
+                                                    Epi ep, TC* __restrict__ C, int ldc, int flags,
                                                     const int* __restrict__ part, int* __restrict__ carry_row,
-                                                    float* __restrict__ carry_val) {
+                                                    float* __restrict__ carry_val, float* __restrict__ head_val) {
     // V columns per lane (4, 8 or 16 bytes); a slice is the 32·V columns of a half wave
     constexpr int SW = 32 * V;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -653,9 +679,13 @@ __global__ __launch_bounds__(256) void k_spmm_slice(int M, int N, int nnz, int c
         float sum[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) sum[v] = half_sum(acc[v]);
-        if (h == 0 && active)
-            write_row<V>(C + (size_t)r * ldc + col, sum, ep, has_rs ? s_rs[rr] : 1.0f, bc, acc_mode,
-                         r != carry_in_row);
+        if (h == 0 && active) {
+            const float rs1 = has_rs ? s_rs[rr] : 1.0f;
+            if (sizeof(TC) == 2 && r == carry_in_row)  // as in k_spmm_stream
+                write_row<V>(head_val + (size_t)wave * N + col, sum, ep, rs1, bc, false, false);
+            else
+                write_row<V>(C + (size_t)r * ldc + col, sum, ep, rs1, bc, acc_mode, r != carry_in_row);
+        }
 #pragma unroll
         for (int v = 0; v < V; ++v) acc[v] = 0.0f;
         ++rr;
@@ -958,9 +988,11 @@ inline size_t stream_lds_bytes(int chunk, bool row_scales) { return 4 * merge_wa
 // a butterfly over the sub-rows joins them in a fixed order — a hub row cut
 // into hundreds of chunks costs a few load round trips, and the sum does not
 // depend on timing.
-template <int V>
+// bf16 rows of C take the row's last part from head_val, which its wave left in fp32.
+template <typename TC, int V>
 __global__ __launch_bounds__(256) void k_carry_fixup(int nwaves, int N, const int* __restrict__ carry_row,
-                                                     const float* __restrict__ carry_val, float* __restrict__ C,
+                                                     const float* __restrict__ carry_val,
+                                                     const float* __restrict__ head_val, TC* __restrict__ C,
                                                      int ldc, Epi ep) {
     constexpr int UF = 8;
     const int lane = threadIdx.x & 63;
@@ -990,9 +1022,14 @@ __global__ __launch_bounds__(256) void k_carry_fixup(int nwaves, int N, const in
     for (int col0 = 0; col0 < N; col0 += lpr * V) {
         const int col = col0 + cl * V;
         const bool cok = col < N;
-        float* cp = C + (size_t)r * ldc + col;
-        float o[V];  // C's row, loaded together with the first carries
-        if (p == 0 && cok) load_c<V>(cp, o);
+        TC* cp = C + (size_t)r * ldc + col;
+        float o[V];  // C's row (or its last part), loaded together with the first carries
+        if constexpr (sizeof(TC) == 2) {
+            const int we = min(w + run, nwaves - 1);
+            if (p == 0 && cok) load_c<V>(head_val + (size_t)we * N + col, o);
+        } else {
+            if (p == 0 && cok) load_c<V>(cp, o);
+        }
         float s[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) s[v] = 0.0f;
@@ -1025,8 +1062,12 @@ __global__ __launch_bounds__(256) void k_carry_fixup(int nwaves, int N, const in
 #pragma unroll
                 for (int v = 0; v < V; ++v) o[v] = fmaxf(o[v], 0.0f);
             }
+            if constexpr (sizeof(TC) == 2) {
+                store_c<V>(cp, o);
+            } else {
 #pragma unroll
-            for (int v = 0; v < V; ++v) cp[v] = o[v];
+                for (int v = 0; v < V; ++v) cp[v] = o[v];
+            }
         }
     }
 }
@@ -1040,13 +1081,13 @@ constexpr int max_vec() {
 inline bool aligned(const void* p, int bytes) { return ((uintptr_t)p % (uintptr_t)bytes) == 0; }
 
 template <typename TB>
-int pick_vec(int N, int ldb, int ldc, const TB* B, const float* C, int want, int lanes) {
+int pick_vec(int N, int ldb, int ldc, const TB* B, const void* C, int want, int lanes, int csize = 4) {
     int v = want;
     if (v <= 0) {
         v = 1;
         while (v < max_vec<TB>() && lanes * v < N) v <<= 1;
     }
-    while (v > 1 && (N % v || ldb % v || ldc % v || !aligned(B, v * (int)sizeof(TB)) || !aligned(C, v * 4))) v >>= 1;
+    while (v > 1 && (N % v || ldb % v || ldc % v || !aligned(B, v * (int)sizeof(TB)) || !aligned(C, v * csize))) v >>= 1;
     return v;
 }
 
@@ -1089,16 +1130,16 @@ int launch_split_vu(int U, dim3 grid, hipStream_t s, int M, int N, int nnz, int 
     return ARMSP_SUCCESS;
 }
 
-template <typename TB, int V>
+template <typename TB, typename TC, int V>
 int launch_stream_vu(int U, dim3 grid, hipStream_t s, int M, int N, int nnz, int chunk, const int* rp, const int* ci,
-                     const float* va, const TB* B, int ldb, const Epi& bs, float* C, int ldc, int flags,
-                     const int* part, int* crow, float* cval) {
+                     const float* va, const TB* B, int ldb, const Epi& bs, TC* C, int ldc, int flags,
+                     const int* part, int* crow, float* cval, float* hval) {
     const size_t lds = stream_lds_bytes(chunk, bs.rscale != nullptr);
     switch (U) {
 #define ARMSP_STREAM_CASE(UU)                                                                                  \
     case UU:                                                                                                   \
-        hipLaunchKernelGGL((k_spmm_stream<TB, V, UU>), grid, dim3(256), lds, s, M, N, nnz, chunk, rp, ci, va, B, ldb, \
-                           bs, C, ldc, flags, part, crow, cval);                                               \
+        hipLaunchKernelGGL((k_spmm_stream<TB, TC, V, UU>), grid, dim3(256), lds, s, M, N, nnz, chunk, rp, ci, va, B, ldb, \
+                           bs, C, ldc, flags, part, crow, cval, hval);                                               \
         break;
         ARMSP_STREAM_CASE(4)
         ARMSP_STREAM_CASE(8)
@@ -1109,10 +1150,10 @@ int launch_stream_vu(int U, dim3 grid, hipStream_t s, int M, int N, int nnz, int
     return ARMSP_SUCCESS;
 }
 
-template <typename TB, int V>
+template <typename TB, typename TC, int V>
 int launch_slice_v(int U, int S, int G, hipStream_t s, int M, int N, int nnz, int chunk, const int* rp,
-                   const int* ci, const float* va, const TB* B, int ldb, const Epi& bs, float* C, int ldc, int flags,
-                   const int* part, int* crow, float* cval) {
+                   const int* ci, const float* va, const TB* B, int ldb, const Epi& bs, TC* C, int ldc, int flags,
+                   const int* part, int* crow, float* cval, float* hval) {
     const size_t lds = stream_lds_bytes(chunk, bs.rscale != nullptr);
     const int64_t nblk = (8 % S == 0) ? ((int64_t)(G + 8 / S - 1) / (8 / S)) * 8 : (int64_t)G * S;
     if (nblk > INT_MAX) return ARMSP_ERROR_NOT_SUPPORTED;
@@ -1120,8 +1161,8 @@ int launch_slice_v(int U, int S, int G, hipStream_t s, int M, int N, int nnz, in
     switch (U) {
 #define ARMSP_SLICE_CASE(UU)                                                                                     \
     case UU:                                                                                                     \
-        hipLaunchKernelGGL((k_spmm_slice<TB, V, UU>), grid, dim3(256), lds, s, M, N, nnz, chunk, S, G, rp, ci, va, B, \
-                           ldb, bs, C, ldc, flags, part, crow, cval);                                            \
+        hipLaunchKernelGGL((k_spmm_slice<TB, TC, V, UU>), grid, dim3(256), lds, s, M, N, nnz, chunk, S, G, rp, ci, va, B, \
+                           ldb, bs, C, ldc, flags, part, crow, cval, hval);                                            \
         break;
         ARMSP_SLICE_CASE(4)
         ARMSP_SLICE_CASE(8)
@@ -1133,20 +1174,20 @@ int launch_slice_v(int U, int S, int G, hipStream_t s, int M, int N, int nnz, in
 }
 
 // lane width sv columns: 4, 8 or 16 bytes per lane
-template <typename TB>
+template <typename TB, typename TC>
 int launch_slice(int sv, int U, int S, int G, hipStream_t s, int M, int N, int nnz, int chunk, const int* rp,
-                 const int* ci, const float* va, const TB* B, int ldb, const Epi& bs, float* C, int ldc, int flags,
-                 const int* part, int* crow, float* cval) {
+                 const int* ci, const float* va, const TB* B, int ldb, const Epi& bs, TC* C, int ldc, int flags,
+                 const int* part, int* crow, float* cval, float* hval) {
     switch (sv * (int)sizeof(TB)) {
         case 4:
-            return launch_slice_v<TB, 4 / sizeof(TB)>(U, S, G, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc,
-                                                      flags, part, crow, cval);
+            return launch_slice_v<TB, TC, 4 / sizeof(TB)>(U, S, G, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc,
+                                                      flags, part, crow, cval, hval);
         case 8:
-            return launch_slice_v<TB, 8 / sizeof(TB)>(U, S, G, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc,
-                                                      flags, part, crow, cval);
+            return launch_slice_v<TB, TC, 8 / sizeof(TB)>(U, S, G, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc,
+                                                      flags, part, crow, cval, hval);
         case 16:
-            return launch_slice_v<TB, 16 / sizeof(TB)>(U, S, G, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc,
-                                                       flags, part, crow, cval);
+            return launch_slice_v<TB, TC, 16 / sizeof(TB)>(U, S, G, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc,
+                                                       flags, part, crow, cval, hval);
         default: return ARMSP_ERROR_INVALID_VALUE;
     }
 }
@@ -1188,8 +1229,8 @@ int launch_split(bool wide, int U, dim3 grid, hipStream_t s, int M, int N, int n
     if (wide || !MERGE || chunk > 2048)  // the LDS staging holds at most 2048 items per wave
         return launch_split_vu<TB, V, MERGE>(U, grid, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc, flags, crow,
                                              cval);
-    return launch_stream_vu<TB, V>(U, grid, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc, flags, part, crow,
-                                   cval);
+    return launch_stream_vu<TB, float, V>(U, grid, s, M, N, nnz, chunk, rp, ci, va, B, ldb, bs, C, ldc, flags, part,
+                                          crow, cval, nullptr);
 }
 
 // Device memory a call may use instead of allocating its workspace (the entry
@@ -1199,9 +1240,9 @@ struct Scratch {
     size_t bytes;
 };
 
-template <typename TB>
+template <typename TB, typename TC = float>
 int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind, const float* val, const TB* B,
-              const float* b_row_scale, int ldb, float* C, int ldc, int flags, const armsp_epilogue* epi,
+              const float* b_row_scale, int ldb, TC* C, int ldc, int flags, const armsp_epilogue* epi,
               const armsp_config* cfg, void* stream, const Scratch* scratch = nullptr) {
     if (M < 0 || K < 0 || N < 0 || nnz < 0) return ARMSP_ERROR_INVALID_VALUE;
     if (M == 0 || N == 0) return ARMSP_SUCCESS;
@@ -1232,7 +1273,12 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     if (flags & ARMSP_TRUNC4) sched = ARMSP_SCHED_ROW;  // truncation is per row
     if (nnz == 0) sched = ARMSP_SCHED_ROW;               // writes (or keeps) every row
 
-    if (sched == ARMSP_SCHED_ROW) {
+    constexpr bool out16 = sizeof(TC) == 2;  // bf16 rows of C: the slice and stream kernels only
+    if constexpr (out16) {
+        if (sched != ARMSP_SCHED_MERGE || flags || N <= 4 || c.group == 1 || c.chunk > 2048 ||
+            ((uint64_t)K * (uint64_t)ldb * sizeof(TB)) > 0xffffffffull)
+            return ARMSP_ERROR_NOT_SUPPORTED;
+    } else if (sched == ARMSP_SCHED_ROW) {
         int G = c.group;
         int V = pick_vec<TB>(N, ldb, ldc, B, C, c.vec, G > 0 ? G : 64);
         if (G <= 0) {
@@ -1264,7 +1310,7 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     if (sched != ARMSP_SCHED_NNZ && sched != ARMSP_SCHED_MERGE) return ARMSP_ERROR_INVALID_VALUE;
 
     const bool merge = sched == ARMSP_SCHED_MERGE;
-    const int V = pick_vec<TB>(N, ldb, ldc, B, C, c.vec, 64);
+    const int V = pick_vec<TB>(N, ldb, ldc, B, C, c.vec, 64, (int)sizeof(TC));
     int U = c.unroll > 0 ? c.unroll : (V <= 2 ? 8 : 4);
     if (U != 4 && U != 8 && U != 16) return ARMSP_ERROR_INVALID_VALUE;
     int chunk = c.chunk > 0 ? c.chunk : 512;
@@ -1313,13 +1359,14 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     void* ws = nullptr;
     const size_t row_bytes = ((size_t)nwaves * sizeof(int) + 255) & ~(size_t)255;
     const size_t val_bytes = ((size_t)nwaves * N * sizeof(float) + 255) & ~(size_t)255;
+    const size_t head_bytes = out16 ? val_bytes : 0;  // the last parts of cut rows, fp32
     const size_t part_bytes = staged ? (size_t)(nwaves + 1) * sizeof(int) : 0;
     int st;
     if (scratch) {  // no allocation: the caller's region, or a clear refusal
-        if (row_bytes + val_bytes + part_bytes > scratch->bytes) return ARMSP_ERROR_NOT_SUPPORTED;
+        if (row_bytes + val_bytes + head_bytes + part_bytes > scratch->bytes) return ARMSP_ERROR_NOT_SUPPORTED;
         ws = scratch->p;
     } else {
-        st = ws_alloc(&ws, row_bytes + val_bytes + part_bytes, s);
+        st = ws_alloc(&ws, row_bytes + val_bytes + head_bytes + part_bytes, s);
         if (st) return st;
     }
     // a caller's region is never freed here
@@ -1328,7 +1375,8 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     };
     int* crow = static_cast<int*>(ws);
     float* cval = reinterpret_cast<float*>(static_cast<char*>(ws) + row_bytes);
-    int* part = staged ? reinterpret_cast<int*>(static_cast<char*>(ws) + row_bytes + val_bytes) : nullptr;
+    float* hval = out16 ? reinterpret_cast<float*>(static_cast<char*>(ws) + row_bytes + val_bytes) : nullptr;
+    int* part = staged ? reinterpret_cast<int*>(static_cast<char*>(ws) + row_bytes + val_bytes + head_bytes) : nullptr;
     if (staged) {
         TimedLaunch t("merge_partition", s);
         st = merge_partition(M, nnz, chunk, nwaves, rowptr, part, s);
@@ -1351,20 +1399,20 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     const int asv = alb / esz;
     const bool auto_slice = merge && !wide && !narrow && c.group == 0 && chunk <= 2048 && slice_rows &&
                             N % asv == 0 && ldb % asv == 0 && ldc % asv == 0 && aligned(B, alb) &&
-                            aligned(C, 4 * asv);
+                            aligned(C, (int)sizeof(TC) * asv);
     const int SV = auto_slice ? asv : (c.vec > 0 ? c.vec : 4 / esz);
     const int slb = SV * esz;
     const bool slice = auto_slice ||
                        (merge && !wide && c.group == 32 && chunk <= 2048 && (slb == 4 || slb == 8 || slb == 16) &&
-                        N % SV == 0 && ldb % SV == 0 && ldc % SV == 0 && aligned(B, slb) && aligned(C, 4 * SV));
+                        N % SV == 0 && ldb % SV == 0 && ldc % SV == 0 && aligned(B, slb) && aligned(C, (int)sizeof(TC) * SV));
     if (c.group == 32 && !slice) {
         release(ws, s);
         return ARMSP_ERROR_NOT_SUPPORTED;
     }
     dim3 grid((unsigned)((nwaves + 3) / 4), tiles);
-    if (narrow) {
+    if (narrow && !out16) {
         TimedLaunch t("spmm", s);
-        st = launch_narrow<TB>(chunk / 64, nwaves, s, M, N, nnz, rowptr, colind, val, B, ldb, bscale, C, ldc, flags,
+        if constexpr (!out16) st = launch_narrow<TB>(chunk / 64, nwaves, s, M, N, nnz, rowptr, colind, val, B, ldb, bscale, C, ldc, flags,
                                part, crow, cval);
         hipError_t e = st ? hipSuccess : hipGetLastError();
         if (st || e != hipSuccess) {
@@ -1375,8 +1423,8 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     } else if (slice) {
         TimedLaunch t("spmm", s);
         const int S = (N + 32 * SV - 1) / (32 * SV);
-        st = launch_slice<TB>(SV, U, S, (int)((nwaves + 3) / 4), s, M, N, nnz, chunk, rowptr, colind, val, B, ldb,
-                              bscale, C, ldc, flags, part, crow, cval);
+        st = launch_slice<TB, TC>(SV, U, S, (int)((nwaves + 3) / 4), s, M, N, nnz, chunk, rowptr, colind, val, B, ldb,
+                              bscale, C, ldc, flags, part, crow, cval, hval);
         hipError_t e = st ? hipSuccess : hipGetLastError();
         if (st || e != hipSuccess) {
             release(ws, s);
@@ -1385,6 +1433,21 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
         t.stop();
     } else {
         TimedLaunch t("spmm", s);
+        if constexpr (out16) {
+#define ARMSP_STREAM_V(VV)                                                                                        \
+    case VV:                                                                                                      \
+        st = launch_stream_vu<TB, TC, VV>(U, grid, s, M, N, nnz, chunk, rowptr, colind, val, B, ldb, bscale, C, ldc, \
+                                          flags, part, crow, cval, hval);                                         \
+        break;
+            switch (V) {
+                ARMSP_STREAM_V(1)
+                ARMSP_STREAM_V(2)
+                ARMSP_STREAM_V(4)
+                ARMSP_STREAM_V(8)
+                default: st = ARMSP_ERROR_INVALID_VALUE;
+            }
+#undef ARMSP_STREAM_V
+        } else {
 #define ARMSP_SPLIT_V(VV)                                                                                          \
     case VV:                                                                                                       \
         st = merge ? launch_split<TB, VV, true>(wide, U, grid, s, M, N, nnz, chunk, rowptr, colind, val, B, ldb,    \
@@ -1408,6 +1471,7 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
             default: st = ARMSP_ERROR_INVALID_VALUE;
         }
 #undef ARMSP_SPLIT_V
+        }
         if (st) {
             release(ws, s);
             return st;
@@ -1421,12 +1485,14 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     }
     {
         TimedLaunch t("spmm_fixup", s);
-        const int fv = (N % 4 == 0 && ldc % 4 == 0 && aligned(C, 16)) ? 4 : 1;
+        const int fv = (N % 4 == 0 && ldc % 4 == 0 && aligned(C, 4 * (int)sizeof(TC))) ? 4 : 1;
         dim3 fgrid((unsigned)((nwaves + 3) / 4), 1);
         if (fv == 4)
-            hipLaunchKernelGGL((k_carry_fixup<4>), fgrid, dim3(256), 0, s, (int)nwaves, N, crow, cval, C, ldc, bscale);
+            hipLaunchKernelGGL((k_carry_fixup<TC, 4>), fgrid, dim3(256), 0, s, (int)nwaves, N, crow, cval, hval, C, ldc,
+                               bscale);
         else
-            hipLaunchKernelGGL((k_carry_fixup<1>), fgrid, dim3(256), 0, s, (int)nwaves, N, crow, cval, C, ldc, bscale);
+            hipLaunchKernelGGL((k_carry_fixup<TC, 1>), fgrid, dim3(256), 0, s, (int)nwaves, N, crow, cval, hval, C, ldc,
+                               bscale);
         hipError_t e = hipGetLastError();
         release(ws, s);
         if (e != hipSuccess) return hip_fail(e);
@@ -1498,6 +1564,13 @@ int armsp_spmm_fp8(int M, int K, int N, int nnz, const int* rowptr, const int* c
                    const armsp_config* cfg, void* stream) {
     return armsp::spmm_impl<uint8_t>(M, K, N, nnz, rowptr, colind, val, Bq, b_row_scale, ldb, C, ldc, flags, nullptr,
                                      cfg, stream);
+}
+
+int armsp_spmm_bf16_out(int M, int K, int N, int nnz, const int* rowptr, const int* colind, const float* val,
+                        const uint16_t* B, int ldb, uint16_t* C, int ldc, const armsp_epilogue* epilogue,
+                        void* stream) {
+    return armsp::spmm_impl<uint16_t, uint16_t>(M, K, N, nnz, rowptr, colind, val, B, nullptr, ldb, C, ldc, 0, epilogue,
+                                                nullptr, stream);
 }
 
 int armsp_spmm_ex(int M, int K, int N, int nnz, const int* rowptr, const int* colind, const float* val, int b_dtype,

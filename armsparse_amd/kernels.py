@@ -164,6 +164,31 @@ def spmm(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tens
     return c
 
 
+def spmm_to_bf16(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tensor], dense: torch.Tensor, *,
+                 row_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """spmm(rowptr, colind, values, dense, row_scale=row_scale).to(torch.bfloat16): the
+    same values, written as bfloat16 by the product itself where the dense operand is
+    bfloat16 on the device (armsp_spmm_bf16_out)."""
+    fn = "spmm"
+    if _selector is None and dense.is_cuda and dense.dtype == torch.bfloat16 and dense.dim() == 2:
+        _check_csr(fn, rowptr, colind, values)
+        _require(dense.stride(1) == 1, f"{fn}: dense rows must be contiguous")
+        m, (k, n), dev = rowptr.numel() - 1, dense.shape, dense.device
+        rp, ci, va = _on_device(rowptr, dev), _on_device(colind, dev), _on_device(values, dev)
+        ep = None
+        if row_scale is not None:
+            _require(row_scale.dtype == torch.float32 and row_scale.numel() == m, f"{fn}: row_scale must be float32[{m}]")
+            row_scale = _on_device(row_scale.contiguous(), dev)
+            ep = ctypes.byref(_lib.Epilogue(None, row_scale.data_ptr(), None, 0))
+        c = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+        st = _lib.lib.armsp_spmm_bf16_out(m, k, n, colind.numel(), _ptr(rp), _ptr(ci), _ptr(va), _ptr(dense),
+                                          dense.stride(0), _ptr(c), c.stride(0), ep, _stream(dev))
+        if st != _lib.ERROR_NOT_SUPPORTED:
+            _lib.check("armsp_spmm_bf16_out", st)
+            return c
+    return spmm(rowptr, colind, values, dense, row_scale=row_scale).to(torch.bfloat16)
+
+
 # ----------------------------------------------------------------- SpMV
 def spmv(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tensor], x: torch.Tensor, *,
          out: Optional[torch.Tensor] = None, accumulate: bool = False, config: ConfigLike = None) -> torch.Tensor:
@@ -543,6 +568,21 @@ def to_bf16(x: torch.Tensor, pitched: bool = False, rows16: bool = False) -> tor
     y = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
     call("armsp_convert_f32_to_bf16", x.numel(), _ptr(x), _ptr(y), _stream(x.device))
     return y
+
+
+def to_bf16_colsum(x: torch.Tensor) -> tuple:
+    """(to_bf16(x, pitched=True), colsum(x)) of a contiguous 2-D float32 device tensor,
+    in one pass over x where its rows are whole 8-column groups."""
+    m, n = x.shape
+    if n % 8 or n > 2048 or x.data_ptr() % 16:
+        return to_bf16(x, pitched=True), colsum(x)
+    _require(x.is_cuda and x.dtype == torch.float32 and x.is_contiguous(), "to_bf16_colsum: needs a contiguous 2-D "
+             "float32 device tensor")
+    y = empty_rows(m, n, torch.bfloat16, x.device)
+    out = torch.empty(n, device=x.device)
+    call("armsp_convert_rows_colsum_bf16", m, n, _ptr(x), x.stride(0), _ptr(y), y.stride(0), _ptr(out),
+         _stream(x.device))
+    return y, out
 
 
 def row_pitch(n: int, element_size: int) -> int:

@@ -59,7 +59,10 @@ class SPMMFunction(torch.autograd.Function):
         grad_feat = grad_ew = None
         if ctx.needs_input_grad[4]:
             g = grad if feat.dtype == torch.float32 else grad.to(feat.dtype)
-            grad_feat = kernels.spmm(colptr, rowind, ew_csc, g).to(feat.dtype)
+            if feat.dtype == torch.bfloat16:
+                grad_feat = kernels.spmm_to_bf16(colptr, rowind, ew_csc, g)
+            else:
+                grad_feat = kernels.spmm(colptr, rowind, ew_csc, g).to(feat.dtype)
         if ctx.needs_input_grad[5] and ew_csr is not None:
             x = feat if feat.dtype == torch.float32 else feat.float()
             grad_ew = kernels.sddmm(rowptr, colind, grad.float(), x.contiguous())
@@ -123,16 +126,23 @@ class GCNAggregate(torch.autograd.Function):
     def backward(ctx, gy):
         colptr, rowind, coef_bwd, out_norm, hdt = ctx.graph
         g = gy.contiguous()
-        dh = dcoef = None
+        dh = dcoef = dbias = None
         if ctx.needs_input_grad[0]:
-            gb = kernels.to_bf16(g.float(), pitched=True) if hdt == torch.bfloat16 else g
+            gb = g
+            if hdt == torch.bfloat16 and ctx.needs_input_grad[9]:  # the bf16 gradient and dbias in one pass
+                gb, dbias = kernels.to_bf16_colsum(g.float())
+            elif hdt == torch.bfloat16:
+                gb = kernels.to_bf16(g.float(), pitched=True)
             if ctx.blocks is not None:
                 dh = kernels.spmm_blocks(ctx.blocks, gb, row_scale=out_norm).to(hdt)
+            elif hdt == torch.bfloat16:
+                dh = kernels.spmm_to_bf16(colptr, rowind, coef_bwd, gb, row_scale=out_norm)
             else:
                 dh = kernels.spmm(colptr, rowind, coef_bwd, gb, row_scale=out_norm).to(hdt)
         if ctx.edge_grad is not None:
             dcoef = _edge_coef_grad(g, *ctx.edge_grad)
-        dbias = kernels.colsum(gy.float()) if ctx.needs_input_grad[9] else None
+        if dbias is None and ctx.needs_input_grad[9]:
+            dbias = kernels.colsum(g.float())
         return dh, None, None, None, None, dcoef, None, None, None, dbias, None
 
 
@@ -246,7 +256,8 @@ class _AggregateBiasReluDropout(torch.autograd.Function):
                                                         pitched=ctx.needs_input_grad[0])
         dh = dcoef = None
         if ctx.needs_input_grad[0]:
-            dh = kernels.spmm(colptr, rowind, coef_bwd, gyb, row_scale=out_norm).to(hdt)
+            dh = (kernels.spmm_to_bf16 if hdt == torch.bfloat16 else kernels.spmm)(colptr, rowind, coef_bwd, gyb,
+                                                                                    row_scale=out_norm).to(hdt)
         if ctx.edge_grad is not None:
             dcoef = _edge_coef_grad(gyb, *ctx.edge_grad)
         return dh, None, None, None, None, dcoef, None, None, None, dbias, None, None

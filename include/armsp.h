@@ -185,6 +185,17 @@ int armsp_spmm_ex(int M, int K, int N, int nnz,
                   float* C, int ldc, int flags, const armsp_epilogue* epilogue,
                   const armsp_config* cfg, void* stream);
 
+/* C (bfloat16) = the same product of a bfloat16 B, each value formed in fp32 and
+ * rounded once, for callers that would convert the fp32 result (the gradient of
+ * bf16 features): no fp32 C is written and read back.  Overwrites C; the
+ * schedule is chosen automatically.  ARMSP_ERROR_NOT_SUPPORTED, before anything
+ * is launched, where the merge-path kernels do not apply: N <= 4, nnz = 0, or B
+ * of 4 GiB and more.  No reference counterpart. */
+int armsp_spmm_bf16_out(int M, int K, int N, int nnz,
+                        const int* rowptr, const int* colind, const float* val,
+                        const uint16_t* B, int ldb, uint16_t* C, int ldc,
+                        const armsp_epilogue* epilogue, void* stream);
+
 /* ------------------------------------------------------------------- SpMV */
 /* y[M] (=|+=) A·x on plain CSR.  Replaces the row split of
  * numaAware/numaAwareSpMV.cpp:102-125 (one launch, no per-node copies). */
@@ -349,6 +360,11 @@ int armsp_convert_f32_to_bf16(int64_t n, const float* x, uint16_t* y, void* stre
  * lines per row). */
 int armsp_convert_rows_f32_to_bf16(int M, int N, const float* x, int64_t ldx, uint16_t* y, int64_t ldy,
                                    void* stream);
+/* The same conversion of 16-byte-aligned rows of N (a multiple of 8, at most 2048)
+ * columns, ldx a multiple of 4 and ldy of 8, with the fp32 column sums of x on the
+ * way (deterministic): the gradient of bf16 features and of their bias in one pass. */
+int armsp_convert_rows_colsum_bf16(int M, int N, const float* x, int64_t ldx, uint16_t* y, int64_t ldy,
+                                   float* colsum, void* stream);
 /* Per-row fp8-e4m3 quantisation: scale[k] = max|B[k,:]| / 448 (1 if the row
  * is zero), Bq = RNE(B / scale) saturated to ±448. */
 int armsp_quantize_fp8_rows(int K, int N, const float* B, int ldb,
