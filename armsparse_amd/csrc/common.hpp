@@ -11,6 +11,11 @@
 namespace armsp {
 
 constexpr int kWave = 64;
+// Up to this many chunks the merge kernels find their own rows (chunk_rows): one launch
+// less where the launches bound a call (4096 rows, 167,772 nonzeros, SpMM N = 64: 16.6
+// -> 13.0 us a call, SpMV 14.9 -> 11.8), and above it the searches cost more than the
+// streaming pass (SpMV of 4M nonzeros with 8,192 chunks: 31.1 -> 32.9 us).
+constexpr int64_t kSearchWaves = 4096;
 
 // ------------------------------------------------------------------ runtime
 // Records the HIP error for armsp_last_hip_error() and maps it to a status.
@@ -187,6 +192,39 @@ __device__ __forceinline__ int partition_at(const int* __restrict__ part, int w,
     const int hi = d < M ? d : M;
     const int i = part[w];
     return i < lo ? lo : (i > hi ? hi : i);
+}
+
+// The rows [i0, i1] of the chunk of diagonals [d0, d1): boundaries `wave` and wave + 1 of
+// the partition, or, without one (part null: inputs of few chunks), found here by the
+// wave — a search over all rows for d0, then over the at most d1 - d0 rows after it.
+__device__ __forceinline__ void chunk_rows(const int* __restrict__ part, int wave, int d0, int d1,
+                                           const int* __restrict__ rowptr, int M, int nnz, int& i0, int& i1) {
+    if (part) {
+        i0 = uniform(partition_at(part, wave, d0, M, nnz));
+        i1 = uniform(partition_at(part, wave + 1, d1, M, nnz));
+        return;
+    }
+    i0 = uniform(merge_path_search_wave(d0, rowptr, M, nnz));
+    // rows i0 + 1 + l·step: how many end at or before the path to d1 reaches them (a prefix of l)
+    const int lane = __lane_id();
+    int lo = i0, hi = d1 - (d0 - i0) < M ? d1 - (d0 - i0) : M;  // no nonzero of [d0, d1): all its items are rows
+    while (lo < hi) {
+        const int span = hi - lo, step = (span + 63) >> 6, i = lo + lane * step;
+        const bool p = (lane * step < span) && rowptr[i + 1] <= d1 - i - 1;
+        const int t = __popcll(__ballot(p));
+        if (step == 1) {
+            lo += t;
+            break;
+        }
+        if (t == 0) {
+            hi = lo;
+        } else {
+            const int nlo = lo + (t - 1) * step + 1;
+            hi = lo + t * step < hi ? lo + t * step : hi;
+            lo = nlo;
+        }
+    }
+    i1 = uniform(lo);
 }
 
 // Number of rows whose end is ≤ j (rows fully before nonzero j).

@@ -208,8 +208,8 @@ __global__ __launch_bounds__(256) void k_sddmm_stream(int M, int Kd, int nnz, in
     const int d1 = (int)min(d0l + chunk, total);
     int i0 = 0, j0 = d0, j1 = d1;
     if constexpr (!COO) {
-        i0 = uniform(partition_at(part, wave, d0, M, nnz));  // merge_partition
-        const int i1 = uniform(partition_at(part, wave + 1, d1, M, nnz));
+        int i1;
+        chunk_rows(part, wave, d0, d1, rowidx, M, nnz, i0, i1);
         j0 = d0 - i0;
         j1 = d1 - i1;
     }
@@ -408,23 +408,26 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
     }
     const int ngroups = (int)((nwaves + 3) / 4);
     const dim3 grid(split ? (unsigned)(((int64_t)ngroups + 3) / 4 * 8) : (unsigned)ngroups);
-    // the staged CSR kernel starts each wave from a precomputed merge-path partition
+    // the staged CSR kernel's waves start from a precomputed merge-path partition, when many
     void* ws = nullptr;
     int* part = nullptr;
     float* out2 = nullptr;
-    if (staged && !coo) {
+    const bool presearch = staged && !coo && nwaves > kSearchWaves;
+    if (presearch || split) {
         const size_t pb = ((size_t)(nwaves + 1) * sizeof(int) + 255) & ~(size_t)255;
         int st = ws_alloc(&ws, pb + (split ? (size_t)nnz * sizeof(float) : 0), s);
         if (st) return st;
-        part = static_cast<int*>(ws);
         if (split) out2 = reinterpret_cast<float*>(static_cast<char*>(ws) + pb);
-        TimedLaunch tp("merge_partition", s);
-        st = merge_partition(M, nnz, chunk, nwaves, rowidx, part, s);
-        if (st) {
-            ws_free(ws, s);
-            return st;
+        if (presearch) {
+            part = static_cast<int*>(ws);
+            TimedLaunch tp("merge_partition", s);
+            st = merge_partition(M, nnz, chunk, nwaves, rowidx, part, s);
+            if (st) {
+                ws_free(ws, s);
+                return st;
+            }
+            tp.stop();
         }
-        tp.stop();
     }
     TimedLaunch t("sddmm", s);
 #define ARMSP_SDDMM_G(WW)                                                                                    \

@@ -472,8 +472,8 @@ __global__ __launch_bounds__(256) void k_spmm_stream(int M, int N, int nnz, int 
     if (d0l >= total) return;
     const int d0 = (int)d0l;
     const int d1 = (int)min(d0l + chunk, total);
-    const int i0 = uniform(partition_at(part, wave, d0, M, nnz));  // merge_partition
-    const int i1 = uniform(partition_at(part, wave + 1, d1, M, nnz));
+    int i0, i1;
+    chunk_rows(part, wave, d0, d1, rowptr, M, nnz, i0, i1);
     const int j0 = d0 - i0, j1 = d1 - i1;
     const int nz = j1 - j0;      // ≤ chunk
     const int nr = i1 - i0 + 1;  // rows i0..i1, ≤ chunk + 1
@@ -634,8 +634,8 @@ __global__ __launch_bounds__(256) void k_spmm_slice(int M, int N, int nnz, int c
     if (d0l >= total) return;
     const int d0 = (int)d0l;
     const int d1 = (int)min(d0l + chunk, total);
-    const int i0 = uniform(partition_at(part, wave, d0, M, nnz));  // merge_partition
-    const int i1 = uniform(partition_at(part, wave + 1, d1, M, nnz));
+    int i0, i1;
+    chunk_rows(part, wave, d0, d1, rowptr, M, nnz, i0, i1);
     const int j0 = d0 - i0, j1 = d1 - i1;
     const int nz = j1 - j0;
     const int nr = i1 - i0 + 1;
@@ -804,8 +804,8 @@ __global__ __launch_bounds__(256) void k_spmm_narrow(int M, int N, int nnz, cons
     if (d0l >= total) return;
     const int d0 = (int)d0l;
     const int d1 = (int)min(d0l + TILE, total);
-    const int i0 = uniform(partition_at(part, wave, d0, M, nnz));  // merge_partition
-    const int i1 = uniform(partition_at(part, wave + 1, d1, M, nnz));
+    int i0, i1;
+    chunk_rows(part, wave, d0, d1, rowptr, M, nnz, i0, i1);
     const int j0 = d0 - i0, j1 = d1 - i1;
     const int nz = j1 - j0, nrows = i1 - i0;  // rows i0..i1-1 end inside the tile
     const uint32_t rowbytes = (uint32_t)ldb * (uint32_t)sizeof(TB);
@@ -1354,13 +1354,14 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     if (tiles > 65535) return ARMSP_ERROR_NOT_SUPPORTED;
 
     // the LDS-staged merge kernels (stream, slice, narrow) start from a precomputed
-    // merge-path partition: nwaves + 1 row boundaries
+    // merge-path partition, nwaves + 1 row boundaries, when they have many chunks
     const bool staged = merge && !wide && chunk <= 2048;
     void* ws = nullptr;
     const size_t row_bytes = ((size_t)nwaves * sizeof(int) + 255) & ~(size_t)255;
     const size_t val_bytes = ((size_t)nwaves * N * sizeof(float) + 255) & ~(size_t)255;
     const size_t head_bytes = out16 ? val_bytes : 0;  // the last parts of cut rows, fp32
-    const size_t part_bytes = staged ? (size_t)(nwaves + 1) * sizeof(int) : 0;
+    const bool presearch = staged && nwaves > kSearchWaves;
+    const size_t part_bytes = presearch ? (size_t)(nwaves + 1) * sizeof(int) : 0;
     int st;
     if (scratch) {  // no allocation: the caller's region, or a clear refusal
         if (row_bytes + val_bytes + head_bytes + part_bytes > scratch->bytes) return ARMSP_ERROR_NOT_SUPPORTED;
@@ -1376,8 +1377,9 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     int* crow = static_cast<int*>(ws);
     float* cval = reinterpret_cast<float*>(static_cast<char*>(ws) + row_bytes);
     float* hval = out16 ? reinterpret_cast<float*>(static_cast<char*>(ws) + row_bytes + val_bytes) : nullptr;
-    int* part = staged ? reinterpret_cast<int*>(static_cast<char*>(ws) + row_bytes + val_bytes + head_bytes) : nullptr;
-    if (staged) {
+    int* part =
+        presearch ? reinterpret_cast<int*>(static_cast<char*>(ws) + row_bytes + val_bytes + head_bytes) : nullptr;
+    if (presearch) {
         TimedLaunch t("merge_partition", s);
         st = merge_partition(M, nnz, chunk, nwaves, rowptr, part, s);
         if (st) {

@@ -55,8 +55,8 @@ __global__ __launch_bounds__(256) void k_spmv_merge(int M, int nnz, const int* _
     if (d0l >= total) return;
     const int d0 = (int)d0l;
     const int d1 = (int)(d0l + TILE < total ? d0l + TILE : total);
-    const int i0 = uniform(partition_at(part, wave, d0, M, nnz));  // merge_partition
-    const int i1 = uniform(partition_at(part, wave + 1, d1, M, nnz));
+    int i0, i1;
+    chunk_rows(part, wave, d0, d1, rowptr, M, nnz, i0, i1);
     const int j0 = d0 - i0, j1 = d1 - i1;
     const int nrows = i1 - i0, nz = j1 - j0;
     int* re = s_re[wid];
@@ -703,7 +703,9 @@ int launch_merge(int M, int nnz, const int* rp, const int* ci, const float* va, 
     int* crow = static_cast<int*>(ws);
     float* cval = reinterpret_cast<float*>(static_cast<char*>(ws) + rb);
     int* part = reinterpret_cast<int*>(static_cast<char*>(ws) + 2 * rb);
-    {
+    if (nwaves <= kSearchWaves) {
+        part = nullptr;
+    } else {
         TimedLaunch t("merge_partition", s);
         st = merge_partition(M, nnz, TILE, nwaves, rp, part, s);
         if (st) {
