@@ -58,8 +58,17 @@ def _on_device(t: Optional[torch.Tensor], dev: torch.device) -> Optional[torch.T
     return t if t.device == dev else t.to(dev)
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+def _all_on_device(dev: torch.device, *tensors) -> tuple:
+    """_on_device of each (compared by device index: half the host time of a device comparison)."""
+    i = dev.index
+    for t in tensors:
+        if t is not None and t.get_device() != i:
+            return tuple(_on_device(t, dev) for t in tensors)
+    return tensors
+
+
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return t.data_ptr() if t is not None else None
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -70,11 +79,16 @@ def _stream(dev: torch.device):
     torch has it: about 5 us less host time per call than torch.cuda.current_stream)."""
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(idx))
-    return ctypes.c_void_p(torch.cuda.current_stream(idx).cuda_stream)
+        return _raw_stream(idx)
+    return torch.cuda.current_stream(idx).cuda_stream
 
 
 def _check_csr(fn: str, rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tensor]) -> None:
+    # one pass over the usual case without building the messages (0.9 -> 0.4 us of a 13 us call)
+    if rowptr.dtype is torch.int32 and colind.dtype is torch.int32 and rowptr.dim() == 1 and rowptr.numel() and \
+            rowptr.is_contiguous() and colind.is_contiguous() and (values is None or (
+                values.dtype is torch.float32 and values.is_contiguous() and values.numel() == colind.numel())):
+        return
     _require(rowptr.dtype == torch.int32, f"{fn}: rowptr must be int32")
     _require(colind.dtype == torch.int32, f"{fn}: colind must be int32")
     _require(rowptr.dim() == 1 and rowptr.numel() >= 1, f"{fn}: rowptr must be 1-D with M+1 entries")
@@ -102,25 +116,24 @@ def spmm(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tens
     """
     fn = "spmm"
     _check_csr(fn, rowptr, colind, values)
-    _require(dense.dim() == 2, f"{fn}: dense must be 2-D")
-    _require(dense.stride(1) == 1, f"{fn}: dense rows must be contiguous")
+    _require(dense.dim() == 2, "spmm: dense must be 2-D")
+    _require(dense.stride(1) == 1, "spmm: dense rows must be contiguous")
     m = rowptr.numel() - 1
     k, n = dense.shape
     nnz = colind.numel()
     host = not dense.is_cuda
     dev = _device() if host else dense.device
-    rp, ci, va = _on_device(rowptr, dev), _on_device(colind, dev), _on_device(values, dev)
-    d = _on_device(dense, dev)
+    rp, ci, va, d = _all_on_device(dev, rowptr, colind, values, dense)
     if out is None:
-        _require(not accumulate, f"{fn}: accumulate needs an output tensor")
-        c = torch.empty((m, n), dtype=torch.float32, device=dev)
+        _require(not accumulate, "spmm: accumulate needs an output tensor")
+        c = d.new_empty((m, n)) if d.dtype is torch.float32 else torch.empty((m, n), dtype=torch.float32, device=dev)
     else:
         _require(out.shape == (m, n) and out.dtype == torch.float32, f"{fn}: out must be float32 [M, N]")
         _require(out.stride(1) == 1, f"{fn}: out rows must be contiguous")
         c = _on_device(out, dev)
     flags = (_lib.ACCUMULATE if accumulate else 0) | (_lib.TRUNC4 if trunc4 else 0)
     nc = n if ncols is None else int(ncols)
-    _require(0 <= nc <= n, f"{fn}: ncols out of range")
+    _require(0 <= nc <= n, "spmm: ncols out of range")
     cfg = _config(config, "spmm", rowptr, m, nnz, nc)
     s = _stream(dev)
     if col_scale is not None or row_scale is not None or bias is not None or relu:
@@ -195,14 +208,14 @@ def spmv(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tens
     """y[M] (=, or += with accumulate) A·x on plain CSR."""
     fn = "spmv"
     _check_csr(fn, rowptr, colind, values)
-    _require(x.dim() == 1 and x.dtype == torch.float32 and x.is_contiguous(), f"{fn}: x must be contiguous float32")
+    _require(x.dim() == 1 and x.dtype is torch.float32 and x.is_contiguous(), "spmv: x must be contiguous float32")
     m, nnz = rowptr.numel() - 1, colind.numel()
     host = not x.is_cuda
     dev = _device() if host else x.device
-    rp, ci, va, xd = (_on_device(t, dev) for t in (rowptr, colind, values, x))
+    rp, ci, va, xd = _all_on_device(dev, rowptr, colind, values, x)
     if out is None:
-        _require(not accumulate, f"{fn}: accumulate needs an output tensor")
-        y = torch.empty(m, dtype=torch.float32, device=dev)
+        _require(not accumulate, "spmv: accumulate needs an output tensor")
+        y = xd.new_empty((m,))
     else:
         _require(out.shape == (m,) and out.dtype == torch.float32 and out.is_contiguous(), f"{fn}: bad out")
         y = _on_device(out, dev)
@@ -232,7 +245,7 @@ def vcsr_spmv(rowptr: torch.Tensor, colind: torch.Tensor, values: torch.Tensor, 
     _require(y.numel() == m, f"{fn}: y must have M entries")
     host = not y.is_cuda
     dev = _device() if host else y.device
-    rp, ci, va, xd, yd = (_on_device(t, dev) for t in (rowptr, colind, values, x, y))
+    rp, ci, va, xd, yd = _all_on_device(dev, rowptr, colind, values, x, y)
     call("armsp_spmv_vcsr_f32", m, nnz, _ptr(rp), _ptr(ci), _ptr(va), _ptr(xd), _ptr(yd),
          (_lib.FUSED_MLA if fused else 0) | (_lib.VCSR_BALANCED if balanced else 0), _stream(dev))
     if host:
@@ -312,11 +325,15 @@ def sddmm(rows: torch.Tensor, colind: torch.Tensor, U: torch.Tensor, V: torch.Te
           scale: Optional[torch.Tensor] = None, coo: bool = False, config: ConfigLike = None) -> torch.Tensor:
     """out[e] = scale[e]·<U[row(e)], V[colind[e]]>; rows is rowptr (CSR) or rowind (COO)."""
     fn = "sddmm"
-    _require(rows.dtype == torch.int32 and colind.dtype == torch.int32, f"{fn}: indices must be int32")
-    _require(rows.is_contiguous() and colind.is_contiguous(), f"{fn}: indices must be contiguous")
-    _require(U.dim() == 2 and V.dim() == 2 and U.shape[1] == V.shape[1], f"{fn}: U, V must be 2-D with equal width")
-    _require(U.dtype == V.dtype and U.dtype in (torch.float32, torch.bfloat16), f"{fn}: U, V must be float32 or bf16")
-    _require(U.stride(1) == 1 and V.stride(1) == 1, f"{fn}: U, V rows must be contiguous")
+    if not (rows.dtype is torch.int32 and colind.dtype is torch.int32 and rows.is_contiguous() and
+            colind.is_contiguous() and U.dim() == 2 and V.dim() == 2 and U.shape[1] == V.shape[1] and
+            U.dtype is V.dtype and U.dtype in (torch.float32, torch.bfloat16) and U.stride(1) == 1 and
+            V.stride(1) == 1):  # say which
+        _require(rows.dtype == torch.int32 and colind.dtype == torch.int32, f"{fn}: indices must be int32")
+        _require(rows.is_contiguous() and colind.is_contiguous(), f"{fn}: indices must be contiguous")
+        _require(U.dim() == 2 and V.dim() == 2 and U.shape[1] == V.shape[1], f"{fn}: U, V must be 2-D with equal width")
+        _require(U.dtype == V.dtype and U.dtype in (torch.float32, torch.bfloat16), f"{fn}: U, V must be float32 or bf16")
+        _require(U.stride(1) == 1 and V.stride(1) == 1, f"{fn}: U, V rows must be contiguous")
     nnz, kd = colind.numel(), U.shape[1]
     m = U.shape[0]
     if coo:
@@ -327,7 +344,7 @@ def sddmm(rows: torch.Tensor, colind: torch.Tensor, U: torch.Tensor, V: torch.Te
         _require(scale.dtype == torch.float32 and scale.numel() == nnz and scale.is_contiguous(), f"{fn}: bad scale")
     host = not U.is_cuda
     dev = _device() if host else U.device
-    rd, ci, ud, vd, sd = (_on_device(t, dev) for t in (rows, colind, U, V, scale))
+    rd, ci, ud, vd, sd = _all_on_device(dev, rows, colind, U, V, scale)
     out = torch.empty(nnz, dtype=torch.float32, device=dev)
     s = _stream(dev)
     if coo:
