@@ -6,15 +6,21 @@
 // tile is staged in LDS, the nonzeros of A's row are taken in CSR order and
 // each B row is scattered by the lanes (its columns are distinct, so one pass
 // has no conflicts), then the tile is written back.  A window of 64 A nonzeros
-// loads its B-row bounds at once, and each B row's entries are loaded one step
-// before they are scattered, so the walk does not wait on memory per nonzero.  Every output element
-// sees the same fmaf sequence as the reference, so the result is bit-exact.
+// loads its B-row bounds at once, and the B rows' entries are loaded kAhead steps
+// before they are scattered, so the walk does not wait on memory per nonzero.  Every
+// output element sees the same fmaf sequence as the reference, so the result is
+// bit-exact.
+// Bound: C read and written (4096² fp32: 27 us at the copy rate) and the steps, one
+// LDS round trip each.  4096² x 4096² at 1%: 62 us with one step ahead and tiles of
+// 4096 columns (two workgroups a CU), 47 with 8 ahead, 44 with tiles of 2048 (1024:
+// 48; 4, 6, 16 ahead: 44, 44, 49).
 #include "common.hpp"
 
 namespace armsp {
 namespace {
 
-constexpr int kTN = 4096;  // columns per wave tile (16 KiB of LDS per wave; 1024 and 2048 time the same)
+constexpr int kTN = 2048;  // columns per wave tile (8 KiB of LDS per wave: 20 waves a CU)
+constexpr int kAhead = 8;  // B rows whose entries are in flight
 
 __global__ __launch_bounds__(256) void k_spgemm_dense(int M, int N, int ntiles, const int* __restrict__ rpA,
                                                       const int* __restrict__ ciA, const float* __restrict__ vA,
@@ -31,14 +37,17 @@ __global__ __launch_bounds__(256) void k_spgemm_dense(int M, int N, int ntiles, 
     const int tn = min(kTN, N - c0);
     float* t = tile[wid];
     float* crow = C + (size_t)m * ldc + c0;
-    if (vec4) {  // C rows 16-byte aligned, tn a multiple of 4
-        for (int k = lane * 4; k < tn; k += 256)
-            *reinterpret_cast<float4*>(&t[k]) = *reinterpret_cast<const float4*>(&crow[k]);
-    } else {
-        for (int k = lane; k < tn; k += 64) t[k] = crow[k];
-    }
-    wave_sync_lds();
-
+    auto stage = [&]() {
+        if (vec4) {  // C rows 16-byte aligned, tn a multiple of 4
+#pragma unroll 16
+            for (int k = lane * 4; k < tn; k += 256)
+                *reinterpret_cast<float4*>(&t[k]) = *reinterpret_cast<const float4*>(&crow[k]);
+        } else {
+#pragma unroll 8
+            for (int k = lane; k < tn; k += 64) t[k] = crow[k];
+        }
+        wave_sync_lds();
+    };
     const int beg = rpA[m], end = rpA[m + 1];
     for (int wbase = beg; wbase < end; wbase += 64) {
         // this window's A nonzeros and the bounds of their B rows, one per lane,
@@ -52,41 +61,46 @@ __global__ __launch_bounds__(256) void k_spgemm_dense(int M, int N, int ntiles, 
             bl = rpB[wk];
             el = rpB[wk + 1];
         }
-        // the first 64 entries of B row q are loaded one step ahead, so a step
-        // scatters while the next step's loads are in flight
+        // the first 64 entries of B row q are loaded kAhead steps ahead of their scatter:
+        // a step is two LDS accesses, a load several times that
         auto fetch = [&](int q, int& j, float& v) {
-            const int bb = read_lane(bl, q), be = read_lane(el, q);
-            const int p = bb + lane;
             j = -1;
             v = 0.0f;
-            if (p < be && lane < 64) {
-                j = ciB[p];
-                v = vB ? vB[p] : 1.0f;
+            if (q < n) {
+                const int p = read_lane(bl, q) + lane;
+                if (p < read_lane(el, q)) {
+                    j = ciB[p];
+                    v = vB ? vB[p] : 1.0f;
+                }
             }
         };
-        int jc;
-        float vc;
-        fetch(0, jc, vc);
-        for (int q = 0; q < n; ++q) {
-            const float a = read_lane(wa, q);
-            int jn = -1;
-            float vn = 0.0f;
-            if (q + 1 < n) fetch(q + 1, jn, vn);
-            // B row q's columns are distinct, so the lanes' updates do not collide
-            {
-                const int j = jc - c0;
-                if (jc >= 0 && j >= 0 && j < tn) t[j] = fmaf(a, vc, t[j]);
+        int jc[kAhead];
+        float vc[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) fetch(u, jc[u], vc[u]);
+        if (wbase == beg) stage();  // C's tile arrives behind the first entries of B
+        for (int q0 = 0; q0 < n; q0 += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int q = q0 + u;
+                if (q >= n) break;  // uniform
+                const float a = read_lane(wa, q);
+                // B row q's columns are distinct, so the lanes' updates do not collide
+                {
+                    const int j = jc[u] - c0;
+                    if (jc[u] >= 0 && j >= 0 && j < tn) t[j] = fmaf(a, vc[u], t[j]);
+                }
+                fetch(q + kAhead, jc[u], vc[u]);
+                const int bb = read_lane(bl, q), be = read_lane(el, q);
+                for (int p = bb + 64 + lane; p < be; p += 64) {  // the rest of a B row over 64 entries
+                    const int j = ciB[p] - c0;
+                    if (j >= 0 && j < tn) t[j] = fmaf(a, vB ? vB[p] : 1.0f, t[j]);
+                }
+                wave_sync_lds();  // step q's updates land before step q+1 touches the same elements
             }
-            const int bb = read_lane(bl, q), be = read_lane(el, q);
-            for (int p = bb + 64 + lane; p < be; p += 64) {  // the rest of a B row over 64 entries
-                const int j = ciB[p] - c0;
-                if (j >= 0 && j < tn) t[j] = fmaf(a, vB ? vB[p] : 1.0f, t[j]);
-            }
-            wave_sync_lds();  // step q's updates land before step q+1 touches the same elements
-            jc = jn;
-            vc = vn;
         }
     }
+    if (beg >= end) return;  // no entries: C keeps its row
     if (vec4) {
         for (int k = lane * 4; k < tn; k += 256)
             *reinterpret_cast<float4*>(&crow[k]) = *reinterpret_cast<const float4*>(&t[k]);
