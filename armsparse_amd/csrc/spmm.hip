@@ -1352,8 +1352,12 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
         // fp32 rows of more than 64 columns and under 24 nonzeros a row on average: 256 items
         // and 4 gathers per batch, which leave more waves on a CU, where 512 are to be had
         // (R-MAT of 150,000 rows, 2M nonzeros, N = 100: 121 -> 98 us; uniform matrices the
-        // same within 1%; with one value a lane uniform matrices lose up to 6%, in bf16 20%)
-        if (chunk == 512 && c.group == 0 && esz == 4 && V >= 2 && nnz < 24 * (int64_t)M) {
+        // same within 1%; with one value a lane uniform matrices lose up to 6%, in bf16 20%).
+        // Not where their carries, 4·(N + 2) bytes a chunk, outgrow the array of the entry
+        // point that allocates nothing: it takes what it would with 512, and both entry
+        // points choose alike
+        if (chunk == 512 && c.group == 0 && esz == 4 && V >= 2 && nnz < 24 * (int64_t)M &&
+            (total + 255) / 256 * 4 * (N + 2) <= (int64_t)ARMSP_NOALLOC_SCRATCH_BYTES - 1024) {
             chunk = 256;
             if (c.unroll <= 0) U = 4;
         }
@@ -1374,7 +1378,9 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     const size_t part_bytes = presearch ? (size_t)(nwaves + 1) * sizeof(int) : 0;
     int st;
     if (scratch) {  // no allocation: the caller's region, or a clear refusal
-        if (row_bytes + val_bytes + head_bytes + part_bytes > scratch->bytes) return ARMSP_ERROR_NOT_SUPPORTED;
+        // (the boundaries count where they are not stored, too: one limit for all sizes)
+        const size_t bounds = staged ? (size_t)(nwaves + 1) * sizeof(int) : 0;
+        if (row_bytes + val_bytes + head_bytes + bounds > scratch->bytes) return ARMSP_ERROR_NOT_SUPPORTED;
         ws = scratch->p;
     } else {
         st = ws_alloc(&ws, row_bytes + val_bytes + head_bytes + part_bytes, s);
