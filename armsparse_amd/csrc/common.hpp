@@ -78,7 +78,9 @@ int device_cus();
 
 // part[w] = rows consumed by the merge path of (row ends, nonzeros) at diagonal
 // min(w·chunk, M + nnz), w = 0..nwaves (nwaves + 1 entries), on stream s.
-int merge_partition(int M, int nnz, int chunk, int64_t nwaves, const int* rowptr, int* part, hipStream_t s);
+// With `skew`, also *skew = whether a few columns take much of the matrix (nnz >= 1).
+int merge_partition(int M, int nnz, int chunk, int64_t nwaves, const int* rowptr, int* part, hipStream_t s,
+                    const int* colind = nullptr, int* skew = nullptr);
 
 // ------------------------------------------------------------ device utils
 __device__ __forceinline__ int wave_lane() { return __lane_id(); }

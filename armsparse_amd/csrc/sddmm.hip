@@ -9,6 +9,7 @@
 // lane L holding nonzero base+L, so the output store is one coalesced line
 // per wave.  The row of a CSR nonzero is found by a per-lane binary search
 // restricted to the wave's row range.
+#include <algorithm>
 #include <climits>
 
 #include "common.hpp"
@@ -173,148 +174,157 @@ __device__ __forceinline__ void gather_vec(__amdgpu_buffer_rsrc_t rs, uint32_t o
     }
 }
 
-// S = 2: the dot products are split into two column halves (Kd is the half),
-// and blocks are numbered so that the 8 XCDs (block b runs on XCD b % 8)
-// alternate halves: each XCD's L2 then caches half of every hot V row.  Half 0
-// goes to out, half 1 to out2; k_sddmm_combine adds them and scales.
+// S = 2: the dot products are split into two column halves, and blocks are
+// numbered so that the 8 XCDs (block b runs on XCD b % 8) alternate halves: each
+// XCD's L2 then caches half of every hot V row.  Half 0 goes to out, half 1 to
+// out2; k_sddmm_combine adds them and scales.  With `skew` the device decides:
+// split where *skew says so (merge_partition).
 template <typename T, int G, int W, bool COO, bool FULL>
 __global__ __launch_bounds__(256) void k_sddmm_stream(int M, int Kd, int nnz, int chunk,
                                                       const int* __restrict__ rowidx, const int* __restrict__ colind,
                                                       const float* __restrict__ scale, const T* __restrict__ U,
                                                       int ldu, const T* __restrict__ V, int ldv,
                                                       const int* __restrict__ part, float* __restrict__ out, int S,
-                                                      int ngroups, float* __restrict__ out2) {
+                                                      int ngroups, float* __restrict__ out2,
+                                                      const int* __restrict__ skew) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
     const int g = lane / G, l = lane & (G - 1);
-    int grp = (int)blockIdx.x;
-    if (S == 2) {
-        const int x = (int)(blockIdx.x & 7u);
-        grp = (int)(blockIdx.x >> 3) * 4 + (x >> 1);
-        if (grp >= ngroups) return;
-        if (x & 1) {  // the upper half of every row of U and V
-            U += Kd;
-            V += Kd;
-            out = out2;
+    if (skew) S = *skew ? 2 : 1;
+    if (S == 2) Kd >>= 1;
+    // the grid is a multiple of 8, so a workgroup's tasks are of one half
+    for (int task = (int)blockIdx.x; task < S * ngroups; task += (int)gridDim.x) {
+        int grp = task;
+        if (S == 2) {
+            const int x = task & 7;
+            grp = (task >> 3) * 4 + (x >> 1);
+            scale = nullptr;
+            if ((x & 1) && out != out2) {  // the upper half of every row of U and V
+                U += Kd;
+                V += Kd;
+                out = out2;
+            }
         }
-        scale = nullptr;
-    }
-    const int wave = uniform(grp * 4 + wid);
-    const int64_t total = COO ? (int64_t)nnz : (int64_t)M + nnz;
-    const int64_t d0l = (int64_t)wave * chunk;
-    if (d0l >= total) return;
-    const int d0 = (int)d0l;
-    const int d1 = (int)min(d0l + chunk, total);
-    int i0 = 0, j0 = d0, j1 = d1;
-    if constexpr (!COO) {
-        int i1;
-        chunk_rows(part, wave, d0, d1, rowidx, M, nnz, i0, i1);
-        j0 = d0 - i0;
-        j1 = d1 - i1;
-    }
-    const int nz = j1 - j0;
-    const size_t wstride = ((size_t)chunk * 8 + (size_t)(chunk + 1) * 4 + 15) & ~(size_t)15;
-    uint2* s_off = reinterpret_cast<uint2*>(smem + wid * wstride);
-    int* s_re = reinterpret_cast<int*>(smem + wid * wstride + (size_t)chunk * 8);
-    const uint32_t urow = (uint32_t)ldu * (uint32_t)sizeof(T), vrow = (uint32_t)ldv * (uint32_t)sizeof(T);
-    int nre = 0;
-    if constexpr (!COO) {
-        nre = d1 - d0 - nz + 1;  // row ends of rows i0..i1
-        for (int k = lane; k < nre; k += 64) s_re[k] = (i0 + k < M) ? rowidx[i0 + k + 1] : INT_MAX;
+        const int wave = uniform(grp * 4 + wid);
+        const int64_t total = COO ? (int64_t)nnz : (int64_t)M + nnz;
+        const int64_t d0l = (int64_t)wave * chunk;
+        if (d0l >= total) continue;
+        const int d0 = (int)d0l;
+        const int d1 = (int)min(d0l + chunk, total);
+        int i0 = 0, j0 = d0, j1 = d1;
+        if constexpr (!COO) {
+            int i1;
+            chunk_rows(part, wave, d0, d1, rowidx, M, nnz, i0, i1);
+            j0 = d0 - i0;
+            j1 = d1 - i1;
+        }
+        const int nz = j1 - j0;
+        const size_t wstride = ((size_t)chunk * 8 + (size_t)(chunk + 1) * 4 + 15) & ~(size_t)15;
+        uint2* s_off = reinterpret_cast<uint2*>(smem + wid * wstride);
+        int* s_re = reinterpret_cast<int*>(smem + wid * wstride + (size_t)chunk * 8);
+        const uint32_t urow = (uint32_t)ldu * (uint32_t)sizeof(T), vrow = (uint32_t)ldv * (uint32_t)sizeof(T);
+        int nre = 0;
+        if constexpr (!COO) {
+            nre = d1 - d0 - nz + 1;  // row ends of rows i0..i1
+            for (int k = lane; k < nre; k += 64) s_re[k] = (i0 + k < M) ? rowidx[i0 + k + 1] : INT_MAX;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        const int nzr = (nz + 63) & ~63;
+        for (int k = lane; k < nzr; k += 64) {
+            uint2 o = make_uint2(0u, 0u);
+            if (k < nz) {
+                const int e = j0 + k;
+                int r;
+                if constexpr (COO) {
+                    r = __builtin_nontemporal_load(rowidx + e);
+                } else {  // rows i0 + (number of row ends ≤ e)
+                    int lo = 0, hi = nre - 1;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (s_re[mid] <= e)
+                            lo = mid + 1;
+                        else
+                            hi = mid;
+                    }
+                    r = i0 + lo;
+                }
+                o = make_uint2((uint32_t)r * urow, (uint32_t)__builtin_nontemporal_load(colind + e) * vrow);
+            }
+            s_off[k] = o;
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    const int nzr = (nz + 63) & ~63;
-    for (int k = lane; k < nzr; k += 64) {
-        uint2 o = make_uint2(0u, 0u);
-        if (k < nz) {
-            const int e = j0 + k;
-            int r;
-            if constexpr (COO) {
-                r = __builtin_nontemporal_load(rowidx + e);
-            } else {  // rows i0 + (number of row ends ≤ e)
-                int lo = 0, hi = nre - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (s_re[mid] <= e)
-                        lo = mid + 1;
-                    else
-                        hi = mid;
-                }
-                r = i0 + lo;
-            }
-            o = make_uint2((uint32_t)r * urow, (uint32_t)__builtin_nontemporal_load(colind + e) * vrow);
-        }
-        s_off[k] = o;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
-    const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(U), (short)0, (int)0xffffffff,
-                                                                         0x00020000);
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(V), (short)0, (int)0xffffffff,
-                                                                         0x00020000);
-    const int steps = (Kd + G * W - 1) / (G * W);  // FULL: Kd = steps·G·W; else Kd % W == 0
-    // dot products whose operands are fetched together: 16 floats of each operand per lane
-    constexpr int QB = (16 / W) < G ? (16 / W) : G;
+        const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(U), (short)0, (int)0xffffffff,
+                                                                             0x00020000);
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(V), (short)0, (int)0xffffffff,
+                                                                             0x00020000);
+        const int steps = (Kd + G * W - 1) / (G * W);  // FULL: Kd = steps·G·W; else Kd % W == 0
+        // dot products whose operands are fetched together: 16 floats of each operand per lane
+        constexpr int QB = (16 / W) < G ? (16 / W) : G;
 
-    for (int base = 0; base < nz; base += 64) {
-        float p[G];
+        for (int base = 0; base < nz; base += 64) {
+            float p[G];
 #pragma unroll
-        for (int q = 0; q < G; ++q) p[q] = 0.0f;
-        for (int t = 0; t < steps; ++t) {
-            const int k = (t * G + l) * W;
-            const bool in = FULL || k < Kd;  // lanes past Kd in the last step read column 0, use 0
-            const uint32_t lo = in ? (uint32_t)(k * (int)sizeof(T)) : 0u;
+            for (int q = 0; q < G; ++q) p[q] = 0.0f;
+            for (int t = 0; t < steps; ++t) {
+                const int k = (t * G + l) * W;
+                const bool in = FULL || k < Kd;  // lanes past Kd in the last step read column 0, use 0
+                const uint32_t lo = in ? (uint32_t)(k * (int)sizeof(T)) : 0u;
 #pragma unroll
-            for (int qb = 0; qb < G; qb += QB) {
-                float a[QB][W], b[QB][W];
+                for (int qb = 0; qb < G; qb += QB) {
+                    float a[QB][W], b[QB][W];
 #pragma unroll
-                for (int q = 0; q < QB; ++q) {
-                    const uint2 o = s_off[base + g * G + qb + q];
-                    gather_vec<T, W>(ru, o.x + lo, a[q]);
-                    gather_vec<T, W>(rv, o.y + lo, b[q]);
-                    if (!FULL && !in) {
+                    for (int q = 0; q < QB; ++q) {
+                        const uint2 o = s_off[base + g * G + qb + q];
+                        gather_vec<T, W>(ru, o.x + lo, a[q]);
+                        gather_vec<T, W>(rv, o.y + lo, b[q]);
+                        if (!FULL && !in) {
 #pragma unroll
-                        for (int i = 0; i < W; ++i) a[q][i] = 0.0f;
+                            for (int i = 0; i < W; ++i) a[q][i] = 0.0f;
+                        }
                     }
+#pragma unroll
+                    for (int q = 0; q < QB; ++q)
+#pragma unroll
+                        for (int i = 0; i < W; ++i) p[qb + q] = fmaf(a[q][i], b[q][i], p[qb + q]);
+                    // keep the next batch's loads below this point: bounded registers, more waves
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-#pragma unroll
-                for (int q = 0; q < QB; ++q)
-#pragma unroll
-                    for (int i = 0; i < W; ++i) p[qb + q] = fmaf(a[q][i], b[q][i], p[qb + q]);
-                // keep the next batch's loads below this point: bounded registers, more waves
-                __builtin_amdgcn_sched_barrier(0);
             }
-        }
 #pragma unroll
-        for (int m = G / 2; m >= 1; m >>= 1) {
-            const bool upper = (l & m) != 0;
+            for (int m = G / 2; m >= 1; m >>= 1) {
+                const bool upper = (l & m) != 0;
 #pragma unroll
-            for (int i = 0; i < m; ++i) {
-                const float send = upper ? p[i] : p[i + m];
-                const float keep = upper ? p[i + m] : p[i];
-                p[i] = keep + __shfl_xor(send, m);
+                for (int i = 0; i < m; ++i) {
+                    const float send = upper ? p[i] : p[i + m];
+                    const float keep = upper ? p[i + m] : p[i];
+                    p[i] = keep + __shfl_xor(send, m);
+                }
             }
-        }
-        const int e = base + lane;
-        if (e < nz) {
-            const int ge = j0 + e;
-            out[ge] = scale ? scale[ge] * p[0] : p[0];
+            const int e = base + lane;
+            if (e < nz) {
+                const int ge = j0 + e;
+                out[ge] = scale ? scale[ge] * p[0] : p[0];
+            }
         }
     }
 }
 
-// out[e] = scale[e] · (out[e] + out2[e]): the two column halves of the split kernel.
+// out[e] = scale[e] · (out[e] + out2[e]): the two column halves of the split kernel
+// (nothing when `skew` says that it did not split).
 __global__ __launch_bounds__(256) void k_sddmm_combine(int nnz, const float* __restrict__ scale,
-                                                       float* __restrict__ out, const float* __restrict__ out2) {
-    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (e >= nnz) return;
-    const float d = out[e] + out2[e];
-    out[e] = scale ? scale[e] * d : d;
+                                                       float* __restrict__ out, const float* __restrict__ out2,
+                                                       const int* __restrict__ skew) {
+    if (skew && !*skew) return;
+    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nnz; e += (int64_t)gridDim.x * blockDim.x) {
+        const float d = out[e] + out2[e];
+        out[e] = scale ? scale[e] * d : d;
+    }
 }
 
 inline size_t sddmm_lds_bytes(int chunk) {
@@ -324,12 +334,12 @@ inline size_t sddmm_lds_bytes(int chunk) {
 template <typename T, int G, int W>
 void launch_sddmm_stream(bool coo, dim3 grid, hipStream_t s, int M, int Kd, int nnz, int chunk, const int* ri,
                          const int* ci, const float* sc, const T* U, int ldu, const T* V, int ldv, const int* part,
-                         float* out, int S, int ngroups, float* out2) {
+                         float* out, int S, int ngroups, float* out2, const int* skew) {
     const size_t lds = sddmm_lds_bytes(chunk);
-    const bool full = Kd % (G * W) == 0;
+    const bool full = (S == 2 || skew ? Kd / 2 : Kd) % (G * W) == 0;
 #define ARMSP_SDDMM_ST(CO, FU)                                                                                 \
     hipLaunchKernelGGL((k_sddmm_stream<T, G, W, CO, FU>), grid, dim3(256), lds, s, M, Kd, nnz, chunk, ri, ci, sc, U, \
-                       ldu, V, ldv, part, out, S, ngroups, out2)
+                       ldu, V, ldv, part, out, S, ngroups, out2, skew)
     if (coo) {
         if (full) ARMSP_SDDMM_ST(true, true); else ARMSP_SDDMM_ST(true, false);
     } else {
@@ -395,33 +405,50 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
     // unroll = 2: split the dot products into column halves spread over the XCDs
     // (each XCD's L2 then holds half of every hot V row), plus one pass that adds
     // the halves — a win on skewed columns whose V rows outgrow the L2 (the 1M
-    // R-MAT at Kd = 128: 13%), a loss where columns are uniform or local, so it is
-    // the selector's choice, not AUTO's.  Where it cannot apply (COO, the unstaged
+    // R-MAT at Kd = 128: 13%), a loss where columns are uniform or local.  Where it cannot apply (COO, the unstaged
     // kernel, odd halves) the call runs unsplit.
     if (c.unroll < 0 || c.unroll > 2) return ARMSP_ERROR_INVALID_VALUE;
     const int KdS = Kd / 2;
     const bool split = c.unroll == 2 && staged && !coo && KdS > 0 && Kd % 2 == 0 && KdS % W == 0 &&
                        aligned(U + KdS, W * (int)sizeof(T)) && aligned(V + KdS, W * (int)sizeof(T));
-    if (split && c.group <= 0) {
+    // AUTO: products of rows of at least 512 bytes (halves of two lines or more) whose V
+    // outgrows the XCDs' L2s (4 MB each) decide on the device, from a sample of the columns
+    // (merge_partition): Kd = 128, fp32, 1M R-MAT of 2^24 nonzeros 1224 us unsplit, 1060
+    // split; R-MAT of 2^18 rows, 2^22 nonzeros, Kd = 256: 573 and 497.  Uniform columns stay
+    // unsplit and pay the sample and a pass that does nothing, 8 us together, so only
+    // products of 4 GB of gathers (0.6 ms) ask; the second half's results take 4 bytes a
+    // nonzero, 256 MB at most.
+    bool adapt = !split && staged && !coo && c.schedule == 0 && c.group == 0 && c.vec == 0 && c.chunk == 0 &&
+                 c.unroll == 0 && KdS > 0 && Kd % 2 == 0 && KdS % W == 0 && nnz <= (1 << 26) && nwaves > kSearchWaves &&
+                 aligned(U + KdS, W * (int)sizeof(T)) && aligned(V + KdS, W * (int)sizeof(T)) &&
+                 (int64_t)Kd * (int64_t)sizeof(T) >= 512 && (int64_t)K * ldv * (int64_t)sizeof(T) >= (64ll << 20) &&
+                 (int64_t)nnz * Kd * (int64_t)sizeof(T) >= (4ll << 30);
+    if ((split || adapt) && c.group <= 0) {
         G = 4;
         while (G < 8 && G * W < KdS) G <<= 1;
     }
-    const int ngroups = (int)((nwaves + 3) / 4);
-    const dim3 grid(split ? (unsigned)(((int64_t)ngroups + 3) / 4 * 8) : (unsigned)ngroups);
+    // workgroups of four waves; a multiple of 8, so that each keeps to one half (and XCD)
+    const int ngroups = (int)((nwaves + 31) / 32 * 8);
     // the staged CSR kernel's waves start from a precomputed merge-path partition, when many
     void* ws = nullptr;
     int* part = nullptr;
     float* out2 = nullptr;
+    int* skew = nullptr;
     const bool presearch = staged && !coo && nwaves > kSearchWaves;
-    if (presearch || split) {
+    if (presearch || split || adapt) {
         const size_t pb = ((size_t)(nwaves + 1) * sizeof(int) + 255) & ~(size_t)255;
-        int st = ws_alloc(&ws, pb + (split ? (size_t)nnz * sizeof(float) : 0), s);
+        int st = ws_alloc(&ws, pb + (split || adapt ? (size_t)nnz * sizeof(float) + 256 : 0), s);
+        if (st && adapt) {  // no room for the second half's results: unsplit
+            adapt = false;
+            st = ws_alloc(&ws, pb, s);
+        }
         if (st) return st;
-        if (split) out2 = reinterpret_cast<float*>(static_cast<char*>(ws) + pb);
+        if (split || adapt) out2 = reinterpret_cast<float*>(static_cast<char*>(ws) + pb + 256);
+        if (adapt) skew = reinterpret_cast<int*>(static_cast<char*>(ws) + pb);
         if (presearch) {
             part = static_cast<int*>(ws);
             TimedLaunch tp("merge_partition", s);
-            st = merge_partition(M, nnz, chunk, nwaves, rowidx, part, s);
+            st = merge_partition(M, nnz, chunk, nwaves, rowidx, part, s, colind, skew);
             if (st) {
                 ws_free(ws, s);
                 return st;
@@ -429,14 +456,15 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
             tp.stop();
         }
     }
+    const dim3 grid(staged ? (unsigned)ngroups : (unsigned)((nwaves + 3) / 4));
     TimedLaunch t("sddmm", s);
 #define ARMSP_SDDMM_G(WW)                                                                                    \
     if (staged) {                                                                                            \
         switch (G) {                                                                                         \
-            case 4: launch_sddmm_stream<T, 4, WW>(coo, grid, s, M, split ? KdS : Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2); break; \
-            case 8: launch_sddmm_stream<T, 8, WW>(coo, grid, s, M, split ? KdS : Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2); break; \
-            case 16: launch_sddmm_stream<T, 16, WW>(coo, grid, s, M, split ? KdS : Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2); break; \
-            default: launch_sddmm_stream<T, 32, WW>(coo, grid, s, M, split ? KdS : Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2); break; \
+            case 4: launch_sddmm_stream<T, 4, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
+            case 8: launch_sddmm_stream<T, 8, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
+            case 16: launch_sddmm_stream<T, 16, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
+            default: launch_sddmm_stream<T, 32, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
         }                                                                                                    \
     } else {                                                                                                 \
         switch (G) {                                                                                         \
@@ -452,9 +480,9 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
         ARMSP_SDDMM_G(WMAX)
     }
 #undef ARMSP_SDDMM_G
-    if (split)
-        hipLaunchKernelGGL(k_sddmm_combine, dim3((unsigned)(((int64_t)nnz + 255) / 256)), dim3(256), 0, s, nnz,
-                           scale, out, out2);
+    if (split || adapt)
+        hipLaunchKernelGGL(k_sddmm_combine, dim3((unsigned)std::min<int64_t>(((int64_t)nnz + 255) / 256, 4096)),
+                           dim3(256), 0, s, nnz, scale, out, out2, skew);
     const hipError_t e = hipGetLastError();
     if (ws) ws_free(ws, s);
     if (e != hipSuccess) return hip_fail(e);

@@ -1,5 +1,5 @@
 """Merge-path kernels around the number of chunks from which a partition is computed, the
-chunks that an automatic SpMM takes."""
+chunks that an automatic SpMM takes, and the column split of an automatic SDDMM."""
 import ctypes
 
 import numpy as np
@@ -66,3 +66,21 @@ def test_allocation_free_product_takes_longer_chunks_where_short_ones_do_not_fit
                                      None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
         outs.append(C)
     assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("kd,dtype,pad", [(128, torch.float32, 0), (136, torch.float32, 4), (256, torch.bfloat16, 0),
+                                          (272, torch.bfloat16, 8)])
+@pytest.mark.parametrize("kind", ["rmat", "uniform"])
+def test_automatic_sddmm_split(kind, kd, dtype, pad):
+    """On skewed columns the automatic call is the split one, on uniform ones the unsplit
+    one, bit for bit; with and without a scale."""
+    a = (data.rmat_csr(18, 1 << 23, seed=9) if kind == "rmat" else data.uniform_csr(1 << 18, 1 << 18, 1 << 23, seed=9))
+    rp, ci, va = dev(a.rowptr, a.colind, a.values)
+    gen = torch.Generator("cuda").manual_seed(kd)
+    U, V = (torch.randn(1 << 18, kd + pad, device="cuda", generator=gen).to(dtype)[:, :kd] for _ in range(2))
+    split = dict(schedule="merge", unroll=2 if kind == "rmat" else 1)
+    for scale in (va, None):
+        auto = kernels.sddmm(rp, ci, U, V, scale=scale)
+        assert torch.equal(auto, kernels.sddmm(rp, ci, U, V, scale=scale, config=split))
+    other = kernels.sddmm(rp, ci, U, V, config=dict(schedule="merge", unroll=1 if kind == "rmat" else 2))
+    assert not torch.equal(auto, other)
