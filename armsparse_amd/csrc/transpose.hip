@@ -91,7 +91,10 @@ __global__ __launch_bounds__(THREADS) void k_radix_hist(int n, int shift, int db
 // each a run of consecutive tiles.
 __global__ __launch_bounds__(1024) void k_radix_scan(int ntiles, int bins, int* __restrict__ hist,
                                                      int* __restrict__ totals) {
-    constexpr int KEEP = 32;  // counts a thread holds between the two sweeps
+    // counts a thread holds between the two sweeps; the rest it reads again, as many at a time
+    // (4096 tiles of 1024 digits 24 us; 26 with the rest one by one; 8 digits a workgroup: 21,
+    // but 12.8 against 8.5 on 1465 tiles)
+    constexpr int KEEP = 32;
     __shared__ int part[64][16];
     const int d = (int)(threadIdx.x & 15u), seg = (int)(threadIdx.x >> 4);
     int* h = hist + (int)blockIdx.x * 16 + d;
@@ -109,10 +112,15 @@ __global__ __launch_bounds__(1024) void k_radix_scan(int ntiles, int bins, int* 
     __syncthreads();
     if (threadIdx.x < 16) {
         int run = 0;
-        for (int q = 0; q < 64; ++q) {
-            const int x = part[q][d];
-            part[q][d] = run;
-            run += x;
+        for (int q0 = 0; q0 < 64; q0 += 16) {  // 16 reads in flight
+            int x[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) x[q] = part[q0 + q][d];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                part[q0 + q][d] = run;
+                run += x[q];
+            }
         }
         totals[blockIdx.x * 16 + d] = run;
     }
@@ -124,10 +132,15 @@ __global__ __launch_bounds__(1024) void k_radix_scan(int ntiles, int bins, int* 
             h[(int64_t)(t0 + i) * bins] = run;
             run += v[i];
         }
-    for (int t = t0 + KEEP; t < t1; ++t) {
-        const int x = h[(int64_t)t * bins];
-        h[(int64_t)t * bins] = run;
-        run += x;
+    for (int t = t0 + KEEP; t < t1; t += KEEP) {
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i) v[i] = t + i < t1 ? h[(int64_t)(t + i) * bins] : 0;
+#pragma unroll
+        for (int i = 0; i < KEEP; ++i)
+            if (t + i < t1) {
+                h[(int64_t)(t + i) * bins] = run;
+                run += v[i];
+            }
     }
 }
 

@@ -27,6 +27,7 @@ def _csr(m, k, nnz, seed):
 @pytest.mark.parametrize("m,k,nnz", [
     (1, 1, 1), (3, 2, 2047), (70, 17, 2048), (5000, 1024, 2049), (9, 1025, 4097), (4000, (1 << 20) + 1, 30_000),
     (100_000, 3, 16_385), (50, 70_000, BIG - 1), (300_000, 300_007, BIG), (1 << 20, 1 << 20, BIG + 16_385),
+    (70_000, 60_000, 20_000_000),  # more tiles than the scan holds counts of
 ])
 def test_transpose_is_a_stable_sort(m, k, nnz, values):
     rp, ci, va, rows = _csr(m, k, nnz, m + k + nnz)
