@@ -198,7 +198,8 @@ __device__ __forceinline__ int partition_at(const int* __restrict__ part, int w,
 
 // The rows [i0, i1] of the chunk of diagonals [d0, d1): boundaries `wave` and wave + 1 of
 // the partition, or, without one (part null: inputs of few chunks), found here by the
-// wave — a search over all rows for d0, then over the at most d1 - d0 rows after it.
+// wave — a search over all rows for d0, then over the at most d1 - d0 rows after it,
+// from d1 - nnz on, so that here too a malformed rowptr ends the chunk by nonzero nnz.
 __device__ __forceinline__ void chunk_rows(const int* __restrict__ part, int wave, int d0, int d1,
                                            const int* __restrict__ rowptr, int M, int nnz, int& i0, int& i1) {
     if (part) {
@@ -209,7 +210,8 @@ __device__ __forceinline__ void chunk_rows(const int* __restrict__ part, int wav
     i0 = uniform(merge_path_search_wave(d0, rowptr, M, nnz));
     // rows i0 + 1 + l·step: how many end at or before the path to d1 reaches them (a prefix of l)
     const int lane = __lane_id();
-    int lo = i0, hi = d1 - (d0 - i0) < M ? d1 - (d0 - i0) : M;  // no nonzero of [d0, d1): all its items are rows
+    int lo = i0 > d1 - nnz ? i0 : d1 - nnz;
+    int hi = d1 - (d0 - i0) < M ? d1 - (d0 - i0) : M;  // no nonzero of [d0, d1): all its items are rows
     while (lo < hi) {
         const int span = hi - lo, step = (span + 63) >> 6, i = lo + lane * step;
         const bool p = (lane * step < span) && rowptr[i + 1] <= d1 - i - 1;
