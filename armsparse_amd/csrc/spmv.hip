@@ -423,16 +423,16 @@ __device__ __forceinline__ float rotate4(float s) {  // lane i of each 16 gets l
 }
 
 template <bool FUSED>
-__device__ void vcsr_medium_rows(int gg, int ngg, const int* __restrict__ list_med, const int* __restrict__ count,
+__device__ void vcsr_medium_rows(uint32_t gg, uint32_t ngg, const int* __restrict__ list_med, const int* __restrict__ count,
                                  const int* __restrict__ rowptr, const int* __restrict__ colind,
                                  const float* __restrict__ val, const float* __restrict__ x, float* __restrict__ y) {
     constexpr int D = VCSR_MED_AHEAD;
     constexpr int IT = 4 * D;  // blocks of an iteration
     const int q = (threadIdx.x >> 2) & 3, l = threadIdx.x & 3;
-    const int nmed = __builtin_amdgcn_readfirstlane(count[2]);
+    const uint32_t nmed = (uint32_t)__builtin_amdgcn_readfirstlane(count[2]);
     // row i of the list; past its end no blocks (row 0's index, so every load stays in bounds)
-    auto row_at = [&](int i) { return i < nmed ? list_med[i] : 0; };
-    auto blocks_of = [&](int i, int r, int b) { return i < nmed ? (rowptr[r + 1] - b) >> 2 : 0; };
+    auto row_at = [&](uint32_t i) { return i < nmed ? list_med[i] : 0; };
+    auto blocks_of = [&](uint32_t i, int r, int b) { return i < nmed ? (rowptr[r + 1] - b) >> 2 : 0; };
     auto columns = [&](int beg, int nb, int pos, int (&c)[D]) {
 #pragma unroll
         for (int u = 0; u < D; ++u) {
@@ -453,7 +453,7 @@ __device__ void vcsr_medium_rows(int gg, int ngg, const int* __restrict__ list_m
         }
     };
     // the group's row, the two after it, and the index of the third
-    int i = gg;
+    uint32_t i = gg;
     int r0 = row_at(i), r1 = row_at(i + ngg), r2 = row_at(i + 2 * ngg), r3 = row_at(i + 3 * ngg);
     int b0 = rowptr[r0], b1 = rowptr[r1], b2 = rowptr[r2];
     int n0 = blocks_of(i, r0, b0), n1 = blocks_of(i + ngg, r1, b1), n2 = blocks_of(i + 2 * ngg, r2, b2);
@@ -499,7 +499,8 @@ __device__ void vcsr_medium_rows(int gg, int ngg, const int* __restrict__ list_m
         const float tot = __fadd_rn(t, __shfl_xor(t, 1, 4));  // (s0+s2)+(s1+s3)
         if (last) {
             if (i < nmed && q == 3 && l == 0) y[r0] = __fadd_rn(y0, tot);
-            i += ngg;
+            // (past the list a group waits there for the wave's others, however long their rows are)
+            i += i < nmed ? ngg : 0u;
             s = 0.0f;
             r0 = r1;
             b0 = b1;
@@ -679,8 +680,8 @@ __global__ __launch_bounds__(256) void k_spmv_vcsr_split(int M, const int* __res
         return;
     }
     if (b < n_long_wg + n_med_wg) {
-        const int gg = (b - n_long_wg) * 16 + (int)(threadIdx.x >> 4);
-        vcsr_medium_rows<FUSED>(gg, n_med_wg * 16, list_med, count, rowptr, colind, val, x, y);
+        const uint32_t gg = (uint32_t)(b - n_long_wg) * 16 + (threadIdx.x >> 4);
+        vcsr_medium_rows<FUSED>(gg, (uint32_t)n_med_wg * 16, list_med, count, rowptr, colind, val, x, y);
         return;
     }
     // the short walker takes what neither list holds: rows of at most VCSR_MED_MIN
