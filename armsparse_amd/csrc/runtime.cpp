@@ -179,7 +179,13 @@ int pool_alloc(void** p, size_t bytes, int dev, hipStream_t s) {
         }
         pool = g_pools[dev];
     }
-    ARMSP_HIP(hipMallocFromPoolAsync(p, bytes, pool, s));
+    const hipError_t e = hipMallocFromPoolAsync(p, bytes, pool, s);
+    if (e != hipSuccess) {
+        // the status tells the caller; left pending, the error would be taken for one of
+        // its next launches where it goes on without the workspace
+        (void)hipGetLastError();
+        return hip_fail(e);
+    }
     return ARMSP_SUCCESS;
 }
 }  // namespace
