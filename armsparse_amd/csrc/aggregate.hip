@@ -20,6 +20,7 @@
 // R-MAT with 2^21 nonzeros at N = 64 took 2551 us, 74 + 5 now; matrices without
 // long rows keep the group per row (1.5M nonzeros, uniform: 65 us, 64 + 4 now), and the
 // wave ranges end at once.
+#include <algorithm>
 #include <climits>
 
 #include "common.hpp"
@@ -224,15 +225,16 @@ __device__ __forceinline__ void max_short_rows(int blk, int tile, int M, int N, 
 // the columns a group of the short one covers in a quarter, a half or all of a wave.
 // (Column slices spread over the XCDs, as in the SpMM, do not pay: 78 -> 84 us on the
 // R-MAT, 68 -> 70 us on the uniform matrix.)
+// `first`: the launch's first workgroup, where they are more than one launch holds.
 template <int V, int G>
-__global__ __launch_bounds__(256) void k_spmm_max(int M, int N, int nnz, int nlong, int chunk, int nshort,
+__global__ __launch_bounds__(256) void k_spmm_max(int first, int M, int N, int nnz, int nlong, int chunk, int nshort,
                                                   int long_row, const int* __restrict__ rowptr, const int* __restrict__ colind,
                                                   const float* __restrict__ val, const float* __restrict__ B,
                                                   int ldb, float init, float* __restrict__ C, int ldc,
                                                   int* __restrict__ argmax, MaxParts parts) {
     constexpr int VL = V == 4 && G == 64 ? 4 : V == 4 && G == 32 ? 2 : 1;
     const int ltiles = nlong ? (N + 64 * VL - 1) / (64 * VL) : 0;
-    const int b = (int)blockIdx.x;
+    const int b = first + (int)blockIdx.x;
     if (b < nlong * ltiles) {
         const int wave = uniform((b / ltiles) * 4 + (int)(threadIdx.x >> 6));
         const int64_t j0 = (int64_t)wave * chunk;
@@ -380,14 +382,14 @@ __global__ __launch_bounds__(kBwdThreads) void k_spmm_max_backward(int64_t total
 }
 
 template <int V>
-int launch_max(int G, unsigned grid, hipStream_t s, int M, int N, int nnz, int nlong, int chunk, int nshort,
+int launch_max(int G, int first, unsigned grid, hipStream_t s, int M, int N, int nnz, int nlong, int chunk, int nshort,
                int long_row, const int* rp, const int* ci, const float* va, const float* B, int ldb, float init,
                float* C, int ldc, int* arg, const MaxParts& parts) {
     switch (G) {
 #define ARMSP_MAX_CASE(GG)                                                                                          \
     case GG:                                                                                                        \
-        hipLaunchKernelGGL((k_spmm_max<V, GG>), dim3(grid), dim3(256), 0, s, M, N, nnz, nlong, chunk, nshort, long_row, \
-                           rp, ci, va, B, ldb, init, C, ldc, arg, parts);                                           \
+        hipLaunchKernelGGL((k_spmm_max<V, GG>), dim3(grid), dim3(256), 0, s, first, M, N, nnz, nlong, chunk, nshort, \
+                           long_row, rp, ci, va, B, ldb, init, C, ldc, arg, parts);                                 \
         break;
         ARMSP_MAX_CASE(4)
         ARMSP_MAX_CASE(8)
@@ -437,12 +439,16 @@ extern "C" int armsp_spmm_max_f32(int M, int K, int N, int nnz, const int* rowpt
     const MaxParts parts{reinterpret_cast<int*>(w), reinterpret_cast<float*>(w + i4),
                          reinterpret_cast<uint32_t*>(w + i4 + v4)};
     if (nshort * stiles > INT_MAX) return ARMSP_ERROR_NOT_SUPPORTED;
-    const unsigned grid = (unsigned)(nlong * ltiles + nshort * stiles);
+    const int64_t blocks = nlong * ltiles + nshort * stiles;
     TimedLaunch t("spmm_max", s);
-    const int st = V == 4 ? launch_max<4>(G, grid, s, M, N, nnz, (int)nlong, chunk, (int)nshort, long_row, rowptr,
-                                          colind, val, B, ldb, init, C, ldc, argmax, parts)
-                          : launch_max<1>(G, grid, s, M, N, nnz, (int)nlong, chunk, (int)nshort, long_row, rowptr,
-                                          colind, val, B, ldb, init, C, ldc, argmax, parts);
+    int st = ARMSP_SUCCESS;
+    for (int64_t first = 0; first < blocks && !st; first += kMaxBlocks256) {
+        const unsigned grid = (unsigned)std::min(blocks - first, kMaxBlocks256);
+        st = V == 4 ? launch_max<4>(G, (int)first, grid, s, M, N, nnz, (int)nlong, chunk, (int)nshort, long_row, rowptr,
+                                    colind, val, B, ldb, init, C, ldc, argmax, parts)
+                    : launch_max<1>(G, (int)first, grid, s, M, N, nnz, (int)nlong, chunk, (int)nshort, long_row, rowptr,
+                                    colind, val, B, ldb, init, C, ldc, argmax, parts);
+    }
     if (!st && nlong)
         hipLaunchKernelGGL(k_max_join, dim3((unsigned)((nwaves + 3) / 4)), dim3(256), 0, s, (int)nwaves, N, parts, C,
                            ldc, argmax);

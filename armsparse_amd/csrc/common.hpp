@@ -11,6 +11,8 @@
 namespace armsp {
 
 constexpr int kWave = 64;
+// A launch holds fewer than 2^32 threads along x: so many workgroups of 256.
+constexpr int64_t kMaxBlocks256 = (1 << 24) - 1;
 // Up to this many chunks the merge kernels find their own rows (chunk_rows): one launch
 // less where the launches bound a call (4096 rows, 167,772 nonzeros, SpMM N = 64: 16.6
 // -> 13.0 us a call, SpMV 14.9 -> 11.8), and above it the searches cost more than the

@@ -1,5 +1,6 @@
 // Dense helpers: counter-based fills (same RNG as the host generators),
 // fp32 → bf16 conversion, per-row fp8-e4m3 quantisation.
+#include <algorithm>
 #include <cmath>
 
 #include "common.hpp"
@@ -65,20 +66,20 @@ __global__ void k_to_bf16_x8(int64_t n, const float* __restrict__ x, uint16_t* _
 
 // rows of N floats at pitch ldx → rows of N bf16 at pitch ldy, a group of G lanes per
 // row.  VEC: aligned rows of a multiple of 8 columns, 8 a lane (170,000 x 256: 85 us
-// one value a lane with a 64-bit division each, about 40 so).
+// one value a lane with a 64-bit division each, about 40 so).  A workgroup takes more
+// than one set of rows only where the launch limit is reached.
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_rows_to_bf16_2d(int64_t M, int N, int G, const float* __restrict__ x,
                                                          int64_t ldx, uint16_t* __restrict__ y, int64_t ldy) {
     constexpr int W = VEC ? 8 : 1;
     const int per = 256 / G;
-    const int64_t m = (int64_t)blockIdx.x * per + threadIdx.x / G;
-    if (m >= M) return;
-    for (int n = (int)(threadIdx.x % G) * W; n < N; n += G * W) {
-        if constexpr (VEC)
-            to_bf16_x8(x + m * ldx + n, y + m * ldy + n);
-        else
-            y[m * ldy + n] = f32_to_bf16_rne(x[m * ldx + n]);
-    }
+    for (int64_t m = (int64_t)blockIdx.x * per + threadIdx.x / G; m < M; m += (int64_t)gridDim.x * per)
+        for (int n = (int)(threadIdx.x % G) * W; n < N; n += G * W) {
+            if constexpr (VEC)
+                to_bf16_x8(x + m * ldx + n, y + m * ldy + n);
+            else
+                y[m * ldy + n] = f32_to_bf16_rne(x[m * ldx + n]);
+        }
 }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -177,7 +178,7 @@ int armsp_convert_f32_to_bf16(int64_t n, const float* x, uint16_t* y, void* stre
     if (n < 0 || (n > 0 && (!x || !y))) return ARMSP_ERROR_INVALID_VALUE;
     if (n == 0) return ARMSP_SUCCESS;
     const int64_t blocks8 = ((n >> 3) + (n & 7) + 255) / 256;
-    if (aligned16(x) && aligned16(y) && blocks8 <= INT32_MAX)
+    if (aligned16(x) && aligned16(y) && blocks8 <= kMaxBlocks256)
         hipLaunchKernelGGL(k_to_bf16_x8, dim3((unsigned)blocks8), dim3(256), 0, as_stream(stream), n, x, y);
     else
         hipLaunchKernelGGL(k_to_bf16, grid_for(n), dim3(256), 0, as_stream(stream), n, x, y);
@@ -194,7 +195,7 @@ int armsp_convert_rows_f32_to_bf16(int M, int N, const float* x, int64_t ldx, ui
     const bool vec = N % 8 == 0 && ldx % 4 == 0 && ldy % 8 == 0 && aligned16(x) && aligned16(y);
     int G = 1;
     while (G < 64 && G * (vec ? 8 : 1) < N) G <<= 1;
-    const dim3 grid((unsigned)(((int64_t)M + 256 / G - 1) / (256 / G)));
+    const dim3 grid((unsigned)std::min(((int64_t)M + 256 / G - 1) / (256 / G), kMaxBlocks256));
     if (vec)
         hipLaunchKernelGGL((k_rows_to_bf16_2d<true>), grid, dim3(256), 0, as_stream(stream), M, N, G, x, ldx, y, ldy);
     else

@@ -35,10 +35,27 @@ static void no_memory() {
     CHECK(fake::asked.size() == 2 && fake::launches.size() == 2);  // the partition and the product
 }
 
+// Sizes that a device's memory holds, whose launches pass 2^32 threads if each row (or
+// eight values) takes a workgroup's lanes of its own.
+static void launch_limits() {
+    fake::reset();
+    CHECK(armsp_spmm_max_f32(16 << 20, 1000, 257, 1 << 20, i32(), i32(), nullptr, f32(), 257, -1e4f, f32(), 257, i32(),
+                             nullptr) == ARMSP_SUCCESS);
+    int64_t blocks = 0;
+    for (const auto& l : fake::launches) blocks += l.grid.x;
+    CHECK(blocks >= 5 * (int64_t)(16 << 20) / 4);  // five column tiles of 64, four rows a workgroup
+    uint16_t* y = reinterpret_cast<uint16_t*>(i32());
+    CHECK(armsp_convert_rows_f32_to_bf16(80 << 20, 264, f32(), 264, y, 264, nullptr) == ARMSP_SUCCESS);
+    CHECK(armsp_convert_rows_f32_to_bf16(80 << 20, 33, f32(), 33, y, 33, nullptr) == ARMSP_SUCCESS);
+    CHECK(armsp_convert_f32_to_bf16(((int64_t)1 << 35) + 8, f32(), y, nullptr) == ARMSP_SUCCESS);
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "no_memory"))
         no_memory();
+    else if (!std::strcmp(what, "launch_limits"))
+        launch_limits();
     else
         return 2;
     return fails ? 1 : 0;
