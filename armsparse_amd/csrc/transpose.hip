@@ -619,17 +619,14 @@ void radix_pass(const RadixPlan& p, int pass, int n, const Records& in, bool csr
 
 // Stable sort of the records by key.  With rowptr, a is the row of each entry of a
 // CSR matrix.  The passes alternate between buf[0] and buf[1] (k, a, v each; `from`:
-// the one to write first); the last one writes a and v to a_last and v_last when
-// they are given.  Returns the sorted records.  other, krange, orange, bad: the
-// range check of k_radix_hist, done by the first pass.
+// the one to write first).  Returns the sorted records.  other, krange, orange, bad:
+// the range check of k_radix_hist, done by the first pass.
 Records radix_sort(const RadixPlan& p, int n, Records in, int M, const int* rowptr, int* hist, int* const (*buf)[3],
-                   int from, int* a_last, float* v_last, const int* other, int krange, int orange, int* bad,
-                   hipStream_t s) {
+                   int from, const int* other, int krange, int orange, int* bad, hipStream_t s) {
     for (int pass = 0; pass < p.passes; ++pass) {
-        const bool last = pass == p.passes - 1;
         int* const* o = buf[(from + pass) & 1];
-        int* ao = last && a_last ? a_last : o[1];
-        float* vo = last && a_last ? v_last : reinterpret_cast<float*>(o[2]);
+        int* ao = o[1];
+        float* vo = reinterpret_cast<float*>(o[2]);
         const bool csr = rowptr && pass == 0;
         const int* chk = pass == 0 ? other : nullptr;
         if (p.tile == RADIX_BIG_TILE)
@@ -835,15 +832,16 @@ extern "C" int armsp_csr_transpose(int M, int K, int nnz, const int* rowptr, con
     const size_t n4 = ((size_t)nnz * 4 + 255) & ~(size_t)255;
     const size_t h4 = (radix_hist_ints(plan) * 4 + 255) & ~(size_t)255;
     void* ws = nullptr;
-    int st = ws_alloc(&ws, (plan.passes > 2 ? 6 : plan.passes > 1 ? 4 : 1) * n4 + h4, s);
+    int st = ws_alloc(&ws, (plan.passes == 1 ? 1 : val ? 4 : 3) * n4 + h4, s);
     if (st) return st;
     char* p = static_cast<char*>(ws);
     int* hist = reinterpret_cast<int*>(p);
     auto arr = [&](int i) { return reinterpret_cast<int*>(p + h4 + i * n4); };
-    // the last pass writes only its keys here; the passes before it, whole records
-    int* const buf[2][3] = {{arr(0), arr(4), arr(5)}, {arr(1), arr(2), arr(3)}};
+    // the last pass, and every second one before it, writes rows and values to the
+    // outputs: what a pass reads is never what it writes
+    int* const buf[2][3] = {{arr(0), rowind, reinterpret_cast<int*>(valT)}, {arr(1), arr(2), arr(3)}};
     const Records sorted = radix_sort(plan, nnz, Records{colind, nullptr, val}, M, rowptr, hist, buf,
-                                      (plan.passes - 1) & 1, rowind, valT, nullptr, 0, 0, nullptr, s);
+                                      (plan.passes - 1) & 1, nullptr, 0, 0, nullptr, s);
     hipLaunchKernelGGL(k_colptr, dim3((unsigned)(((int64_t)nnz / 4 + 1 + 255) / 256)), dim3(256), 0, s, nnz, K,
                        sorted.k, colptr);
     hipError_t e = hipGetLastError();
@@ -891,10 +889,10 @@ extern "C" int armsp_coo_to_csr(int M, int K, int nnz, const int* rows, const in
     // stays inside its buffers whatever they are, and k_coo_emit writes nothing when
     // one is out of range: a single wait at the end serves the check.
     hipLaunchKernelGGL(k_clear_int, dim3(1), dim3(1), 0, s, bad);
-    const Records bc = radix_sort(pc, nnz, Records{cols, rows, vals}, 0, nullptr, hist, buf, 0, nullptr, nullptr,
-                                  rows, K, M, bad, s);
-    const Records br = radix_sort(pr, nnz, Records{bc.a, bc.k, bc.v}, 0, nullptr, hist, buf, pc.passes & 1, nullptr,
-                                  nullptr, nullptr, 0, 0, nullptr, s);
+    const Records bc = radix_sort(pc, nnz, Records{cols, rows, vals}, 0, nullptr, hist, buf, 0, rows, K, M,
+                                  bad, s);
+    const Records br = radix_sort(pr, nnz, Records{bc.a, bc.k, bc.v}, 0, nullptr, hist, buf, pc.passes & 1,
+                                  nullptr, 0, 0, nullptr, s);
     hipLaunchKernelGGL(k_coo_count, dim3((unsigned)ctiles), dim3(TPB), 0, s, nnz, M, br.k, br.a, br.v,
                        drop_zeros, cnt);
     exclusive_scan(ctiles, cnt, scanws, s);

@@ -50,12 +50,25 @@ static void launch_limits() {
     CHECK(armsp_convert_f32_to_bf16(((int64_t)1 << 35) + 8, f32(), y, nullptr) == ARMSP_SUCCESS);
 }
 
+// The transpose of a matrix of more than 2^20 columns (three passes) asks for at most the
+// five arrays of nonzeros and the counts of 256 digits per 4096 that its first form took.
+static void transpose_workspace() {
+    const int nnz = 1 << 26;
+    for (float* val : {(float*)nullptr, f32()}) {
+        fake::reset();
+        CHECK(armsp_csr_transpose(1 << 20, (1 << 20) + 1, nnz, i32(), i32(), val, i32(), i32(), val, nullptr) == ARMSP_SUCCESS);
+        CHECK(fake::asked.size() == 1 && fake::asked[0] <= 5 * (size_t)nnz * 4 + (size_t)nnz / 4096 * 256 * 4);
+    }
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "no_memory"))
         no_memory();
     else if (!std::strcmp(what, "launch_limits"))
         launch_limits();
+    else if (!std::strcmp(what, "transpose_workspace"))
+        transpose_workspace();
     else
         return 2;
     return fails ? 1 : 0;
