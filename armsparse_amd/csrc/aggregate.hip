@@ -89,7 +89,8 @@ __device__ __forceinline__ void max_long_rows(int wave, int j0, int j1, int tile
     const bool active = col < N;
     const float* bp = B + (active ? col : tile0);  // lanes past N read the tile's first column
     int carry = -1;
-    for (int rb = uniform(rows_ending_by_wave(j0, rowptr, M)); rb < M; rb += 64) {
+    int idle = 0;  // windows of 64 rows in a row that held no entry
+    for (int rb = uniform(rows_ending_by_wave(j0, rowptr, M)); rb < M;) {
         const int rl = rb + lane;
         const int sl = rl < M ? rowptr[rl] : INT_MAX, el = rl < M ? rowptr[rl + 1] : INT_MAX;
         // (a malformed rowptr cannot carry the walk outside its range: see the clamps below)
@@ -156,7 +157,16 @@ __device__ __forceinline__ void max_long_rows(int wave, int j0, int j1, int tile
                 }
             }
         }
-        if (read_lane(el, 63) >= j1) break;  // later rows begin after the range
+        const int e63 = read_lane(el, 63);
+        if (e63 >= j1) break;  // later rows begin after the range
+        // a long run of empty rows is searched for its end, not walked (a million of them:
+        // 16,000 dependent steps); short ones pass sooner than a search does
+        idle = e63 == read_lane(sl, 0) ? idle + 1 : 0;
+        rb += 64;
+        if (idle == 4) {
+            rb = max(rb, uniform(rows_ending_by_wave(e63, rowptr, M)));
+            idle = 0;
+        }
     }
     if (tile0 == 0 && lane == 0) parts.carry_row[wave] = carry;
 }
