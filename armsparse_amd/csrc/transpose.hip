@@ -45,6 +45,12 @@ constexpr int SCAN_CHUNK = 2048;  // 256 threads × 8
 // that XCD's L2 (in launch order instead: 480 -> 503 us).
 constexpr int RADIX_MAX_BITS = 10;
 constexpr int RADIX_MIN_BITS = 4;  // k_radix_scan takes 16 digits a workgroup
+// A tile of more rows than so many times its records finds each record's row by a search:
+// walking the rows, few of which hold an entry, would make that tile's time.  Uniform
+// matrices of 2^19 columns, rows walked against searched: 4M entries in 4096-record tiles,
+// 8, 16 and 64 rows an entry 168, 256, 1001 us against 209, 326, 553; 100,000 entries in
+// 2048-record tiles, 8, 16, 64, 200 rows an entry 56, 68, 185, 608 us against 57, 58, 65, 82.
+constexpr int radix_mark_rows(int threads) { return threads > 256 ? 24 : 8; }
 
 // Tile of block b: XCD b % 8 walks a contiguous eighth of the tiles (-1: none).
 __device__ __forceinline__ int xcd_tile(int ntiles) {
@@ -203,35 +209,53 @@ __global__ __launch_bounds__(THREADS) void k_radix_scatter(int n, int shift, int
     }
     for (int i = tid; i < WAVES * bins / 2; i += THREADS) reinterpret_cast<uint32_t*>(wcnt)[i] = 0u;
     if constexpr (CSR_ROWS) {
-        // every row that begins inside the tile marks its first entry (the last such
-        // row where empty rows share it); a running maximum over the marks gives rows
-        for (int i = tid; i < T; i += THREADS) stage[i] = 0;
         const int p0 = (int)tbase, p1 = p0 + cnt;
-        const int r0 = uniform(min(rows_ending_by_wave(p0, rowptr, M), M - 1));
-        __syncthreads();
-        for (int rb = r0 + 1 + w * 64; rb < M; rb += THREADS) {
-            const int r = rb + lane;
-            const int b = r < M ? rowptr[r] : INT_MAX;
-            if (b >= p0 && b < p1) atomicMax(&stage[b - p0], r - r0);
-            if (read_lane(b, 0) >= p1) break;  // later rows begin after the tile
+        // rows of the tile's first and last entry
+        if (w < 2) {
+            const int r = min(rows_ending_by_wave(w ? p1 - 1 : p0, rowptr, M), M - 1);
+            if (lane == 0) red[w] = r;
         }
+        for (int i = tid; i < T; i += THREADS) stage[i] = 0;
         __syncthreads();
-        int run = 0;
+        const int r0 = uniform(red[0]), r1 = max(uniform(red[1]), r0);
+        __syncthreads();
+        if (r1 - r0 <= radix_mark_rows(THREADS) * T) {
+            // every row that begins inside the tile marks its first entry (the last such
+            // row where empty rows share it); a running maximum over the marks gives rows
+            for (int rb = r0 + 1 + w * 64; rb <= r1; rb += THREADS) {
+                const int r = rb + lane;
+                const int b = r <= r1 ? rowptr[r] : INT_MAX;
+                if (b >= p0 && b < p1) atomicMax(&stage[b - p0], r - r0);
+            }
+            __syncthreads();
+            int run = 0;
 #pragma unroll
-        for (int r = 0; r < IPT; ++r) {  // the lane's row: the last mark at or before it
-            const int m = stage[w * WT + r * 64 + lane];
-            const uint64_t marks = __ballot(m != 0) & (~0ull >> (63 - lane));
-            const int from = __shfl(m, marks ? 63 - __builtin_clzll(marks) : 0);
-            a[r] = marks ? from : run;
-            run = read_lane(a[r], 63);
+            for (int r = 0; r < IPT; ++r) {  // the lane's row: the last mark at or before it
+                const int m = stage[w * WT + r * 64 + lane];
+                const uint64_t marks = __ballot(m != 0) & (~0ull >> (63 - lane));
+                const int from = __shfl(m, marks ? 63 - __builtin_clzll(marks) : 0);
+                a[r] = marks ? from : run;
+                run = read_lane(a[r], 63);
+            }
+            if (lane == 0) red[w] = run;
+            __syncthreads();
+            int before = 0;
+#pragma unroll
+            for (int q = 0; q < WAVES; ++q) before = max(before, q < w ? red[q] : 0);
+#pragma unroll
+            for (int r = 0; r < IPT; ++r) a[r] = r0 + max(a[r], before);
+        } else {
+            // mostly empty rows: each record searches the last row that begins at or before it
+#pragma unroll
+            for (int r = 0; r < IPT; ++r) a[r] = r0;
+            for (int step = 1 << (31 - __builtin_clz(r1 - r0)); step; step >>= 1) {
+#pragma unroll
+                for (int r = 0; r < IPT; ++r) {
+                    const int i = min(w * WT + r * 64 + lane, cnt - 1);
+                    if (step <= r1 - a[r] && rowptr[a[r] + step] <= p0 + i) a[r] += step;
+                }
+            }
         }
-        if (lane == 0) red[w] = run;
-        __syncthreads();
-        int before = 0;
-#pragma unroll
-        for (int q = 0; q < WAVES; ++q) before = max(before, q < w ? red[q] : 0);
-#pragma unroll
-        for (int r = 0; r < IPT; ++r) a[r] = r0 + max(a[r], before);
     }
     __syncthreads();
     // rank among the wave's records of the same digit, in order

@@ -55,3 +55,37 @@ def test_max_over_a_run_of_empty_rows():
         times.append(best_ms(lambda: kernels.spmm_max(*d)))
     print("run of empty rows at the end, in the middle: %.3f, %.3f ms" % tuple(times))
     assert times[1] <= 3 * times[0]
+
+
+def transposed(rp, ci, va, k):
+    order = np.argsort(ci, kind="stable")
+    cp = np.zeros(k + 1, np.int32)
+    np.cumsum(np.bincount(ci, minlength=k), out=cp[1:])
+    rows = np.repeat(np.arange(len(rp) - 1, dtype=np.int32), np.diff(rp))
+    return cp, rows[order], va[order]
+
+
+def test_transpose_over_a_run_of_empty_rows():
+    m, each, k = 4_000_000, 1000, 300
+    times = []
+    for middle in (False, True):
+        rp, ci, va = gap(m, each, k, 5, middle)
+        d = dev(rp, ci, va)
+        for got, want in zip(kernels.csr_transpose(*d, k), transposed(rp, ci, va, k)):
+            assert np.array_equal(got.cpu().numpy(), want)
+        times.append(best_ms(lambda: kernels.csr_transpose(*d, k)))
+    print("run of empty rows at the end, in the middle: %.3f, %.3f ms" % tuple(times))
+    assert times[1] <= 3 * times[0]
+
+
+@pytest.mark.parametrize("nnz,rows_per_entry", [(n, q) for n in (1, 2047, 2049, 70_000) for q in (7, 8, 9, 100)] +
+                         [((2 << 20) + n, q) for n in (5, 4095) for q in (23, 25)])
+def test_transpose_of_mostly_empty_rows(nnz, rows_per_entry):
+    """Tiles on both sides of the number of rows from which records search for theirs."""
+    m, k = nnz * rows_per_entry, 1500
+    r = np.random.default_rng(nnz)
+    rp = np.zeros(m + 1, np.int32)
+    np.cumsum(np.bincount(r.integers(0, m, nnz), minlength=m), out=rp[1:])
+    ci, va = r.integers(0, k, nnz).astype(np.int32), r.standard_normal(nnz).astype(np.float32)
+    for got, want in zip(kernels.csr_transpose(*dev(rp, ci, va), k), transposed(rp, ci, va, k)):
+        assert np.array_equal(got.cpu().numpy(), want)
