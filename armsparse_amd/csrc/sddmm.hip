@@ -174,144 +174,167 @@ __device__ __forceinline__ void gather_vec(__amdgpu_buffer_rsrc_t rs, uint32_t o
     }
 }
 
-// S = 2: the dot products are split into two column halves, and blocks are
-// numbered so that the 8 XCDs (block b runs on XCD b % 8) alternate halves: each
-// XCD's L2 then caches half of every hot V row.  Half 0 goes to out, half 1 to
-// out2; k_sddmm_combine adds them and scales.  With `skew` the device decides:
-// split where *skew says so (merge_partition).
+// The nonzeros of one wave: chunk items from wave·chunk on.
+template <typename T, int G, int W, bool COO, bool FULL>
+__device__ __forceinline__ void sddmm_chunk(int wave, int M, int Kd, int nnz, int chunk,
+                                            const int* __restrict__ rowidx, const int* __restrict__ colind,
+                                            const float* __restrict__ scale, const T* __restrict__ U, int ldu,
+                                            const T* __restrict__ V, int ldv, const int* __restrict__ part,
+                                            float* __restrict__ out) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63;
+    const int wid = threadIdx.x >> 6;
+    const int g = lane / G, l = lane & (G - 1);
+    const int64_t total = COO ? (int64_t)nnz : (int64_t)M + nnz;
+    const int64_t d0l = (int64_t)wave * chunk;
+    if (d0l >= total) return;
+    const int d0 = (int)d0l;
+    const int d1 = (int)min(d0l + chunk, total);
+    int i0 = 0, j0 = d0, j1 = d1;
+    if constexpr (!COO) {
+        int i1;
+        chunk_rows(part, wave, d0, d1, rowidx, M, nnz, i0, i1);
+        j0 = d0 - i0;
+        j1 = d1 - i1;
+    }
+    const int nz = j1 - j0;
+    const size_t wstride = ((size_t)chunk * 8 + (size_t)(chunk + 1) * 4 + 15) & ~(size_t)15;
+    uint2* s_off = reinterpret_cast<uint2*>(smem + wid * wstride);
+    int* s_re = reinterpret_cast<int*>(smem + wid * wstride + (size_t)chunk * 8);
+    const uint32_t urow = (uint32_t)ldu * (uint32_t)sizeof(T), vrow = (uint32_t)ldv * (uint32_t)sizeof(T);
+    int nre = 0;
+    if constexpr (!COO) {
+        nre = d1 - d0 - nz + 1;  // row ends of rows i0..i1
+        for (int k = lane; k < nre; k += 64) s_re[k] = (i0 + k < M) ? rowidx[i0 + k + 1] : INT_MAX;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    const int nzr = (nz + 63) & ~63;
+    for (int k = lane; k < nzr; k += 64) {
+        uint2 o = make_uint2(0u, 0u);
+        if (k < nz) {
+            const int e = j0 + k;
+            int r;
+            if constexpr (COO) {
+                r = __builtin_nontemporal_load(rowidx + e);
+            } else {  // rows i0 + (number of row ends ≤ e)
+                int lo = 0, hi = nre - 1;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (s_re[mid] <= e)
+                        lo = mid + 1;
+                    else
+                        hi = mid;
+                }
+                r = i0 + lo;
+            }
+            o = make_uint2((uint32_t)r * urow, (uint32_t)__builtin_nontemporal_load(colind + e) * vrow);
+        }
+        s_off[k] = o;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+    const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(U), (short)0, (int)0xffffffff,
+                                                                         0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(V), (short)0, (int)0xffffffff,
+                                                                         0x00020000);
+    const int steps = (Kd + G * W - 1) / (G * W);  // FULL: Kd = steps·G·W; else Kd % W == 0
+    // dot products whose operands are fetched together: 16 floats of each operand per lane
+    constexpr int QB = (16 / W) < G ? (16 / W) : G;
+
+    for (int base = 0; base < nz; base += 64) {
+        float p[G];
+#pragma unroll
+        for (int q = 0; q < G; ++q) p[q] = 0.0f;
+        for (int t = 0; t < steps; ++t) {
+            const int k = (t * G + l) * W;
+            const bool in = FULL || k < Kd;  // lanes past Kd in the last step read column 0, use 0
+            const uint32_t lo = in ? (uint32_t)(k * (int)sizeof(T)) : 0u;
+#pragma unroll
+            for (int qb = 0; qb < G; qb += QB) {
+                float a[QB][W], b[QB][W];
+#pragma unroll
+                for (int q = 0; q < QB; ++q) {
+                    const uint2 o = s_off[base + g * G + qb + q];
+                    gather_vec<T, W>(ru, o.x + lo, a[q]);
+                    gather_vec<T, W>(rv, o.y + lo, b[q]);
+                    if (!FULL && !in) {
+#pragma unroll
+                        for (int i = 0; i < W; ++i) a[q][i] = 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < QB; ++q)
+#pragma unroll
+                    for (int i = 0; i < W; ++i) p[qb + q] = fmaf(a[q][i], b[q][i], p[qb + q]);
+                // keep the next batch's loads below this point: bounded registers, more waves
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int m = G / 2; m >= 1; m >>= 1) {
+            const bool upper = (l & m) != 0;
+#pragma unroll
+            for (int i = 0; i < m; ++i) {
+                const float send = upper ? p[i] : p[i + m];
+                const float keep = upper ? p[i + m] : p[i];
+                p[i] = keep + __shfl_xor(send, m);
+            }
+        }
+        const int e = base + lane;
+        if (e < nz) {
+            const int ge = j0 + e;
+            out[ge] = scale ? scale[ge] * p[0] : p[0];
+        }
+    }
+}
+
 template <typename T, int G, int W, bool COO, bool FULL>
 __global__ __launch_bounds__(256) void k_sddmm_stream(int M, int Kd, int nnz, int chunk,
                                                       const int* __restrict__ rowidx, const int* __restrict__ colind,
                                                       const float* __restrict__ scale, const T* __restrict__ U,
                                                       int ldu, const T* __restrict__ V, int ldv,
-                                                      const int* __restrict__ part, float* __restrict__ out, int S,
-                                                      int ngroups, float* __restrict__ out2,
-                                                      const int* __restrict__ skew) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
-    const int g = lane / G, l = lane & (G - 1);
-    if (skew) S = *skew ? 2 : 1;
-    if (S == 2) Kd >>= 1;
+                                                      const int* __restrict__ part, float* __restrict__ out) {
+    sddmm_chunk<T, G, W, COO, FULL>(uniform((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)), M, Kd, nnz, chunk, rowidx,
+                                    colind, scale, U, ldu, V, ldv, part, out);
+}
+
+// CSR products whose dot products are split into two column halves, and blocks are
+// numbered so that the 8 XCDs (block b runs on XCD b % 8) alternate halves: each
+// XCD's L2 then caches half of every hot V row.  Half 0 goes to out, half 1 to
+// out2; k_sddmm_combine adds them and scales.  ADAPT: the device decides, split where
+// *skew says so (merge_partition), and a workgroup takes two tasks then.  A kernel of its
+// own: the choice and the loop over tasks take 7 to 9 VGPRs, a wave per SIMD of the
+// products that never split (bf16 64 -> 71, COO 64 -> 73: 0.97 times their speed).
+// FULL is the halves', and so the whole rows'.
+template <typename T, int G, int W, bool FULL, bool ADAPT>
+__global__ __launch_bounds__(256) void k_sddmm_split(int M, int Kd, int nnz, int chunk,
+                                                     const int* __restrict__ rowidx, const int* __restrict__ colind,
+                                                     const float* __restrict__ scale, const T* __restrict__ U,
+                                                     int ldu, const T* __restrict__ V, int ldv,
+                                                     const int* __restrict__ part, float* __restrict__ out,
+                                                     int ngroups, float* __restrict__ out2,
+                                                     const int* __restrict__ skew) {
+    const bool split = !ADAPT || *skew;
     // the grid is a multiple of 8, so a workgroup's tasks are of one half
-    for (int task = (int)blockIdx.x; task < S * ngroups; task += (int)gridDim.x) {
-        int grp = task;
-        if (S == 2) {
-            const int x = task & 7;
-            grp = (task >> 3) * 4 + (x >> 1);
-            scale = nullptr;
-            if ((x & 1) && out != out2) {  // the upper half of every row of U and V
-                U += Kd;
-                V += Kd;
-                out = out2;
-            }
+    if (split) {
+        Kd >>= 1;
+        scale = nullptr;
+        if (blockIdx.x & 1u) {  // the upper half of every row of U and V
+            U += Kd;
+            V += Kd;
+            out = out2;
         }
-        const int wave = uniform(grp * 4 + wid);
-        const int64_t total = COO ? (int64_t)nnz : (int64_t)M + nnz;
-        const int64_t d0l = (int64_t)wave * chunk;
-        if (d0l >= total) continue;
-        const int d0 = (int)d0l;
-        const int d1 = (int)min(d0l + chunk, total);
-        int i0 = 0, j0 = d0, j1 = d1;
-        if constexpr (!COO) {
-            int i1;
-            chunk_rows(part, wave, d0, d1, rowidx, M, nnz, i0, i1);
-            j0 = d0 - i0;
-            j1 = d1 - i1;
-        }
-        const int nz = j1 - j0;
-        const size_t wstride = ((size_t)chunk * 8 + (size_t)(chunk + 1) * 4 + 15) & ~(size_t)15;
-        uint2* s_off = reinterpret_cast<uint2*>(smem + wid * wstride);
-        int* s_re = reinterpret_cast<int*>(smem + wid * wstride + (size_t)chunk * 8);
-        const uint32_t urow = (uint32_t)ldu * (uint32_t)sizeof(T), vrow = (uint32_t)ldv * (uint32_t)sizeof(T);
-        int nre = 0;
-        if constexpr (!COO) {
-            nre = d1 - d0 - nz + 1;  // row ends of rows i0..i1
-            for (int k = lane; k < nre; k += 64) s_re[k] = (i0 + k < M) ? rowidx[i0 + k + 1] : INT_MAX;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-        const int nzr = (nz + 63) & ~63;
-        for (int k = lane; k < nzr; k += 64) {
-            uint2 o = make_uint2(0u, 0u);
-            if (k < nz) {
-                const int e = j0 + k;
-                int r;
-                if constexpr (COO) {
-                    r = __builtin_nontemporal_load(rowidx + e);
-                } else {  // rows i0 + (number of row ends ≤ e)
-                    int lo = 0, hi = nre - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if (s_re[mid] <= e)
-                            lo = mid + 1;
-                        else
-                            hi = mid;
-                    }
-                    r = i0 + lo;
-                }
-                o = make_uint2((uint32_t)r * urow, (uint32_t)__builtin_nontemporal_load(colind + e) * vrow);
-            }
-            s_off[k] = o;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-        const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(U), (short)0, (int)0xffffffff,
-                                                                             0x00020000);
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(V), (short)0, (int)0xffffffff,
-                                                                             0x00020000);
-        const int steps = (Kd + G * W - 1) / (G * W);  // FULL: Kd = steps·G·W; else Kd % W == 0
-        // dot products whose operands are fetched together: 16 floats of each operand per lane
-        constexpr int QB = (16 / W) < G ? (16 / W) : G;
-
-        for (int base = 0; base < nz; base += 64) {
-            float p[G];
-#pragma unroll
-            for (int q = 0; q < G; ++q) p[q] = 0.0f;
-            for (int t = 0; t < steps; ++t) {
-                const int k = (t * G + l) * W;
-                const bool in = FULL || k < Kd;  // lanes past Kd in the last step read column 0, use 0
-                const uint32_t lo = in ? (uint32_t)(k * (int)sizeof(T)) : 0u;
-#pragma unroll
-                for (int qb = 0; qb < G; qb += QB) {
-                    float a[QB][W], b[QB][W];
-#pragma unroll
-                    for (int q = 0; q < QB; ++q) {
-                        const uint2 o = s_off[base + g * G + qb + q];
-                        gather_vec<T, W>(ru, o.x + lo, a[q]);
-                        gather_vec<T, W>(rv, o.y + lo, b[q]);
-                        if (!FULL && !in) {
-#pragma unroll
-                            for (int i = 0; i < W; ++i) a[q][i] = 0.0f;
-                        }
-                    }
-#pragma unroll
-                    for (int q = 0; q < QB; ++q)
-#pragma unroll
-                        for (int i = 0; i < W; ++i) p[qb + q] = fmaf(a[q][i], b[q][i], p[qb + q]);
-                    // keep the next batch's loads below this point: bounded registers, more waves
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-#pragma unroll
-            for (int m = G / 2; m >= 1; m >>= 1) {
-                const bool upper = (l & m) != 0;
-#pragma unroll
-                for (int i = 0; i < m; ++i) {
-                    const float send = upper ? p[i] : p[i + m];
-                    const float keep = upper ? p[i + m] : p[i];
-                    p[i] = keep + __shfl_xor(send, m);
-                }
-            }
-            const int e = base + lane;
-            if (e < nz) {
-                const int ge = j0 + e;
-                out[ge] = scale ? scale[ge] * p[0] : p[0];
-            }
-        }
+    }
+    const int tasks = split ? 2 * ngroups : ngroups;
+    for (int task = (int)blockIdx.x; task < tasks; task += (int)gridDim.x) {
+        const int grp = split ? (task >> 3) * 4 + ((task & 7) >> 1) : task;
+        sddmm_chunk<T, G, W, false, FULL>(uniform(grp * 4 + (int)(threadIdx.x >> 6)), M, Kd, nnz, chunk, rowidx, colind,
+                                          scale, U, ldu, V, ldv, part, out);
+        if constexpr (!ADAPT) break;  // a workgroup per task
     }
 }
 
@@ -334,17 +357,27 @@ inline size_t sddmm_lds_bytes(int chunk) {
 template <typename T, int G, int W>
 void launch_sddmm_stream(bool coo, dim3 grid, hipStream_t s, int M, int Kd, int nnz, int chunk, const int* ri,
                          const int* ci, const float* sc, const T* U, int ldu, const T* V, int ldv, const int* part,
-                         float* out, int S, int ngroups, float* out2, const int* skew) {
+                         float* out, bool halves, int ngroups, float* out2, const int* skew) {
     const size_t lds = sddmm_lds_bytes(chunk);
-    const bool full = (S == 2 || skew ? Kd / 2 : Kd) % (G * W) == 0;
+    const bool full = (halves ? Kd / 2 : Kd) % (G * W) == 0;
 #define ARMSP_SDDMM_ST(CO, FU)                                                                                 \
     hipLaunchKernelGGL((k_sddmm_stream<T, G, W, CO, FU>), grid, dim3(256), lds, s, M, Kd, nnz, chunk, ri, ci, sc, U, \
-                       ldu, V, ldv, part, out, S, ngroups, out2, skew)
-    if (coo) {
+                       ldu, V, ldv, part, out)
+#define ARMSP_SDDMM_SP(FU, AD)                                                                                    \
+    hipLaunchKernelGGL((k_sddmm_split<T, G, W, FU, AD>), grid, dim3(256), lds, s, M, Kd, nnz, chunk, ri, ci, sc, U, ldu, \
+                       V, ldv, part, out, ngroups, out2, skew)
+    if (halves && skew) {
+        if constexpr (G <= 8) {  // AUTO's group
+            if (full) ARMSP_SDDMM_SP(true, true); else ARMSP_SDDMM_SP(false, true);
+        }
+    } else if (halves) {
+        if (full) ARMSP_SDDMM_SP(true, false); else ARMSP_SDDMM_SP(false, false);
+    } else if (coo) {
         if (full) ARMSP_SDDMM_ST(true, true); else ARMSP_SDDMM_ST(true, false);
     } else {
         if (full) ARMSP_SDDMM_ST(false, true); else ARMSP_SDDMM_ST(false, false);
     }
+#undef ARMSP_SDDMM_SP
 #undef ARMSP_SDDMM_ST
 }
 
@@ -427,7 +460,7 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
         G = 4;
         while (G < 8 && G * W < KdS) G <<= 1;
     }
-    // workgroups of four waves; a multiple of 8, so that each keeps to one half (and XCD)
+    // workgroups of four waves; for the split a multiple of 8, so that each keeps to one half (and XCD)
     const int ngroups = (int)((nwaves + 31) / 32 * 8);
     // the staged CSR kernel's waves start from a precomputed merge-path partition, when many
     void* ws = nullptr;
@@ -456,15 +489,15 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
             tp.stop();
         }
     }
-    const dim3 grid(staged ? (unsigned)ngroups : (unsigned)((nwaves + 3) / 4));
+    const dim3 grid(split ? 2 * (unsigned)ngroups : adapt ? (unsigned)ngroups : (unsigned)((nwaves + 3) / 4));
     TimedLaunch t("sddmm", s);
 #define ARMSP_SDDMM_G(WW)                                                                                    \
     if (staged) {                                                                                            \
         switch (G) {                                                                                         \
-            case 4: launch_sddmm_stream<T, 4, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
-            case 8: launch_sddmm_stream<T, 8, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
-            case 16: launch_sddmm_stream<T, 16, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
-            default: launch_sddmm_stream<T, 32, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split ? 2 : 1, ngroups, out2, skew); break; \
+            case 4: launch_sddmm_stream<T, 4, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
+            case 8: launch_sddmm_stream<T, 8, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
+            case 16: launch_sddmm_stream<T, 16, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
+            default: launch_sddmm_stream<T, 32, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
         }                                                                                                    \
     } else {                                                                                                 \
         switch (G) {                                                                                         \
