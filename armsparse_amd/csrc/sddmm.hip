@@ -11,6 +11,7 @@
 // restricted to the wave's row range.
 #include <algorithm>
 #include <climits>
+#include <cstdlib>
 
 #include "common.hpp"
 
@@ -251,7 +252,7 @@ __device__ __forceinline__ void sddmm_chunk(int wave, int M, int Kd, int nnz, in
         for (int q = 0; q < G; ++q) p[q] = 0.0f;
         for (int t = 0; t < steps; ++t) {
             const int k = (t * G + l) * W;
-            const bool in = FULL || k < Kd;  // lanes past Kd in the last step read column 0, use 0
+            const bool in = FULL || k < Kd;  // lanes past Kd in the last step read column 0 and drop it
             const uint32_t lo = in ? (uint32_t)(k * (int)sizeof(T)) : 0u;
 #pragma unroll
             for (int qb = 0; qb < G; qb += QB) {
@@ -261,15 +262,13 @@ __device__ __forceinline__ void sddmm_chunk(int wave, int M, int Kd, int nnz, in
                     const uint2 o = s_off[base + g * G + qb + q];
                     gather_vec<T, W>(ru, o.x + lo, a[q]);
                     gather_vec<T, W>(rv, o.y + lo, b[q]);
-                    if (!FULL && !in) {
-#pragma unroll
-                        for (int i = 0; i < W; ++i) a[q][i] = 0.0f;
-                    }
                 }
+                if (FULL || in) {  // (not a zeroed operand: writing it would wait for its load, one by one)
 #pragma unroll
-                for (int q = 0; q < QB; ++q)
+                    for (int q = 0; q < QB; ++q)
 #pragma unroll
-                    for (int i = 0; i < W; ++i) p[qb + q] = fmaf(a[q][i], b[q][i], p[qb + q]);
+                        for (int i = 0; i < W; ++i) p[qb + q] = fmaf(a[q][i], b[q][i], p[qb + q]);
+                }
                 // keep the next batch's loads below this point: bounded registers, more waves
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -302,16 +301,16 @@ __global__ __launch_bounds__(256) void k_sddmm_stream(int M, int Kd, int nnz, in
                                     colind, scale, U, ldu, V, ldv, part, out);
 }
 
-// CSR products whose dot products are split into two column halves, and blocks are
-// numbered so that the 8 XCDs (block b runs on XCD b % 8) alternate halves: each
-// XCD's L2 then caches half of every hot V row.  Half 0 goes to out, half 1 to
-// out2; k_sddmm_combine adds them and scales.  ADAPT: the device decides, split where
+// CSR products whose dot products are split into two column halves, [0, Ka) and [Ka, Kd),
+// and blocks are numbered so that the 8 XCDs (block b runs on XCD b % 8) alternate
+// halves: each XCD's L2 then caches half of every hot V row.  Half 0 goes to out, half
+// 1 to out2; k_sddmm_combine adds them and scales.  ADAPT: the device decides, split where
 // *skew says so (merge_partition), and a workgroup takes two tasks then.  A kernel of its
 // own: the choice and the loop over tasks take 7 to 9 VGPRs, a wave per SIMD of the
 // products that never split (bf16 64 -> 71, COO 64 -> 73: 0.97 times their speed).
-// FULL is the halves', and so the whole rows'.
+// FULL: both halves, and so the whole rows, are whole steps.
 template <typename T, int G, int W, bool FULL, bool ADAPT>
-__global__ __launch_bounds__(256) void k_sddmm_split(int M, int Kd, int nnz, int chunk,
+__global__ __launch_bounds__(256) void k_sddmm_split(int M, int Kd, int Ka, int nnz, int chunk,
                                                      const int* __restrict__ rowidx, const int* __restrict__ colind,
                                                      const float* __restrict__ scale, const T* __restrict__ U,
                                                      int ldu, const T* __restrict__ V, int ldv,
@@ -321,19 +320,21 @@ __global__ __launch_bounds__(256) void k_sddmm_split(int M, int Kd, int nnz, int
     const bool split = !ADAPT || *skew;
     // the grid is a multiple of 8, so a workgroup's tasks are of one half
     if (split) {
-        Kd >>= 1;
         scale = nullptr;
         if (blockIdx.x & 1u) {  // the upper half of every row of U and V
-            U += Kd;
-            V += Kd;
+            U += Ka;
+            V += Ka;
             out = out2;
+            Kd -= Ka;
+        } else {
+            Kd = Ka;
         }
     }
     const int tasks = split ? 2 * ngroups : ngroups;
     for (int task = (int)blockIdx.x; task < tasks; task += (int)gridDim.x) {
         const int grp = split ? (task >> 3) * 4 + ((task & 7) >> 1) : task;
-        sddmm_chunk<T, G, W, false, FULL>(uniform(grp * 4 + (int)(threadIdx.x >> 6)), M, Kd, nnz, chunk, rowidx, colind,
-                                          scale, U, ldu, V, ldv, part, out);
+        const int wave = uniform(grp * 4 + (int)(threadIdx.x >> 6));
+        sddmm_chunk<T, G, W, false, FULL>(wave, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out);
         if constexpr (!ADAPT) break;  // a workgroup per task
     }
 }
@@ -357,20 +358,20 @@ inline size_t sddmm_lds_bytes(int chunk) {
 template <typename T, int G, int W>
 void launch_sddmm_stream(bool coo, dim3 grid, hipStream_t s, int M, int Kd, int nnz, int chunk, const int* ri,
                          const int* ci, const float* sc, const T* U, int ldu, const T* V, int ldv, const int* part,
-                         float* out, bool halves, int ngroups, float* out2, const int* skew) {
+                         float* out, int Ka, int ngroups, float* out2, const int* skew) {
     const size_t lds = sddmm_lds_bytes(chunk);
-    const bool full = (halves ? Kd / 2 : Kd) % (G * W) == 0;
+    const bool full = Kd % (G * W) == 0 && Ka % (G * W) == 0;
 #define ARMSP_SDDMM_ST(CO, FU)                                                                                 \
     hipLaunchKernelGGL((k_sddmm_stream<T, G, W, CO, FU>), grid, dim3(256), lds, s, M, Kd, nnz, chunk, ri, ci, sc, U, \
                        ldu, V, ldv, part, out)
 #define ARMSP_SDDMM_SP(FU, AD)                                                                                    \
-    hipLaunchKernelGGL((k_sddmm_split<T, G, W, FU, AD>), grid, dim3(256), lds, s, M, Kd, nnz, chunk, ri, ci, sc, U, ldu, \
+    hipLaunchKernelGGL((k_sddmm_split<T, G, W, FU, AD>), grid, dim3(256), lds, s, M, Kd, Ka, nnz, chunk, ri, ci, sc, U, ldu, \
                        V, ldv, part, out, ngroups, out2, skew)
-    if (halves && skew) {
+    if (Ka && skew) {
         if constexpr (G <= 8) {  // AUTO's group
             if (full) ARMSP_SDDMM_SP(true, true); else ARMSP_SDDMM_SP(false, true);
         }
-    } else if (halves) {
+    } else if (Ka) {
         if (full) ARMSP_SDDMM_SP(true, false); else ARMSP_SDDMM_SP(false, false);
     } else if (coo) {
         if (full) ARMSP_SDDMM_ST(true, true); else ARMSP_SDDMM_ST(true, false);
@@ -460,6 +461,15 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
         G = 4;
         while (G < 8 && G * W < KdS) G <<= 1;
     }
+    // The lower half ends at the whole step of G·W columns nearest the middle, where there is
+    // one inside the row, so at most the upper half ends in a part-empty step and its rows
+    // start on a line where the whole rows do (halves of Kd / 2: fp32 160 on the 1M R-MAT of
+    // 2^23 nonzeros 641 us unsplit, 1050 split, 635 so; 136: 771, 1054, 750).  AUTO splits
+    // only where the halves then differ by less than a step (fp32 160 and 224 stay unsplit:
+    // half the XCDs would have 1.5 and 1.3 times the others' work).
+    int Ka = (KdS + G * W / 2) / (G * W) * (G * W);
+    if (Ka <= 0 || Ka >= Kd) Ka = KdS;
+    if (Ka % (G * W) != 0 || std::abs(Kd - 2 * Ka) >= G * W) adapt = false;
     // workgroups of four waves; for the split a multiple of 8, so that each keeps to one half (and XCD)
     const int ngroups = (int)((nwaves + 31) / 32 * 8);
     // the staged CSR kernel's waves start from a precomputed merge-path partition, when many
@@ -494,10 +504,10 @@ int sddmm_impl(bool coo, int M, int K, int Kd, int nnz, const int* rowidx, const
 #define ARMSP_SDDMM_G(WW)                                                                                    \
     if (staged) {                                                                                            \
         switch (G) {                                                                                         \
-            case 4: launch_sddmm_stream<T, 4, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
-            case 8: launch_sddmm_stream<T, 8, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
-            case 16: launch_sddmm_stream<T, 16, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
-            default: launch_sddmm_stream<T, 32, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt, ngroups, out2, skew); break; \
+            case 4: launch_sddmm_stream<T, 4, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt ? Ka : 0, ngroups, out2, skew); break; \
+            case 8: launch_sddmm_stream<T, 8, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt ? Ka : 0, ngroups, out2, skew); break; \
+            case 16: launch_sddmm_stream<T, 16, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt ? Ka : 0, ngroups, out2, skew); break; \
+            default: launch_sddmm_stream<T, 32, WW>(coo, grid, s, M, Kd, nnz, chunk, rowidx, colind, scale, U, ldu, V, ldv, part, out, split || adapt ? Ka : 0, ngroups, out2, skew); break; \
         }                                                                                                    \
     } else {                                                                                                 \
         switch (G) {                                                                                         \
