@@ -1333,10 +1333,14 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
                                           (esz == 2 && N * esz >= 128 && N * esz < 512 && (N * esz) % 128 == 0));
     // half-wave slices, and a whole wave per nonzero on narrow rows of B (N < 32), run
     // best with 256 items per wave; slices with 4 gathers per batch, narrow rows with 8
-    // (a 825,000-row R-MAT of 12.5M nonzeros, bf16 N = 8: 240 us with 4, 190 with 8)
+    // (a 825,000-row R-MAT of 12.5M nonzeros, bf16 N = 8: 240 us with 4, 190 with 8; seven
+    // uniform and R-MAT matrices, N = 5 to 31: 1 to 24% less time), but for fp8, and fp32 of
+    // 24 columns and more, on rows of under 8 nonzeros, which end inside most batches
+    // (uniform 141,670 rows of 6: fp8 N = 16 30.8 us with 4, 35.5 with 8; fp32 N = 24 32.2, 33.2)
     if (merge && !wide && !narrow && c.group == 0 && (slice_rows || N < 32)) {
         if (c.chunk <= 0) chunk = 256;
-        if (c.unroll <= 0) U = slice_rows ? 4 : 8;
+        const bool short_rows = nnz < 8 * (int64_t)M && (esz == 1 || (esz == 4 && N >= 24));
+        if (c.unroll <= 0) U = slice_rows || short_rows ? 4 : 8;
     }
     if (narrow) {  // default: runs of 8 items for N ≤ 2, of 4 above (the staged products fill the LDS)
         if (c.chunk <= 0) chunk = N <= 2 ? 512 : 256;
@@ -1352,7 +1356,7 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
         // fp32 rows of more than 64 columns and under 24 nonzeros a row on average: 256 items
         // and 4 gathers per batch, which leave more waves on a CU, where 512 are to be had
         // (R-MAT of 150,000 rows, 2M nonzeros, N = 100: 121 -> 98 us; uniform matrices the
-        // same within 1%; with one value a lane uniform matrices lose up to 6%, in bf16 20%).
+        // same within 2%; with one value a lane uniform matrices lose up to 6%, in bf16 20%).
         // Not where their carries, 4·(N + 2) bytes a chunk, outgrow the array of the entry
         // point that allocates nothing: it takes what it would with 512, and both entry
         // points choose alike

@@ -10,12 +10,20 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
+#include <map>
+#include <string>
 #include <vector>
 
 namespace fake {
 struct Launch {
+    std::string kernel;  // mangled
     dim3 grid, block;
 };
+// kernels by the host address that launches name; filled while the library is loaded
+inline std::map<const void*, std::string>& kernels() {
+    static std::map<const void*, std::string> k;
+    return k;
+}
 inline hipError_t pending = hipSuccess;
 inline size_t memory = ~(size_t)0;  // what one allocation can get
 inline std::vector<size_t> asked;   // sizes of the allocations, also of those that failed
@@ -36,6 +44,15 @@ inline void reset() {
 #undef hipGetDevice
 #undef hipMallocFromPoolAsync
 extern "C" {
+void** __hipRegisterFatBinary(const void*) {
+    static void* module;
+    return &module;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+    fake::kernels()[host] = name;
+}
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError() {
@@ -68,14 +85,14 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
     *grid = fake::next_grid, *block = fake::next_block, *lds = fake::next_lds, *s = fake::next_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
     const dim3 g = grid, b = block;
     const uint64_t x = (uint64_t)g.x * b.x, y = (uint64_t)g.y * b.y, z = (uint64_t)g.z * b.z;
     if (!x || !y || !z) return fake::fail(hipErrorInvalidConfiguration);
     if (x > UINT32_MAX || y > UINT32_MAX || z > UINT32_MAX || g.y > 65535 || g.z > 65535 ||
         (uint64_t)b.x * b.y * b.z > 1024)
         return fake::fail(hipErrorInvalidConfiguration);
-    fake::launches.push_back({g, b});
+    fake::launches.push_back({fake::kernels()[f], g, b});
     return hipSuccess;
 }
 }

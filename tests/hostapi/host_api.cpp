@@ -61,6 +61,39 @@ static void transpose_workspace() {
     }
 }
 
+static bool launched(const std::string& part) {
+    for (const auto& l : fake::launches)
+        if (l.kernel.find(part) != std::string::npos) return true;
+    return false;
+}
+
+// Gathers per batch (the last template argument) of an automatic product on rows of B under
+// 32 columns, by type, width and the nonzeros a row holds.
+static void narrow_batches() {
+    const int M = 141670, nnz = 870517;  // 6 a row
+    const uint8_t* q = reinterpret_cast<const uint8_t*>(f32());
+    auto fp8 = [&](int nz, int n) {
+        fake::reset();
+        CHECK(armsp_spmm_fp8(M, M, n, nz, i32(), i32(), f32(), q, f32(), n, f32(), n, 0, nullptr, nullptr) == ARMSP_SUCCESS);
+    };
+    auto fp32 = [&](int nz, int n) {
+        fake::reset();
+        CHECK(armsp_spmm_f32(M, M, n, nz, i32(), i32(), f32(), f32(), n, f32(), n, 0, nullptr, nullptr) == ARMSP_SUCCESS);
+    };
+    for (int n : {5, 16, 31}) {
+        fp8(nnz, n);
+        CHECK(launched("k_spmm_streamIhfLi1ELi4E"));
+        fp8(4 * nnz, n);
+        CHECK(launched("k_spmm_streamIhfLi1ELi8E"));
+    }
+    fp32(nnz, 16);
+    CHECK(launched("k_spmm_streamIffLi1ELi8E"));
+    fp32(nnz, 24);
+    CHECK(launched("k_spmm_streamIffLi1ELi4E"));
+    fp32(4 * nnz, 24);
+    CHECK(launched("k_spmm_streamIffLi1ELi8E"));
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "no_memory"))
@@ -69,6 +102,8 @@ int main(int argc, char** argv) {
         launch_limits();
     else if (!std::strcmp(what, "transpose_workspace"))
         transpose_workspace();
+    else if (!std::strcmp(what, "narrow_batches"))
+        narrow_batches();
     else
         return 2;
     return fails ? 1 : 0;
