@@ -338,7 +338,9 @@ int vcsr_long_blocks() {
 // 1.5 ms for the 1M R-MAT's 10^5 medium rows, one per wave 117 us, one per 1024
 // rows 13 us, one per 8192 8 us).
 constexpr int VCSR_FIND_THREADS = 1024;
-// Rows per thread: 8, or 1 for matrices of few workgroups.
+// R rows per thread, as many as leave 256 workgroups or more: with fewer the CUs without one
+// wait for the others' loads (calls on uniform matrices with R = 1, 2, 4, 8: 200,000 rows of
+// 5 26.2, 26.8, 27.8, 30.1 us; 2^20 rows of 16 312, 307, 304, 305).
 template <int R>
 __global__ __launch_bounds__(VCSR_FIND_THREADS) void k_vcsr_find_long(int M, const int* __restrict__ rowptr,
                                                                       int long_blocks, int* __restrict__ list,
@@ -832,13 +834,19 @@ int armsp_spmv_vcsr_f32(int M, int nnz_padded, const int* rowptr, const int* col
         list = count + 64;
         list_med = list + M;
         hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, s, count);
-        if (M <= 128 * VCSR_FIND_THREADS)
-            hipLaunchKernelGGL((k_vcsr_find_long<1>), dim3((unsigned)((M + VCSR_FIND_THREADS - 1) / VCSR_FIND_THREADS)),
-                               dim3(VCSR_FIND_THREADS), 0, s, M, rowptr, long_blocks, list, list_med, count);
+        auto find = [&](auto kernel, int rows) {  // rows per thread
+            const int64_t per = (int64_t)rows * VCSR_FIND_THREADS;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)((M + per - 1) / per)), dim3(VCSR_FIND_THREADS), 0, s, M, rowptr,
+                               long_blocks, list, list_med, count);
+        };
+        if (M <= 1 << 18)
+            find(k_vcsr_find_long<1>, 1);
+        else if (M <= 1 << 19)
+            find(k_vcsr_find_long<2>, 2);
+        else if (M <= 1 << 22)
+            find(k_vcsr_find_long<4>, 4);
         else
-            hipLaunchKernelGGL((k_vcsr_find_long<8>),
-                               dim3((unsigned)(((int64_t)M + 8 * VCSR_FIND_THREADS - 1) / (8 * VCSR_FIND_THREADS))),
-                               dim3(VCSR_FIND_THREADS), 0, s, M, rowptr, long_blocks, list, list_med, count);
+            find(k_vcsr_find_long<8>, 8);
     }
     TimedLaunch t("spmv_vcsr", s);
     const unsigned short_wg = (unsigned)(((int64_t)M * 4 + 255) / 256);

@@ -18,6 +18,7 @@ namespace fake {
 struct Launch {
     std::string kernel;  // mangled
     dim3 grid, block;
+    int arg2;  // the third argument, for kernels whose third is an int
 };
 // kernels by the host address that launches name; filled while the library is loaded
 inline std::map<const void*, std::string>& kernels() {
@@ -85,14 +86,15 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
     *grid = fake::next_grid, *block = fake::next_block, *lds = fake::next_lds, *s = fake::next_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t, hipStream_t) {
     const dim3 g = grid, b = block;
     const uint64_t x = (uint64_t)g.x * b.x, y = (uint64_t)g.y * b.y, z = (uint64_t)g.z * b.z;
     if (!x || !y || !z) return fake::fail(hipErrorInvalidConfiguration);
     if (x > UINT32_MAX || y > UINT32_MAX || z > UINT32_MAX || g.y > 65535 || g.z > 65535 ||
         (uint64_t)b.x * b.y * b.z > 1024)
         return fake::fail(hipErrorInvalidConfiguration);
-    fake::launches.push_back({fake::kernels()[f], g, b});
+    const std::string& name = fake::kernels()[f];
+    fake::launches.push_back({name, g, b, name.find("k_vcsr_find_long") != std::string::npos ? *(const int*)args[2] : 0});
     return hipSuccess;
 }
 }

@@ -94,6 +94,16 @@ static void narrow_batches() {
     CHECK(launched("k_spmm_streamIffLi1ELi8E"));
 }
 
+// Rows per thread of the VCSR listing kernel: 256 workgroups or more where the matrix has them.
+static void vcsr_listing() {
+    const struct { int rows, per; } want[] = {{1 << 18, 1}, {(1 << 18) + 1, 2}, {200000, 1}, {1 << 20, 4}, {1 << 23, 8}};
+    for (const auto& w : want) {
+        fake::reset();
+        CHECK(armsp_spmv_vcsr_f32(w.rows, 1 << 24, i32(), i32(), f32(), f32(), f32(), 0, nullptr) == ARMSP_SUCCESS);
+        CHECK(launched("k_vcsr_find_longILi" + std::to_string(w.per) + "E"));
+    }
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "no_memory"))
@@ -104,6 +114,8 @@ int main(int argc, char** argv) {
         transpose_workspace();
     else if (!std::strcmp(what, "narrow_batches"))
         narrow_batches();
+    else if (!std::strcmp(what, "vcsr_listing"))
+        vcsr_listing();
     else
         return 2;
     return fails ? 1 : 0;

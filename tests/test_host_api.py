@@ -26,7 +26,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["no_memory", "launch_limits", "transpose_workspace", "narrow_batches"])
+@pytest.mark.parametrize("check", ["no_memory", "launch_limits", "transpose_workspace", "narrow_batches",
+                                   "vcsr_listing"])
 def test_host_code(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=300)
     print(r.stdout, r.stderr[-2000:])
