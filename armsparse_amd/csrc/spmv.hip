@@ -304,7 +304,6 @@ __global__ __launch_bounds__(256) void k_spmv_vcsr(int M, const int* __restrict_
 // iteration of a medium row in flight); with 4 batches and 32 blocks ahead 91 VGPRs,
 // 5 waves, 286 us.  (345 us with a wave per medium row
 // and a staging wave that also added.)
-constexpr int VCSR_LONG_DEFAULT = 256;    // calls at 192, 256, 384: 322, 239, 242 us; 2048 rows, 60,000 nonzeros: 24, 25, 29
 constexpr int VCSR_MED_MIN = 16;          // rows of more blocks than this (and at most long_blocks) are medium
 constexpr int VCSR_MED_AHEAD = 4;         // steps of 4 blocks of an iteration of a medium row
 constexpr int VCSR_BATCH = 192;           // blocks per batch, one per lane of the staging waves
@@ -318,14 +317,19 @@ constexpr int VCSR_MED_WG_PER_CU = 16;
 constexpr int VCSR_LONG_WG_PER_CU = 2;
 
 // Rows longer than this many blocks take the workgroup-per-row path
-// (ARMSP_VCSR_LONG_BLOCKS overrides it, read once per process).
-int vcsr_long_blocks() {
+// (ARMSP_VCSR_LONG_BLOCKS overrides it, read once per process).  A medium row takes 16
+// lanes about 0.6 us per 16 blocks, so in a matrix of few blocks the longest of them is the
+// call's time, while a large one has more long rows than workgroups to take them (calls at
+// 64, 128, 256 blocks: 1024-row power-law graph of 36 nonzeros a row 15.1, 16.6, 21.3 us;
+// R-MAT of 20,000 rows of 30 33.1, 25.5, 30.0; 200,000 rows of 25 170, 98, 78; the 1M
+// R-MAT 680, 318, 228, and 229 at 384).
+int vcsr_long_blocks(int nnz_padded) {
     static const int v = [] {
         const char* e = getenv("ARMSP_VCSR_LONG_BLOCKS");
-        const int n = e ? atoi(e) : 0;
-        return n > 0 ? n : VCSR_LONG_DEFAULT;
+        return e ? std::max(atoi(e), 0) : 0;
     }();
-    return v;
+    const int blocks = nnz_padded / 4;
+    return v ? v : blocks <= 1 << 17 ? 64 : blocks <= 1 << 20 ? 128 : 256;
 }
 
 // Lists the long rows (more than long_blocks blocks) in list — those over 8 times the
@@ -820,7 +824,7 @@ int armsp_spmv_vcsr_f32(int M, int nnz_padded, const int* rowptr, const int* col
     // of 4 as well), so with unaligned operands every long row is a medium one.
     const bool aligned = ((uintptr_t)val % 16) == 0 && ((uintptr_t)x % 16) == 0;
     // (a long-row limit below VCSR_MED_MIN acts as VCSR_MED_MIN: rows up to it are the short walker's)
-    const int lb = vcsr_long_blocks();
+    const int lb = vcsr_long_blocks(nnz_padded);
     const int long_blocks = aligned ? (lb < VCSR_MED_MIN ? VCSR_MED_MIN : lb) : INT_MAX / 8;
     const bool split_long = nnz_padded / 4 > VCSR_MED_MIN;
     void* ws = nullptr;

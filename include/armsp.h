@@ -209,9 +209,10 @@ int armsp_spmv_f32(int M, int K, int nnz,
  * sparse_dense_vector (SpMV.cpp:155-179): per row four partial sums
  * s_l += val*x (unfused, or fused with ARMSP_FUSED_MLA) reduced as
  * (s0+s2)+(s1+s3), bit-exact with the reference's order.  Rows of up to 16
- * blocks get a 4-lane group each, rows of up to 256 blocks 16 lanes each, longer
- * rows (ARMSP_VCSR_LONG_BLOCKS in the environment moves the 256) a workgroup
- * each when val and x are 16-byte aligned, all in one launch; every walker
+ * blocks get a 4-lane group each, rows of up to 256 blocks (128 or 64 in
+ * matrices of up to 2^20 or 2^17 blocks) 16 lanes each, longer rows
+ * (ARMSP_VCSR_LONG_BLOCKS in the environment sets the limit) a workgroup each
+ * when val and x are 16-byte aligned, all in one launch; every walker
  * still adds each row's blocks in order, so the longest row's chain of adds
  * bounds the call.  ARMSP_VCSR_BALANCED runs
  * the merge-path SpMV over the same arrays instead (rows of any length spread

@@ -102,6 +102,14 @@ static void vcsr_listing() {
         CHECK(armsp_spmv_vcsr_f32(w.rows, 1 << 24, i32(), i32(), f32(), f32(), f32(), 0, nullptr) == ARMSP_SUCCESS);
         CHECK(launched("k_vcsr_find_longILi" + std::to_string(w.per) + "E"));
     }
+    // the limit from which a row is long: by the blocks of the matrix
+    const struct { int blocks, limit; } limits[] = {
+        {5000, 64}, {1 << 17, 64}, {(1 << 17) + 1, 128}, {1 << 20, 128}, {(1 << 20) + 1, 256}, {1 << 28, 256}};
+    for (const auto& w : limits) {
+        fake::reset();
+        CHECK(armsp_spmv_vcsr_f32(5000, 4 * w.blocks, i32(), i32(), f32(), f32(), f32(), 0, nullptr) == ARMSP_SUCCESS);
+        for (const auto& l : fake::launches) CHECK(l.kernel.find("find_long") == std::string::npos || l.arg2 == w.limit);
+    }
 }
 
 int main(int argc, char** argv) {
