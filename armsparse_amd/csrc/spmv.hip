@@ -436,6 +436,7 @@ __device__ void vcsr_medium_rows(uint32_t gg, uint32_t ngg, const int* __restric
     constexpr int IT = 4 * D;  // blocks of an iteration
     const int q = (threadIdx.x >> 2) & 3, l = threadIdx.x & 3;
     const uint32_t nmed = (uint32_t)__builtin_amdgcn_readfirstlane(count[2]);
+    if ((uint32_t)__builtin_amdgcn_readfirstlane((int)gg) >= nmed) return;  // none for this wave
     // row i of the list; past its end no blocks (row 0's index, so every load stays in bounds)
     auto row_at = [&](uint32_t i) { return i < nmed ? list_med[i] : 0; };
     auto blocks_of = [&](uint32_t i, int r, int b) { return i < nmed ? (rowptr[r + 1] - b) >> 2 : 0; };
@@ -540,6 +541,7 @@ __device__ void vcsr_long_rows(int M, const int* __restrict__ list, int* __restr
     const int t = (int)threadIdx.x - 64;  // staging lane of waves 1-3; wave 0 adds
     const int l = (int)threadIdx.x & 3;
     const int nfront = count[0], nlong = nfront + count[3];
+    if (nlong == 0) return;  // (512 workgroups' turns at the counter take microseconds)
     while (true) {
         if (threadIdx.x == 0) *s_row = atomicAdd(&count[1], 1);
         __syncthreads();
