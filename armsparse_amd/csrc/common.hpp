@@ -18,6 +18,10 @@ constexpr int64_t kMaxBlocks256 = (1 << 24) - 1;
 // -> 13.0 us a call, SpMV 14.9 -> 11.8), and above it the searches cost more than the
 // streaming pass (SpMV of 4M nonzeros with 8,192 chunks: 31.1 -> 32.9 us).
 constexpr int64_t kSearchWaves = 4096;
+// Where every column slice or tile walks the chunks, it searches them again: so many searches
+// (fp32 SpMM, searched against a partition: 687 chunks x 8 slices 16.9 and 17.9 us, 1718 x 4
+// 18.8 and 19.4, 3437 x 4 28.0 and 27.9, 1718 x 8 31.8 and 31.2, 3437 x 16 94.1 and 84.5).
+constexpr int64_t kSearches = 2 * kSearchWaves;
 
 // ------------------------------------------------------------------ runtime
 // Records the HIP error for armsp_last_hip_error() and maps it to a status.
@@ -204,7 +208,7 @@ __device__ __forceinline__ int partition_at(const int* __restrict__ part, int w,
 // from d1 - nnz on, so that here too a malformed rowptr ends the chunk by nonzero nnz.
 __device__ __forceinline__ void chunk_rows(const int* __restrict__ part, int wave, int d0, int d1,
                                            const int* __restrict__ rowptr, int M, int nnz, int& i0, int& i1) {
-    if (part) {
+    if (__builtin_expect(part != nullptr, 1)) {  // the search placed out of the way
         i0 = uniform(partition_at(part, wave, d0, M, nnz));
         i1 = uniform(partition_at(part, wave + 1, d1, M, nnz));
         return;

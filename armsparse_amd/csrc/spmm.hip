@@ -1371,6 +1371,26 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     const unsigned tiles = (unsigned)((N + 64 * V - 1) / (64 * V));
     if (tiles > 65535) return ARMSP_ERROR_NOT_SUPPORTED;
 
+    // group 32: half a wave per nonzero over column slices of B (k_spmm_slice), each lane
+    // 4 bytes of B (vec 0) or vec columns of 4, 8 or 16 bytes.
+    // AUTO (group 0): when a row of B spans two or more 256-byte slices, half a wave per
+    // nonzero with 8-byte lanes, the slices spread over the XCDs — on power-law matrices
+    // each XCD's L2 then holds half (or less) of every hot row (measured: 18–25% faster
+    // on the 1M R-MAT at N=128/256 fp32, 8% at N=256 bf16, within 6% elsewhere)
+    // bf16 rows of 128-511 bytes: half-wave slices with 4-byte lanes (1M R-MAT: N = 128
+    // 637 -> 574 us, N = 64 336 -> 315 us)
+    const int alb = N * esz >= 512 ? 8 : 4;  // AUTO's lane bytes
+    const int asv = alb / esz;
+    const bool auto_slice = merge && !wide && !narrow && c.group == 0 && chunk <= 2048 && slice_rows &&
+                            N % asv == 0 && ldb % asv == 0 && ldc % asv == 0 && aligned(B, alb) &&
+                            aligned(C, (int)sizeof(TC) * asv);
+    const int SV = auto_slice ? asv : (c.vec > 0 ? c.vec : 4 / esz);
+    const int slb = SV * esz;
+    const bool slice = auto_slice ||
+                       (merge && !wide && c.group == 32 && chunk <= 2048 && (slb == 4 || slb == 8 || slb == 16) &&
+                        N % SV == 0 && ldb % SV == 0 && ldc % SV == 0 && aligned(B, slb) && aligned(C, (int)sizeof(TC) * SV));
+    if (c.group == 32 && !slice) return ARMSP_ERROR_NOT_SUPPORTED;
+
     // the LDS-staged merge kernels (stream, slice, narrow) start from a precomputed
     // merge-path partition, nwaves + 1 row boundaries, when they have many chunks
     const bool staged = merge && !wide && chunk <= 2048;
@@ -1378,7 +1398,8 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     const size_t row_bytes = ((size_t)nwaves * sizeof(int) + 255) & ~(size_t)255;
     const size_t val_bytes = ((size_t)nwaves * N * sizeof(float) + 255) & ~(size_t)255;
     const size_t head_bytes = out16 ? val_bytes : 0;  // the last parts of cut rows, fp32
-    const bool presearch = staged && nwaves > kSearchWaves;
+    const int passes = slice ? (N + 32 * SV - 1) / (32 * SV) : narrow ? 1 : (int)tiles;
+    const bool presearch = staged && (nwaves > kSearchWaves || nwaves * passes > kSearches);
     const size_t part_bytes = presearch ? (size_t)(nwaves + 1) * sizeof(int) : 0;
     int st;
     if (scratch) {  // no allocation: the caller's region, or a clear refusal
@@ -1409,28 +1430,6 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
         t.stop();
     }
 
-    // group 32: half a wave per nonzero over column slices of B (k_spmm_slice), each lane
-    // 4 bytes of B (vec 0) or vec columns of 4, 8 or 16 bytes.
-    // AUTO (group 0): when a row of B spans two or more 256-byte slices, half a wave per
-    // nonzero with 8-byte lanes, the slices spread over the XCDs — on power-law matrices
-    // each XCD's L2 then holds half (or less) of every hot row (measured: 18–25% faster
-    // on the 1M R-MAT at N=128/256 fp32, 8% at N=256 bf16, within 6% elsewhere)
-    // bf16 rows of 128-511 bytes: half-wave slices with 4-byte lanes (1M R-MAT: N = 128
-    // 637 -> 574 us, N = 64 336 -> 315 us)
-    const int alb = N * esz >= 512 ? 8 : 4;  // AUTO's lane bytes
-    const int asv = alb / esz;
-    const bool auto_slice = merge && !wide && !narrow && c.group == 0 && chunk <= 2048 && slice_rows &&
-                            N % asv == 0 && ldb % asv == 0 && ldc % asv == 0 && aligned(B, alb) &&
-                            aligned(C, (int)sizeof(TC) * asv);
-    const int SV = auto_slice ? asv : (c.vec > 0 ? c.vec : 4 / esz);
-    const int slb = SV * esz;
-    const bool slice = auto_slice ||
-                       (merge && !wide && c.group == 32 && chunk <= 2048 && (slb == 4 || slb == 8 || slb == 16) &&
-                        N % SV == 0 && ldb % SV == 0 && ldc % SV == 0 && aligned(B, slb) && aligned(C, (int)sizeof(TC) * SV));
-    if (c.group == 32 && !slice) {
-        release(ws, s);
-        return ARMSP_ERROR_NOT_SUPPORTED;
-    }
     dim3 grid((unsigned)((nwaves + 3) / 4), tiles);
     if (narrow && !out16) {
         TimedLaunch t("spmm", s);

@@ -112,6 +112,22 @@ static void vcsr_listing() {
     }
 }
 
+// A partition where the waves' searches, one per chunk and column slice, would be many.
+static void partitions() {
+    auto spmm = [&](int M, int nnz, int N) {
+        fake::reset();
+        float* p = reinterpret_cast<float*>(1ull << 34);  // on a 128-byte line, as slices need
+        CHECK(armsp_spmm_f32(M, M, N, nnz, i32(), i32(), f32(), p, N, p, N, 0, nullptr, nullptr) == ARMSP_SUCCESS);
+        CHECK(launched("k_spmm_slice"));
+        return launched("k_merge_partition");
+    };
+    CHECK(!spmm(4000, 40000, 512));   // 688 chunks of 64, 8 slices
+    CHECK(!spmm(10000, 100000, 256));  // 1719 and 4
+    CHECK(spmm(10000, 100000, 512));   // 1719 and 8
+    CHECK(spmm(20000, 200000, 512));
+    CHECK(spmm(100000, 1000000, 256));
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "no_memory"))
@@ -124,6 +140,8 @@ int main(int argc, char** argv) {
         narrow_batches();
     else if (!std::strcmp(what, "vcsr_listing"))
         vcsr_listing();
+    else if (!std::strcmp(what, "partitions"))
+        partitions();
     else
         return 2;
     return fails ? 1 : 0;
