@@ -15,7 +15,8 @@
 //  short rows — a group of G lanes per row, V columns per lane, U gathers of the
 //          row in flight;
 //  long rows — waves that each take a fixed range of nonzeros and fold what it holds
-//          of the long rows; k_max_join folds the parts of a cut row in order.
+//          of the long rows; k_max_join folds the parts of a cut row in order.  In small
+//          inputs a workgroup per long row instead, which needs no second launch.
 // A hub row walked by one group bounds the call, whatever else runs: a 131,072-row
 // R-MAT with 2^21 nonzeros at N = 64 took 2551 us, 74 + 5 now; matrices without
 // long rows keep the group per row (1.5M nonzeros, uniform: 65 us, 64 + 4 now), and the
@@ -58,6 +59,13 @@ inline int max_long_row(int M, int nnz) {
     return twice_mean > 32 ? (int)twice_mean : 32;
 }
 
+// Nonzeros times lanes per group up to which a workgroup takes each long row, without parts
+// in memory and without the second launch, which is 3 of 14 us where no row is long (uniform,
+// 1024 rows of 8 to 4096 of 8, N = 4 to 64: 10.5 us, 13.7 to 14.3 with it; a power-law graph
+// of 1024 rows of 8 10.7 and 14.0).  Beyond, a hub row keeps its workgroup's four waves busy
+// for longer than the launch takes (R-MAT of 8192 rows of 10, N = 64: 18.2 and 15.0).
+constexpr int64_t kMaxJoin = 1 << 19;
+
 // A row cut by the waves' ranges is a sequence of parts.  The part that holds the
 // row's start folds from `init`, the others from -inf with no position, so every part
 // of the others names one.  Joining two parts in order, the later wins unless the
@@ -66,6 +74,12 @@ inline int max_long_row(int M, int nnz) {
 // before: its position is stored with the top bit set.
 constexpr uint32_t kNoPos = 0xffffffffu;
 constexpr uint32_t kSawNan = 0x80000000u;
+__device__ __forceinline__ void max_join(float& acc, uint32_t& arg, float x, uint32_t p) {
+    if (p == kNoPos) return;  // no entries in the later part
+    const bool keep = !(p & kSawNan) && acc > x;
+    acc = keep ? acc : x;
+    arg = keep ? arg : p | (arg != kNoPos ? arg & kSawNan : 0u);
+}
 
 // Where the long-row walker leaves its parts: per wave the part of a row that goes on
 // past its range (of row carry_row[wave], else -1) and the part of a row that began
@@ -171,6 +185,111 @@ __device__ __forceinline__ void max_long_rows(int wave, int j0, int j1, int tile
     if (tile0 == 0 && lane == 0) parts.carry_row[wave] = carry;
 }
 
+// The long rows that begin among the nonzeros [j0, j1), a workgroup of four waves per row:
+// every group of G lanes folds a part of the row, the parts are joined in order, within
+// the waves by shuffles and across them in LDS.  Columns as in max_short_rows.
+template <int V, int G>
+__device__ __forceinline__ void max_group_rows(int j0, int j1, int tile, int M, int N, int long_row,
+                                               const int* __restrict__ rowptr, const int* __restrict__ colind,
+                                               const float* __restrict__ val, const float* __restrict__ B, int ldb,
+                                               float init, float* __restrict__ C, int ldc, int* __restrict__ argmax) {
+    constexpr int U = V == 1 ? 8 : 4, S = 64 / G, P = 4 * S;
+    __shared__ float s_acc[4][G * V];
+    __shared__ uint32_t s_arg[4][G * V];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l = lane & (G - 1), part = w * S + lane / G;
+    const int col = (tile * G + l) * V;
+    const bool active = col < N;
+    const float* bp = B + (active ? col : 0);
+    int idle = 0;  // windows of 64 rows in a row that held no entry, as in max_long_rows
+    for (int rb = uniform(rows_ending_by_wave(j0, rowptr, M)); rb < M;) {
+        const int rl = rb + lane;
+        const int sl = rl < M ? rowptr[rl] : INT_MAX, el = rl < M ? rowptr[rl + 1] : INT_MAX;
+        // the same for the four waves, so they meet at the same barriers
+        uint64_t longs = __ballot(rl < M && el - sl > long_row && sl >= j0 && sl < j1);
+        for (; longs; longs &= longs - 1) {
+            const int k = __builtin_ctzll(longs);
+            const int r = rb + k, s = read_lane(sl, k), e = read_lane(el, k);
+            const int p0 = s + (int)((int64_t)(e - s) * part / P), p1 = s + (int)((int64_t)(e - s) * (part + 1) / P);
+            float acc[V];
+            uint32_t arg[V];
+            bool nan[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                acc[v] = -__builtin_inff();
+                arg[v] = kNoPos;
+                nan[v] = false;
+            }
+            for (int base = p0; base < p1; base += G) {
+                const int n = min(G, p1 - base);
+                int c = 0;
+                float a = 0.0f;
+                if (l < n) {
+                    c = colind[base + l];
+                    a = val ? val[base + l] : 1.0f;
+                }
+                for (int i = 0; i < n; i += U) {
+                    float b[U][V], f[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {  // past n: again the last entry, not folded
+                        const int q = min(i + u, n - 1);
+                        f[u] = __shfl(a, q, G);
+                        load_v<V>(bp + (size_t)__shfl(c, q, G) * ldb, b[u]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (i + u < n) {
+#pragma unroll
+                            for (int v = 0; v < V; ++v) {
+                                const float x = f[u] * b[u][v];
+                                const bool keep = acc[v] > x;
+                                acc[v] = keep ? acc[v] : x;
+                                arg[v] = keep ? arg[v] : (uint32_t)(base + i + u);
+                                nan[v] |= x != x;
+                            }
+                        }
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                uint32_t g = arg[v] == kNoPos ? kNoPos : arg[v] | (nan[v] ? kSawNan : 0u);
+#pragma unroll
+                for (int d = 1; d < S; d <<= 1) {  // (lanes past the wave's end give what no one takes)
+                    const float x = __shfl_down(acc[v], d * G);
+                    const uint32_t q = __shfl_down(g, d * G);
+                    max_join(acc[v], g, x, q);
+                }
+                if (lane < G) {
+                    s_acc[w][l * V + v] = acc[v];
+                    s_arg[w][l * V + v] = g;
+                }
+            }
+            __syncthreads();
+            if (w == 0 && lane < G && active) {
+                float o[V];
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    float acc0 = init;
+                    uint32_t g = kNoPos;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) max_join(acc0, g, s_acc[q][l * V + v], s_arg[q][l * V + v]);
+                    o[v] = acc0;
+                    if (argmax) argmax[(size_t)r * N + col + v] = g == kNoPos ? -1 : (int)(g & ~kSawNan);
+                }
+                store_v<V>(C + (size_t)r * ldc + col, o);
+            }
+            __syncthreads();  // the parts are read before the next row's are written
+        }
+        const int e63 = read_lane(el, 63);
+        if (e63 >= j1) break;
+        idle = e63 == read_lane(sl, 0) ? idle + 1 : 0;
+        rb += 64;
+        if (idle == 4) {
+            rb = max(rb, uniform(rows_ending_by_wave(e63, rowptr, M)));
+            idle = 0;
+        }
+    }
+}
+
 // Rows of at most long_row nonzeros, a group of G lanes each.
 template <int V, int G>
 __device__ __forceinline__ void max_short_rows(int blk, int tile, int M, int N, int long_row,
@@ -230,27 +349,35 @@ __device__ __forceinline__ void max_short_rows(int blk, int tile, int M, int N, 
     }
 }
 
-// Workgroups [0, nlong · column tiles) walk the long rows, `chunk` nonzeros a wave
-// (first: they take longest); the rest the short rows.  The long walker's lanes hold
-// the columns a group of the short one covers in a quarter, a half or all of a wave.
+// Workgroups [0, nlong · column tiles) walk the long rows (first: they take longest), the
+// rest the short rows.  JOIN: `chunk` nonzeros a wave, whose parts k_max_join
+// joins; the lanes hold the columns a group of the short walker covers in a quarter, a
+// half or all of a wave.  Otherwise the rows that begin in `chunk` nonzeros a workgroup.
 // (Column slices spread over the XCDs, as in the SpMM, do not pay: 78 -> 84 us on the
 // R-MAT, 68 -> 70 us on the uniform matrix.)
 // `first`: the launch's first workgroup, where they are more than one launch holds.
-template <int V, int G>
+template <int V, int G, bool JOIN>
 __global__ __launch_bounds__(256) void k_spmm_max(int first, int M, int N, int nnz, int nlong, int chunk, int nshort,
-                                                  int long_row, const int* __restrict__ rowptr, const int* __restrict__ colind,
-                                                  const float* __restrict__ val, const float* __restrict__ B,
-                                                  int ldb, float init, float* __restrict__ C, int ldc,
-                                                  int* __restrict__ argmax, MaxParts parts) {
+                                                  int long_row, const int* __restrict__ rowptr,
+                                                  const int* __restrict__ colind, const float* __restrict__ val,
+                                                  const float* __restrict__ B, int ldb, float init,
+                                                  float* __restrict__ C, int ldc, int* __restrict__ argmax,
+                                                  MaxParts parts) {
     constexpr int VL = V == 4 && G == 64 ? 4 : V == 4 && G == 32 ? 2 : 1;
-    const int ltiles = nlong ? (N + 64 * VL - 1) / (64 * VL) : 0;
+    constexpr int tile = JOIN ? 64 * VL : G * V;
+    const int ltiles = nlong ? (N + tile - 1) / tile : 0;
     const int b = first + (int)blockIdx.x;
     if (b < nlong * ltiles) {
-        const int wave = uniform((b / ltiles) * 4 + (int)(threadIdx.x >> 6));
-        const int64_t j0 = (int64_t)wave * chunk;
-        if (j0 < nnz)
-            max_long_rows<VL>(wave, (int)j0, (int)min(j0 + chunk, (int64_t)nnz), (b % ltiles) * 64 * VL, M, N, long_row,
-                              rowptr, colind, val, B, ldb, init, C, ldc, argmax, parts);
+        const int range = JOIN ? uniform((b / ltiles) * 4 + (int)(threadIdx.x >> 6)) : b / ltiles;
+        const int64_t j0 = (int64_t)range * chunk;
+        if (j0 >= nnz) return;
+        const int j1 = (int)min(j0 + chunk, (int64_t)nnz);
+        if constexpr (JOIN)
+            max_long_rows<VL>(range, (int)j0, j1, (b % ltiles) * 64 * VL, M, N, long_row, rowptr, colind, val, B, ldb,
+                              init, C, ldc, argmax, parts);
+        else
+            max_group_rows<V, G>((int)j0, j1, b % ltiles, M, N, long_row, rowptr, colind, val, B, ldb, init, C, ldc,
+                                 argmax);
         return;
     }
     const int rb = b - nlong * ltiles;
@@ -392,14 +519,18 @@ __global__ __launch_bounds__(kBwdThreads) void k_spmm_max_backward(int64_t total
 }
 
 template <int V>
-int launch_max(int G, int first, unsigned grid, hipStream_t s, int M, int N, int nnz, int nlong, int chunk, int nshort,
-               int long_row, const int* rp, const int* ci, const float* va, const float* B, int ldb, float init,
+int launch_max(int G, int first, unsigned grid, hipStream_t s, int M, int N, int nnz, int nlong, int chunk, bool join,
+               int nshort, int long_row, const int* rp, const int* ci, const float* va, const float* B, int ldb, float init,
                float* C, int ldc, int* arg, const MaxParts& parts) {
     switch (G) {
 #define ARMSP_MAX_CASE(GG)                                                                                          \
     case GG:                                                                                                        \
-        hipLaunchKernelGGL((k_spmm_max<V, GG>), dim3(grid), dim3(256), 0, s, first, M, N, nnz, nlong, chunk, nshort, \
-                           long_row, rp, ci, va, B, ldb, init, C, ldc, arg, parts);                                 \
+        if (join)                                                                                                   \
+            hipLaunchKernelGGL((k_spmm_max<V, GG, true>), dim3(grid), dim3(256), 0, s, first, M, N, nnz, nlong, chunk, \
+                               nshort, long_row, rp, ci, va, B, ldb, init, C, ldc, arg, parts);                     \
+        else                                                                                                        \
+            hipLaunchKernelGGL((k_spmm_max<V, GG, false>), dim3(grid), dim3(256), 0, s, first, M, N, nnz, nlong, chunk, \
+                               nshort, long_row, rp, ci, va, B, ldb, init, C, ldc, arg, parts);                     \
         break;
         ARMSP_MAX_CASE(4)
         ARMSP_MAX_CASE(8)
@@ -430,36 +561,38 @@ extern "C" int armsp_spmm_max_f32(int M, int K, int N, int nnz, const int* rowpt
     int G = 4;
     while (G < 64 && G * V < N) G <<= 1;
     const int64_t nshort = ((int64_t)M * G + 255) / 256, stiles = (N + G * V - 1) / (G * V);
-    if (stiles > 65535) return ARMSP_ERROR_NOT_SUPPORTED;
-    // the long rows' waves: 512 nonzeros each, fewer until 16 waves per CU are in flight
-    int chunk = 512;
+    if (stiles > 65535 || nshort * stiles > INT_MAX) return ARMSP_ERROR_NOT_SUPPORTED;
+    const int long_row = max_long_row(M, nnz);
+    // small inputs: a workgroup per long row, 64 nonzeros' rows each.  Else the long rows'
+    // waves: 512 nonzeros each, fewer until 16 waves per CU are in flight
+    const bool join = (int64_t)nnz * G > kMaxJoin;
+    int chunk = join ? 512 : 64;
     while (chunk > 64 && nnz / chunk < 16 * device_cus()) chunk >>= 1;
     const int64_t nwaves = ((int64_t)nnz + chunk - 1) / chunk;
     const int VL = V == 4 && G == 64 ? 4 : V == 4 && G == 32 ? 2 : 1;
-    const int64_t ltiles = (N + 64 * VL - 1) / (64 * VL);
-    const int long_row = max_long_row(M, nnz);
-    int64_t nlong = nnz > long_row ? (nwaves + 3) / 4 : 0;
+    const int64_t ltiles = join ? (N + 64 * VL - 1) / (64 * VL) : stiles;
+    int64_t nlong = nnz <= long_row ? 0 : join ? (nwaves + 3) / 4 : nwaves;
     const size_t i4 = ((size_t)nwaves * 4 + 255) & ~(size_t)255;
     const size_t v4 = ((size_t)nwaves * 2 * N * 4 + 255) & ~(size_t)255;
     void* ws = nullptr;
     // (without workspace, as under capture with no arena reserved, every row is a short one)
-    if (nlong * ltiles + nshort * stiles > INT_MAX || (nlong && ws_alloc(&ws, i4 + 2 * v4, s) != ARMSP_SUCCESS))
+    if (nlong * ltiles + nshort * stiles > INT_MAX ||
+        (nlong && join && ws_alloc(&ws, i4 + 2 * v4, s) != ARMSP_SUCCESS))
         nlong = 0;
     char* w = static_cast<char*>(ws);
     const MaxParts parts{reinterpret_cast<int*>(w), reinterpret_cast<float*>(w + i4),
                          reinterpret_cast<uint32_t*>(w + i4 + v4)};
-    if (nshort * stiles > INT_MAX) return ARMSP_ERROR_NOT_SUPPORTED;
     const int64_t blocks = nlong * ltiles + nshort * stiles;
     TimedLaunch t("spmm_max", s);
     int st = ARMSP_SUCCESS;
     for (int64_t first = 0; first < blocks && !st; first += kMaxBlocks256) {
         const unsigned grid = (unsigned)std::min(blocks - first, kMaxBlocks256);
-        st = V == 4 ? launch_max<4>(G, (int)first, grid, s, M, N, nnz, (int)nlong, chunk, (int)nshort, long_row, rowptr,
-                                    colind, val, B, ldb, init, C, ldc, argmax, parts)
-                    : launch_max<1>(G, (int)first, grid, s, M, N, nnz, (int)nlong, chunk, (int)nshort, long_row, rowptr,
-                                    colind, val, B, ldb, init, C, ldc, argmax, parts);
+        st = V == 4 ? launch_max<4>(G, (int)first, grid, s, M, N, nnz, (int)nlong, chunk, join, (int)nshort, long_row,
+                                    rowptr, colind, val, B, ldb, init, C, ldc, argmax, parts)
+                    : launch_max<1>(G, (int)first, grid, s, M, N, nnz, (int)nlong, chunk, join, (int)nshort, long_row,
+                                    rowptr, colind, val, B, ldb, init, C, ldc, argmax, parts);
     }
-    if (!st && nlong)
+    if (!st && nlong && join)
         hipLaunchKernelGGL(k_max_join, dim3((unsigned)((nwaves + 3) / 4)), dim3(256), 0, s, (int)nwaves, N, parts, C,
                            ldc, argmax);
     const hipError_t e = hipGetLastError();

@@ -22,7 +22,7 @@ static int* i32() { return reinterpret_cast<int*>(1ull << 33); }
 static void no_memory() {
     fake::reset();
     fake::memory = 0;
-    CHECK(armsp_spmm_max_f32(1000, 1000, 64, 100000, i32(), i32(), f32(), f32(), 64, -1e4f, f32(), 64, i32(), nullptr) ==
+    CHECK(armsp_spmm_max_f32(1000, 1000, 64, 2000000, i32(), i32(), f32(), f32(), 64, -1e4f, f32(), 64, i32(), nullptr) ==
           ARMSP_SUCCESS);
     CHECK(fake::asked.size() == 1 && fake::launches.size() == 1);  // it asked, and ran without
 
@@ -128,6 +128,19 @@ static void partitions() {
     CHECK(spmm(100000, 1000000, 256));
 }
 
+// Max aggregation of a small input is one launch and asks for no workspace.
+static void max_launches() {
+    for (int n : {4, 64}) {
+        fake::reset();
+        CHECK(armsp_spmm_max_f32(1024, 1024, n, 30000, i32(), i32(), nullptr, f32(), n, -1e4f, f32(), n, i32(), nullptr) ==
+              ARMSP_SUCCESS);
+        CHECK(fake::launches.size() == 1 && fake::asked.empty());
+    }
+    CHECK(armsp_spmm_max_f32(20000, 20000, 64, 600000, i32(), i32(), nullptr, f32(), 64, -1e4f, f32(), 64, i32(),
+                             nullptr) == ARMSP_SUCCESS);
+    CHECK(launched("k_max_join"));
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!std::strcmp(what, "no_memory"))
@@ -142,6 +155,8 @@ int main(int argc, char** argv) {
         vcsr_listing();
     else if (!std::strcmp(what, "partitions"))
         partitions();
+    else if (!std::strcmp(what, "max_launches"))
+        max_launches();
     else
         return 2;
     return fails ? 1 : 0;

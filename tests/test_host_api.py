@@ -27,7 +27,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["no_memory", "launch_limits", "transpose_workspace", "narrow_batches",
-                                   "vcsr_listing", "partitions"])
+                                   "vcsr_listing", "partitions", "max_launches"])
 def test_host_code(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=300)
     print(r.stdout, r.stderr[-2000:])
