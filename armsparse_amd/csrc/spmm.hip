@@ -1334,12 +1334,12 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
     // half-wave slices, and a whole wave per nonzero on narrow rows of B (N < 32), run
     // best with 256 items per wave; slices with 4 gathers per batch, narrow rows with 8
     // (a 825,000-row R-MAT of 12.5M nonzeros, bf16 N = 8: 240 us with 4, 190 with 8; seven
-    // uniform and R-MAT matrices, N = 5 to 31: 1 to 24% less time), but for fp8, and fp32 of
-    // 24 columns and more, on rows of under 8 nonzeros, which end inside most batches
-    // (uniform 141,670 rows of 6: fp8 N = 16 30.8 us with 4, 35.5 with 8; fp32 N = 24 32.2, 33.2)
+    // uniform and R-MAT matrices, N = 5 to 31: up to 24% less time, R-MATs of 1 to 2M up to 5%
+    // more), but for fp32 of 24 columns and more on rows of under 8 nonzeros, which end
+    // inside most batches (uniform 141,670 rows of 6, N = 24 32.2 us with 4, 33.2 with 8)
     if (merge && !wide && !narrow && c.group == 0 && (slice_rows || N < 32)) {
         if (c.chunk <= 0) chunk = 256;
-        const bool short_rows = nnz < 8 * (int64_t)M && (esz == 1 || (esz == 4 && N >= 24));
+        const bool short_rows = nnz < 8 * (int64_t)M && esz == 4 && N >= 24;
         if (c.unroll <= 0) U = slice_rows || short_rows ? 4 : 8;
     }
     if (narrow) {  // default: runs of 8 items for N ≤ 2, of 4 above (the staged products fill the LDS)
@@ -1353,6 +1353,12 @@ int spmm_impl(int M, int K, int N, int nnz, const int* rowptr, const int* colind
         const int64_t want = 16 * (int64_t)device_cus();
         while (chunk > 64 && (total + chunk - 1) / chunk < want) chunk >>= 1;
         if (chunk == 64 && N < 32 && c.unroll <= 0) U = 4;
+        // (fp8 with 8 leaves 24 waves on a CU, with 4 it leaves 32: where all waves are on the
+        // device at once only with 4; uniform 141,670 rows of 6, N = 16: 30.8 us with 4, 35.5
+        // with 8; R-MAT of 50,574 rows of 19 30.3 and 34.2; 60,000 rows of 20 42.6 and 43.1)
+        const int64_t waves = (total + chunk - 1) / chunk;
+        if (esz == 1 && N < 32 && c.unroll <= 0 && waves > 24 * (int64_t)device_cus() && waves <= 32 * (int64_t)device_cus())
+            U = 4;
         // fp32 rows of more than 64 columns and under 24 nonzeros a row on average: 256 items
         // and 4 gathers per batch, which leave more waves on a CU, where 512 are to be had
         // (R-MAT of 150,000 rows, 2M nonzeros, N = 100: 121 -> 98 us; uniform matrices the

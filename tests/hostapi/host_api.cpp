@@ -68,9 +68,9 @@ static bool launched(const std::string& part) {
 }
 
 // Gathers per batch (the last template argument) of an automatic product on rows of B under
-// 32 columns, by type, width and the nonzeros a row holds.
+// 32 columns, by type, width, the waves and the nonzeros a row holds.
 static void narrow_batches() {
-    const int M = 141670, nnz = 870517;  // 6 a row
+    int M = 141670, nnz = 870517;  // 6 a row, 7908 waves
     const uint8_t* q = reinterpret_cast<const uint8_t*>(f32());
     auto fp8 = [&](int nz, int n) {
         fake::reset();
@@ -85,6 +85,13 @@ static void narrow_batches() {
         CHECK(launched("k_spmm_streamIhfLi1ELi4E"));
         fp8(4 * nnz, n);
         CHECK(launched("k_spmm_streamIhfLi1ELi8E"));
+        M = 50574;
+        fp8(975971, n);  // 8021 waves
+        CHECK(launched("k_spmm_streamIhfLi1ELi4E"));
+        M = 20000;
+        fp8(700000, n);  // 5625
+        CHECK(launched("k_spmm_streamIhfLi1ELi8E"));
+        M = 141670;
     }
     fp32(nnz, 16);
     CHECK(launched("k_spmm_streamIffLi1ELi8E"));
