@@ -597,9 +597,12 @@ def to_bf16_colsum(x: torch.Tensor) -> tuple:
     _require(x.is_cuda and x.dtype == torch.float32 and x.is_contiguous(), "to_bf16_colsum: needs a contiguous 2-D "
              "float32 device tensor")
     y = empty_rows(m, n, torch.bfloat16, x.device)
-    out = torch.empty(n, device=x.device)
-    call("armsp_convert_rows_colsum_bf16", m, n, _ptr(x), x.stride(0), _ptr(y), y.stride(0), _ptr(out),
-         _stream(x.device))
+    out = torch.empty(n, dtype=torch.float32, device=x.device)
+    st = _lib.lib.armsp_convert_rows_colsum_bf16(m, n, _ptr(x), x.stride(0), _ptr(y), y.stride(0), _ptr(out),
+                                                 _stream(x.device))
+    if st == _lib.ERROR_ALLOC:  # (no workspace, as under capture without an arena: two passes need less or none)
+        return to_bf16(x, pitched=True), colsum(x)
+    _lib.check("armsp_convert_rows_colsum_bf16", st)
     return y, out
 
 
