@@ -413,7 +413,7 @@ def spmm_datareuse(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[
     d = dense.contiguous()
     if out is None:
         _require(not accumulate, f"{fn}: accumulate needs an output tensor")
-        out = torch.empty((m, n), device=dense.device)
+        out = torch.empty((m, n), dtype=torch.float32, device=dense.device)
     _require(out.shape == (m, n) and out.is_contiguous(), f"{fn}: out must be a contiguous [M, N] tensor")
     call("armsp_spmm_datareuse_f32", m, k, n, nnz, _ptr(rowptr), _ptr(colind), _ptr(values), _ptr(flag), _ptr(d), n,
          _ptr(out), n, _lib.ACCUMULATE if accumulate else 0, _stream(dense.device))
@@ -435,7 +435,7 @@ def spmm_max(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.
     m, nnz = rowptr.numel() - 1, colind.numel()
     k, n = dense.shape
     d = dense.contiguous()
-    out = torch.empty((m, n), device=dense.device)
+    out = torch.empty((m, n), dtype=torch.float32, device=dense.device)
     arg = torch.empty((m, n), dtype=torch.int32, device=dense.device) if return_argmax else None
     call("armsp_spmm_max_f32", m, k, n, nnz, _ptr(rowptr), _ptr(colind), _ptr(values), _ptr(d), n, float(init),
          _ptr(out), n, _ptr(arg), _stream(dense.device))
@@ -449,7 +449,7 @@ def spmm_max_backward(colind: torch.Tensor, values: Optional[torch.Tensor], grad
     _require(argmax.shape == grad_out.shape and argmax.dtype == torch.int32, f"{fn}: argmax must match grad_out")
     m, n = grad_out.shape
     g = grad_out.contiguous().float()
-    db = torch.zeros((num_src, n), device=grad_out.device)
+    db = torch.zeros((num_src, n), dtype=torch.float32, device=grad_out.device)
     call("armsp_spmm_max_backward_f32", m, num_src, n, colind.numel(), _ptr(colind), _ptr(values), _ptr(g), n,
          _ptr(argmax.contiguous()), _ptr(db), n, _stream(grad_out.device))
     return db
@@ -541,7 +541,7 @@ def bias_relu_dropout_backward(g: torch.Tensor, mask: torch.Tensor, p: float, wa
     m, n = g.shape
     _require(mask.dtype == torch.uint8 and mask.shape == (m, n // 8) and mask.is_contiguous(), f"{fn}: bad mask")
     gy = empty_rows(m, n, torch.bfloat16, g.device) if pitched else torch.empty_like(g)
-    dbias = torch.empty(n, device=g.device) if want_dbias else None
+    dbias = torch.empty(n, dtype=torch.float32, device=g.device) if want_dbias else None
     call("armsp_bias_relu_dropout_backward_bf16", m, n, _ptr(g), _ptr(mask), float(p), _ptr(gy), gy.stride(0),
          _ptr(dbias), _stream(g.device))
     return gy, dbias
@@ -551,7 +551,7 @@ def colsum(x: torch.Tensor) -> torch.Tensor:
     """x.sum(0) for a 2-D float32 device tensor, deterministic (armsp_colsum_f32)."""
     _require(x.is_cuda and x.dtype == torch.float32 and x.dim() == 2, "colsum: needs a 2-D float32 device tensor")
     x = x.contiguous()
-    out = torch.empty(x.shape[1], device=x.device)
+    out = torch.empty(x.shape[1], dtype=torch.float32, device=x.device)
     call("armsp_colsum_f32", x.shape[0], x.shape[1], _ptr(x), _ptr(out), _stream(x.device))
     return out
 
