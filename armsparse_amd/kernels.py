@@ -126,7 +126,8 @@ def spmm(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tens
     rp, ci, va, d = _all_on_device(dev, rowptr, colind, values, dense)
     if out is None:
         _require(not accumulate, "spmm: accumulate needs an output tensor")
-        c = d.new_empty((m, n)) if d.dtype is torch.float32 else torch.empty((m, n), dtype=torch.float32, device=dev)
+        c = d.new_empty((m, n)) if d.dtype is torch.float32 and type(d) is torch.Tensor else \
+            torch.empty((m, n), dtype=torch.float32, device=dev)
     else:
         _require(out.shape == (m, n) and out.dtype == torch.float32, f"{fn}: out must be float32 [M, N]")
         _require(out.stride(1) == 1, f"{fn}: out rows must be contiguous")
@@ -216,7 +217,7 @@ def spmv(rowptr: torch.Tensor, colind: torch.Tensor, values: Optional[torch.Tens
     rp, ci, va, xd = _all_on_device(dev, rowptr, colind, values, x)
     if out is None:
         _require(not accumulate, "spmv: accumulate needs an output tensor")
-        y = xd.new_empty((m,))
+        y = xd.new_empty((m,)) if type(xd) is torch.Tensor else torch.empty(m, dtype=torch.float32, device=dev)
     else:
         _require(out.shape == (m,) and out.dtype == torch.float32 and out.is_contiguous(), f"{fn}: bad out")
         y = _on_device(out, dev)
