@@ -19,9 +19,19 @@
 namespace armsp {
 namespace {
 
-constexpr int kTN = 2048;  // columns per wave tile (8 KiB of LDS per wave: 20 waves a CU)
+// Columns per wave tile: 2048 (8 KiB of LDS per wave: 20 waves a CU) or 4096 (10 waves).
+// Every tile walks all entries of the B rows, so rows of several hundred entries over many
+// tiles favour the wider ones: 2048 rows of 40 times 65,536 columns, B rows of 655, 2357 us
+// with 2048, 2233 with 4096; 20 times 32,768, rows of 1638, 1573 and 1519.  Short B rows and
+// few tiles favour the waves (rows of 82 times 8192 523 and 553; of 819 times 16,384 447 and
+// 456; of 262 times 131,072 1359 and 1433), and so do wider products, whose B outgrows the
+// L2s (rows of 1311 times 131,072 4454 and 4494; of 2621 times 262,144 1331 and 1365).
+inline int tile_columns(int K, int N, int nnzB) {
+    return N > 16384 && N <= 65536 && nnzB > 300ll * K ? 4096 : 2048;
+}
 constexpr int kAhead = 8;  // B rows whose entries are in flight
 
+template <int kTN>
 __global__ __launch_bounds__(256) void k_spgemm_dense(int M, int N, int ntiles, const int* __restrict__ rpA,
                                                       const int* __restrict__ ciA, const float* __restrict__ vA,
                                                       const int* __restrict__ rpB, const int* __restrict__ ciB,
@@ -119,15 +129,22 @@ extern "C" int armsp_spgemm_dense_f32(int M, int K, int N, int nnzA, const int* 
     if (M < 0 || K < 0 || N < 0 || nnzA < 0 || nnzB < 0) return ARMSP_ERROR_INVALID_VALUE;
     if (M == 0 || N == 0 || nnzA == 0 || nnzB == 0) return ARMSP_SUCCESS;
     if (!rowptrA || !colindA || !rowptrB || !colindB || !C || ldc < N) return ARMSP_ERROR_INVALID_VALUE;
-    const int ntiles = (N + kTN - 1) / kTN;
+    const int tn = tile_columns(K, N, nnzB);
+    const int ntiles = (N + tn - 1) / tn;
     const int64_t items = (int64_t)M * ntiles;
     if (items > 0x7fffffffLL - 4) return ARMSP_ERROR_NOT_SUPPORTED;
     hipStream_t s = as_stream(stream);
     TimedLaunch t("spgemm", s);
     // 16-byte row staging when every tile row starts 16-byte aligned and is whole float4s
     const int vec4 = ((uintptr_t)C % 16 == 0 && ldc % 4 == 0 && N % 4 == 0) ? 1 : 0;
-    hipLaunchKernelGGL(k_spgemm_dense, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, M, N, ntiles, rowptrA,
-                       colindA, valA, rowptrB, colindB, valB, C, ldc, vec4);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, M, N, ntiles, rowptrA, colindA, valA,
+                           rowptrB, colindB, valB, C, ldc, vec4);
+    };
+    if (tn == 4096)
+        launch(k_spgemm_dense<4096>);
+    else
+        launch(k_spgemm_dense<2048>);
     ARMSP_LAUNCHED();
     t.stop();
     return ARMSP_SUCCESS;
