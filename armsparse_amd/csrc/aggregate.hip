@@ -189,7 +189,7 @@ __device__ __forceinline__ void max_long_rows(int wave, int j0, int j1, int tile
 // every group of G lanes folds a part of the row, the parts are joined in order, within
 // the waves by shuffles and across them in LDS.  Columns as in max_short_rows.
 template <int V, int G>
-__device__ __forceinline__ void max_group_rows(int j0, int j1, int tile, int M, int N, int long_row,
+__device__ __forceinline__ void max_group_rows(int j0, int j1, int tile, int M, int N, int nnz, int long_row,
                                                const int* __restrict__ rowptr, const int* __restrict__ colind,
                                                const float* __restrict__ val, const float* __restrict__ B, int ldb,
                                                float init, float* __restrict__ C, int ldc, int* __restrict__ argmax) {
@@ -208,7 +208,8 @@ __device__ __forceinline__ void max_group_rows(int j0, int j1, int tile, int M, 
         uint64_t longs = __ballot(rl < M && el - sl > long_row && sl >= j0 && sl < j1);
         for (; longs; longs &= longs - 1) {
             const int k = __builtin_ctzll(longs);
-            const int r = rb + k, s = read_lane(sl, k), e = read_lane(el, k);
+            // (a malformed rowptr cannot carry the walk past nonzero nnz)
+            const int r = rb + k, s = read_lane(sl, k), e = min(read_lane(el, k), nnz);
             const int p0 = s + (int)((int64_t)(e - s) * part / P), p1 = s + (int)((int64_t)(e - s) * (part + 1) / P);
             float acc[V];
             uint32_t arg[V];
@@ -292,7 +293,7 @@ __device__ __forceinline__ void max_group_rows(int j0, int j1, int tile, int M, 
 
 // Rows of at most long_row nonzeros, a group of G lanes each.
 template <int V, int G>
-__device__ __forceinline__ void max_short_rows(int blk, int tile, int M, int N, int long_row,
+__device__ __forceinline__ void max_short_rows(int blk, int tile, int M, int N, int nnz, int long_row,
                                                const int* __restrict__ rowptr, const int* __restrict__ colind,
                                                const float* __restrict__ val, const float* __restrict__ B, int ldb,
                                                float init, float* __restrict__ C, int ldc, int* __restrict__ argmax) {
@@ -302,8 +303,9 @@ __device__ __forceinline__ void max_short_rows(int blk, int tile, int M, int N, 
     if (row >= M) return;
     const int col = (tile * G + lane) * V;
     const bool active = col < N;
-    const int beg = rowptr[row], end = rowptr[row + 1];
-    if (end - beg > long_row) return;
+    const int beg = rowptr[row], stop = rowptr[row + 1];
+    if (stop - beg > long_row) return;
+    const int end = min(stop, nnz);  // (a malformed rowptr may promise more)
     const float* bp = B + (active ? col : 0);
     float acc[V];
     int arg[V];
@@ -376,12 +378,12 @@ __global__ __launch_bounds__(256) void k_spmm_max(int first, int M, int N, int n
             max_long_rows<VL>(range, (int)j0, j1, (b % ltiles) * 64 * VL, M, N, long_row, rowptr, colind, val, B, ldb,
                               init, C, ldc, argmax, parts);
         else
-            max_group_rows<V, G>((int)j0, j1, b % ltiles, M, N, long_row, rowptr, colind, val, B, ldb, init, C, ldc,
+            max_group_rows<V, G>((int)j0, j1, b % ltiles, M, N, nnz, long_row, rowptr, colind, val, B, ldb, init, C, ldc,
                                  argmax);
         return;
     }
     const int rb = b - nlong * ltiles;
-    max_short_rows<V, G>(rb % nshort, rb / nshort, M, N, nlong ? long_row : INT_MAX, rowptr, colind, val, B, ldb,
+    max_short_rows<V, G>(rb % nshort, rb / nshort, M, N, nnz, nlong ? long_row : INT_MAX, rowptr, colind, val, B, ldb,
                          init, C, ldc, argmax);
 }
 

@@ -14,7 +14,7 @@ HIP_INCLUDE = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
-@pytest.mark.parametrize("program", ["chunk_rows", "vcsr_medium", "max_gap"])
+@pytest.mark.parametrize("program", ["chunk_rows", "vcsr_medium", "max_gap", "max_bounds"])
 def test_device_functions_stay_in_range(program, tmp_path):
     exe = str(tmp_path / program)
     # (the entry points of an included source are never called: their callees stay unresolved)

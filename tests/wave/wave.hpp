@@ -33,6 +33,7 @@ constexpr int kLanes = 64;
 constexpr size_t kStack = 256 << 10;
 
 inline int g_lane = 0;
+inline int g_wave = 0;  // the wave's place in its workgroup
 inline uint64_t g_slot[2][kLanes], g_here[2];
 inline int g_round = 0;
 inline ucontext_t g_main, g_ctx[kLanes];
@@ -103,7 +104,7 @@ inline T value(uint64_t u) {
 // ------------------------------------------------ the device functions the sources use
 using std::max;
 using std::min;
-inline uint3 wave_thread() { return {(unsigned)wave::g_lane, 0, 0}; }
+inline uint3 wave_thread() { return {(unsigned)(64 * wave::g_wave + wave::g_lane), 0, 0}; }
 #define threadIdx wave_thread()
 inline uint3 blockIdx;
 inline dim3 blockDim(wave::kLanes), gridDim;
@@ -173,8 +174,10 @@ struct WaveFloats {
 #define __builtin_amdgcn_sbfe(v, at, n) ((int)((uint32_t)(v) << (32 - (at) - (n))) >> (32 - (n)))
 #define __builtin_nontemporal_load(p) (*(p))
 #define __builtin_nontemporal_store(v, p) ((void)(*(p) = (v)))
-// (not emulated, parsed only: what works across waves)
-inline void __syncthreads() { std::abort(); }
+// Waves of a workgroup run one after the other, if a test runs them: what one leaves in LDS
+// before a barrier the others do not see.
+inline void __syncthreads() { wave_sync(); }
+// (not emulated, parsed only)
 template <typename T>
 inline T atomicAdd(T*, T) { std::abort(); }
 template <typename T>
