@@ -194,7 +194,7 @@ __device__ __forceinline__ void sddmm_chunk(int wave, int M, int Kd, int nnz, in
     int i0 = 0, j0 = d0, j1 = d1;
     if constexpr (!COO) {
         int i1;
-        chunk_rows(part, wave, d0, d1, rowidx, M, nnz, i0, i1);
+        chunk_rows<true>(part, wave, d0, d1, rowidx, M, nnz, i0, i1);
         j0 = d0 - i0;
         j1 = d1 - i1;
     }

@@ -605,8 +605,8 @@ __device__ void vcsr_long_rows(int M, const int* __restrict__ list, int* __restr
                 }
             }
         } else {
-            // 32 blocks a step, the next step's LDS reads in flight during the adds (a batch
-            // holds whole steps, so a read past the row's end stays inside the batch)
+            // VCSR_STEP blocks a step, the next step's LDS reads in flight during the adds (a batch
+            // holds whole pairs of steps, so a read past the row's end stays inside the batch)
             __builtin_amdgcn_s_setprio(3);  // the chain of adds is the row's time: first in the SIMD's queue
             float s = 0.0f;
             for (int k = 0; k < nbat; ++k) {
@@ -694,7 +694,7 @@ __global__ __launch_bounds__(256) void k_spmv_vcsr_split(int M, const int* __res
     }
     // the short walker takes what neither list holds: rows of at most VCSR_MED_MIN
     // blocks (the long-row limit is never below it; a constant here lets the
-    // compiler drop the walker's batch loop for longer rows: 66 VGPRs, not 111)
+    // compiler drop the walker's batch loop for longer rows: a kernel of 62 VGPRs, not 111)
     vcsr_short_rows((unsigned)(b - n_long_wg - n_med_wg), M, rowptr, colind, val, x, y, FUSED ? 1 : 0, VCSR_MED_MIN);
 }
 

@@ -40,7 +40,7 @@ constexpr int SCAN_CHUNK = 2048;  // 256 threads × 8
 // take two passes), the value travels with its key, and the row of a CSR entry
 // is formed in the first pass from rowptr.  (Sorting positions in 8-bit digits
 // and gathering rows and values at the end took 1523 us for the 1M R-MAT's 2^24
-// entries; 393 us now: 205 MB read and 213 MB written a pass, by the counters.)
+// entries; 383 us now: 205 MB read and 213 MB written a pass, by the counters.)
 // Consecutive tiles go to one XCD, so the lines two tiles share are completed in
 // that XCD's L2 (in launch order instead: 480 -> 503 us).
 constexpr int RADIX_MAX_BITS = 10;
@@ -591,9 +591,9 @@ void exclusive_scan(int64_t n, int* data, int* ws, hipStream_t s) {
 struct RadixPlan {
     int db, passes, tile, ntiles;
 };
-// Tiles of 512 threads × 8 records: longer runs per digit than shorter tiles, yet
-// four workgroups a CU, whose phases overlap (1M R-MAT transpose and 6M triplets to
-// CSR: 2048 records 506 and 401 us, 4096 393 and 373, 8192 430 and 407, 16,384 525
+// Tiles of 512 threads × 8 records: longer runs per digit than shorter tiles, yet two
+// workgroups a CU (97 VGPRs), whose phases overlap (1M R-MAT transpose and 6M triplets
+// to CSR, when measured: 2048 records 506 and 401 us, 4096 393 and 373, 8192 430 and 407, 16,384 525
 // and 501; 512 threads against 256 and 1024: 393, 457, 525 us).  With fewer records
 // than RADIX_BIG some CUs would have no such tile, so they are 2,048.
 constexpr int RADIX_BIG = 2 << 20;
